@@ -1,0 +1,193 @@
+"""What this library is timed on: the depthwise layers of the networks that use them, through the public Python API.
+
+A case is one pass over a few layers: ``"train"`` is the forward pass of every layer and then, in one autograd call, the
+gradients of every input, filter (and scale and bias, where there are any); ``"infer"`` is the forward pass alone under
+``no_grad``.  ``op`` says which function runs: ``DepthwiseConv2d`` modules (``"conv"``), ``depthwise_conv2d_fused`` with
+a folded batch-norm and SiLU (``"fused"``), or ``depthwise_conv2d_general`` with a dilation (``"general"``).  The layers
+are called one after another on independent tensors: what stands between them in a network is not this library's work.
+"""
+import math
+import os
+import sys
+
+import torch
+
+# the package's folder stands in the repository's root, which is the working folder
+_PACKAGE = os.path.join(os.getcwd(), "depthwise-conv-pytorch_amd")
+if _PACKAGE not in sys.path:
+    sys.path.insert(0, _PACKAGE)
+
+from torch_dwconv import DepthwiseConv2d, depthwise_conv2d_fused, depthwise_conv2d_general  # noqa: E402
+
+_DTYPES = {"fp32": torch.float32, "fp16": torch.float16, "bf16": torch.bfloat16}
+
+# depthwise layers of EfficientNet-B0 in network order: (C, halvings of the resolution before the layer, k, stride)
+_EFFNET_B0 = ((32, 1, 3, 1), (96, 1, 3, 2), (144, 2, 3, 1), (144, 2, 5, 2), (240, 3, 5, 1), (240, 3, 3, 2),
+              (480, 4, 3, 1), (480, 4, 5, 1), (672, 4, 5, 1), (672, 4, 5, 2), (1152, 5, 5, 1), (1152, 5, 3, 1))
+# the four stages of ConvNeXt-T: (C, what the resolution is divided by)
+_CONVNEXT_T = ((96, 4), (192, 8), (384, 16), (768, 32))
+# dilations of a segmentation head on a stride-8 backbone
+_ATROUS_RATES = (6, 12, 18)
+
+_LARGEST_BYTES = 5.6e9  # of a drawn case: what the largest listed one moves
+
+
+def _layers(case):
+    """(N, C, H, W, k, stride, padding, dilation) of every layer of the case."""
+    n = case["batch"]
+    if case["net"] == "effnet":
+        sizes = [case["res"]]
+        for _ in range(5):
+            sizes.append((sizes[-1] + 1) // 2)
+        return [(n, c, sizes[level], sizes[level], k, s, k // 2, 1) for c, level, k, s in _EFFNET_B0]
+    if case["net"] == "convnext":
+        return [(n, c, case["res"] // d, case["res"] // d, 7, 1, 3, 1) for c, d in _CONVNEXT_T]
+    if case["net"] == "atrous":
+        return [(n, case["channels"], case["res"], case["res"], 3, 1, rate, rate) for rate in _ATROUS_RATES]
+    k = case["kernel"]
+    return [(n, case["channels"], case["res"], case["res"], k, case["stride"], k // 2, 1)]
+
+
+def _out_size(size, k, stride, pad, dil):
+    return (size + 2 * pad - dil * (k - 1) - 1) // stride + 1
+
+
+def _case(net, op, call, dtype, layout, batch, res, **more):
+    return {"net": net, "op": op, "call": call, "dtype": dtype, "layout": layout, "batch": batch, "res": res, **more}
+
+
+def listed():
+    def case(name, *args, **more):
+        return {"name": name, **_case(*args, **more)}
+
+    return [
+        # one image through a deployed EfficientNet-B0 (batch-norm folded, half precision): twelve short launches
+        case("infer_effnet224_b1_fp16", "effnet", "fused", "infer", "fp16", "nchw", 1, 224),
+        # one small layer of a training step, the reference's own kind of test size: forward and backward of 19 MB
+        case("train_layer56_b8_fp32", "layer", "conv", "train", "fp32", "nchw", 8, 56, channels=32, kernel=3, stride=1),
+        # serving in batches, channels-last and bfloat16, at a resolution whose maps are powers of two
+        case("infer_effnet256_b64_bf16_nhwc", "effnet", "fused", "infer", "bf16", "nhwc", 64, 256),
+        # the library's headline: a training step of the twelve layers in full precision
+        case("train_effnet224_b128_fp32", "effnet", "conv", "train", "fp32", "nchw", 128, 224),
+        # the same step in mixed precision
+        case("train_effnet224_b128_bf16", "effnet", "conv", "train", "bf16", "nchw", 128, 224),
+        # and channels-last, the layout that the 1x1 convolutions around these layers prefer in mixed precision
+        case("train_effnet224_b128_bf16_nhwc", "effnet", "conv", "train", "bf16", "nhwc", 128, 224),
+        # ragged maps (150, 75, 38, 19 and 10 wide: EfficientNet-B3's resolution) in mixed precision
+        case("train_effnet300_b64_bf16", "effnet", "conv", "train", "bf16", "nchw", 64, 300),
+        # training with batch-norm and SiLU fused into the convolution, all four gradients
+        case("train_fused_effnet224_b128_fp32", "effnet", "fused", "train", "fp32", "nchw", 128, 224),
+        # 7x7 filters on maps of 56 to 7, full precision
+        case("train_convnext224_b64_fp32", "convnext", "conv", "train", "fp32", "nchw", 64, 224),
+        # the same in bfloat16 and channels-last, ConvNeXt's own layout
+        case("train_convnext224_b64_bf16_nhwc", "convnext", "conv", "train", "bf16", "nhwc", 64, 224),
+        # large feature maps, as in image generation and restoration networks
+        case("train_layer256_k5_b16_fp32", "layer", "conv", "train", "fp32", "nchw", 16, 256, channels=64, kernel=5, stride=1),
+        # the dilated 3x3 layers of a segmentation head on a 513-pixel input
+        case("train_atrous65_b16_fp32", "atrous", "general", "train", "fp32", "nchw", 16, 65, channels=256),
+    ]
+
+
+def _log_int(rng, low, high):
+    return int(round(math.exp(rng.uniform(math.log(low), math.log(high)))))
+
+
+def draw(rng):
+    """One more case: a network of the list (or a single layer) at any batch, resolution, element type and layout."""
+    while True:
+        net = rng.choice(("effnet", "effnet", "effnet", "convnext", "layer", "atrous"))
+        dtype = rng.choice(("fp32", "bf16", "fp16"))
+        layout = "nchw" if net == "atrous" else rng.choice(("nchw", "nchw", "nhwc"))
+        call = rng.choice(("train", "train", "infer"))
+        op = "general" if net == "atrous" else "fused" if call == "infer" or rng.random() < 0.25 else "conv"
+        if net == "effnet":
+            case = _case(net, op, call, dtype, layout, _log_int(rng, 1, 128), rng.randint(160, 320))
+        elif net == "convnext":
+            case = _case(net, "conv", call, dtype, layout, _log_int(rng, 1, 64), 32 * rng.randint(5, 9))
+        elif net == "atrous":
+            case = _case(net, op, call, dtype, layout, _log_int(rng, 2, 16), rng.randint(33, 97),
+                         channels=8 * rng.randint(8, 32))
+        else:
+            case = _case(net, op, call, dtype, layout, _log_int(rng, 1, 64), _log_int(rng, 7, 256),
+                         channels=_log_int(rng, 4, 96) * 4, kernel=rng.choice((3, 5, 7)), stride=rng.choice((1, 1, 2)))
+        if work(case)["bytes"] <= _LARGEST_BYTES and work(case)["flops"] <= 25e9:
+            return case
+
+
+def prepare(case, seed):
+    """Activations and output gradients of unit variance, filters of variance 1 / k^2, folded batch-norms around one."""
+    dev = torch.device("cuda")
+    dtype = _DTYPES[case["dtype"]]
+    fmt = torch.channels_last if case["layout"] == "nhwc" else torch.contiguous_format
+    gen = torch.Generator(dev).manual_seed(seed)
+    train = case["call"] == "train"
+
+    def normal(*shape, scale=1.0, as_type=dtype, layout=torch.contiguous_format):
+        t = torch.randn(*shape, generator=gen, device=dev) * scale
+        return t.to(as_type).contiguous(memory_format=layout)
+
+    layers = []
+    for n, c, h, w, k, s, p, d in _layers(case):
+        layer = {"x": normal(n, c, h, w, layout=fmt).requires_grad_(train), "stride": s, "padding": p, "dilation": d}
+        weight = normal(c, 1, k, k, scale=1.0 / k)
+        if case["op"] == "conv":
+            layer["module"] = DepthwiseConv2d(c, c, k, stride=s, padding=p).to(dev, dtype)
+            with torch.no_grad():
+                layer["module"].weight.copy_(weight)
+            layer["params"] = [layer["module"].weight]
+        else:
+            layer["params"] = [weight.requires_grad_(train)]
+        if case["op"] == "fused":
+            bias = normal(c, scale=0.3, as_type=torch.float32).requires_grad_(train)
+            scale = (1.0 + normal(c, scale=0.1, as_type=torch.float32)).requires_grad_(train)
+            layer["params"] += [bias, scale]
+        if train:
+            layer["gy"] = normal(n, c, _out_size(h, k, s, p, d), _out_size(w, k, s, p, d), layout=fmt)
+        layers.append(layer)
+    return {"op": case["op"], "train": train, "layers": layers}
+
+
+def _forward(op, layer):
+    if op == "conv":
+        return layer["module"](layer["x"])
+    if op == "general":
+        return depthwise_conv2d_general(layer["x"], layer["params"][0], layer["stride"], layer["padding"], layer["dilation"])
+    weight, bias, scale = layer["params"]
+    return depthwise_conv2d_fused(layer["x"], weight, bias, scale, "silu", layer["stride"], layer["padding"])
+
+
+def run(state):
+    op, layers = state["op"], state["layers"]
+    if not state["train"]:
+        with torch.no_grad():
+            return [_forward(op, layer) for layer in layers]
+    outputs = [_forward(op, layer) for layer in layers]
+    wanted = [t for layer in layers for t in (layer["x"], *layer["params"])]
+    grads = torch.autograd.grad(outputs, wanted, [layer["gy"] for layer in layers])
+    return [o.detach() for o in outputs] + list(grads)
+
+
+def work(case):
+    """Every input read once, every output written once; a multiply-add counts as two operations."""
+    size = 4 if case["dtype"] == "fp32" else 2
+    train = case["call"] == "train"
+    moved = flops = 0
+    for n, c, h, w, k, s, p, d in _layers(case):
+        nx, nw = n * c * h * w, c * k * k
+        ny = n * c * _out_size(h, k, s, p, d) * _out_size(w, k, s, p, d)
+        params = nw * size + (8 * c if case["op"] == "fused" else 0)
+        moved += (nx + ny) * size + params
+        flops += 2 * ny * k * k
+        if train:
+            moved += (ny + nx) * size + params
+            flops += 4 * ny * k * k
+    return {"bytes": moved, "flops": flops}
+
+
+def tolerance(case):
+    """About four times the error against the same function in 64 bits.  Sums are 32 bits wide (3e-7 measured) and 16-bit
+    results are rounded once (1.7e-3 for bfloat16, 2.1e-4 for float16); training with the fused epilogue also rounds the
+    gradient of the convolution's result (2.5e-3 and 3e-4)."""
+    rel = {"fp32": 2e-6, "fp16": 9e-4, "bf16": 7e-3}[case["dtype"]]
+    twice_rounded = case["op"] == "fused" and case["call"] == "train" and case["dtype"] != "fp32"
+    return {"rel": 1.5 * rel if twice_rounded else rel}
