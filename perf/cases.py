@@ -191,3 +191,52 @@ def tolerance(case):
     rel = {"fp32": 2e-6, "fp16": 9e-4, "bf16": 7e-3}[case["dtype"]]
     twice_rounded = case["op"] == "fused" and case["call"] == "train" and case["dtype"] != "fp32"
     return {"rel": 1.5 * rel if twice_rounded else rel}
+
+
+def _exact_layer(op, train, layer):
+    """(y, gradients) of one layer in 64 bits: one strided slice of the zero-padded input per tap."""
+    x = layer["x"].detach().double().contiguous()
+    w = layer["params"][0].detach().double()
+    s, p, d = layer["stride"], layer["padding"], layer["dilation"]
+    k, h, width = w.shape[-1], x.shape[2], x.shape[3]
+    oh, ow = _out_size(h, k, s, p, d), _out_size(width, k, s, p, d)
+    padded = torch.nn.functional.pad(x, (p, p, p, p))
+
+    def window(t, i, j):
+        return t[:, :, i * d:i * d + s * (oh - 1) + 1:s, j * d:j * d + s * (ow - 1) + 1:s]
+
+    conv = x.new_zeros(x.shape[0], x.shape[1], oh, ow)
+    for i in range(k):
+        for j in range(k):
+            conv.addcmul_(window(padded, i, j), w[:, :, i, j].view(1, -1, 1, 1))
+    y, slope = conv, None
+    if op == "fused":
+        bias, scale = (t.detach().double().view(1, -1, 1, 1) for t in layer["params"][1:])
+        z = conv * scale + bias
+        gate = torch.sigmoid(z)
+        y, slope = z * gate, gate * (1 + z * (1 - gate))
+    if not train:
+        return y, []
+    gy = layer["gy"].double().contiguous()
+    more = []
+    if op == "fused":
+        gy = gy * slope
+        more = [gy.sum((0, 2, 3)), (gy * conv).sum((0, 2, 3))]
+        gy = gy * scale
+    gx, gw = torch.zeros_like(padded), torch.zeros_like(w)
+    for i in range(k):
+        for j in range(k):
+            window(gx, i, j).addcmul_(gy, w[:, :, i, j].view(1, -1, 1, 1))
+            gw[:, 0, i, j] = (window(padded, i, j) * gy).sum((0, 2, 3))
+    return y, [gx[:, :, p:p + h, p:p + width].contiguous(), gw, *more]
+
+
+def exact(case, seed):
+    """What ``run`` returns, in 64 bits and by plain torch: exact values of the same 16- or 32-bit inputs."""
+    state = prepare(case, seed)
+    outputs, grads = [], []
+    for layer in state["layers"]:
+        y, more = _exact_layer(state["op"], state["train"], layer)
+        outputs.append(y)
+        grads += more
+    return outputs + grads
