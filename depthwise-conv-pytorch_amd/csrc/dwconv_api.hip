@@ -457,6 +457,8 @@ int general_forward_any(const T *in, const T *taps, T *out, int batch, int chann
                 r = try_launch_fir_tiled<T>(in, taps, out, gg, static_cast<hipStream_t>(stream));
                 if (r >= 0) return r;
             }
+            r = try_launch_atrous_forward<T>(in, taps, out, g, static_cast<hipStream_t>(stream));
+            if (r >= 0) return r;
             if (multiplier == 1) {  // any other dilation, stride or filter extent: the any-geometry tiled kernel
                 Geometry gg{batch, channel, in_h, in_w, kernel_h, kernel_w, 1, 1, stride_h, stride_w,
                             pad_h, pad_h, pad_w, pad_w, g.out_h, g.out_w, 1};
@@ -491,6 +493,8 @@ size_t general_workspace_any(const GeneralGeometry &g)
     if constexpr (!std::is_same<T, double>::value) {
         const size_t st = general_stack_workspace(g);
         if (st > need) need = st;
+        const size_t at = atrous_workspace(g, sizeof(T));
+        if (at > need) need = at;
         if (dilated_small(g)) {
             const size_t sm = wgrad_small_workspace(dilated_wgrad_geometry(g));
             if (sm > need) need = sm;
@@ -554,6 +558,8 @@ int general_backward_any(const T *in, const T *gy, const T *taps, T *gx, T *gw, 
                 rc = try_launch_bwd_small<T>(in, gy, taps, gx, gw, ws, ws_bytes, dilated_wgrad_geometry(g), stream);
                 if (rc >= 0) return rc;
             }
+            rc = try_launch_atrous_backward<T>(in, gy, taps, gx, gw, ws, ws_bytes, g, stream);
+            if (rc >= 0) return rc;
             if (multiplied_tiled(g)) {
                 // the two passes on their own; either falls back to the per-element kernels where the tiled one
                 // does not take the shape

@@ -335,6 +335,14 @@ int epilogue_backward(const IO *conv, const IO *out_grad, const float *scale, co
                       float *param_grad, void *ws, size_t ws_bytes, int batch, int channel, int out_h, int out_w, int act,
                       bool channels_last, hipStream_t stream);
 
+// ---- dilated 3x3 layers at stride 1 with "same" padding: dwconv_atrous.hip (-1 / 0 where they do not cover g) ----
+size_t atrous_workspace(const GeneralGeometry &g, size_t esize);
+template <typename IO>
+int try_launch_atrous_forward(const IO *in, const IO *taps, IO *out, const GeneralGeometry &g, hipStream_t stream);
+template <typename IO>
+int try_launch_atrous_backward(const IO *in, const IO *gy, const IO *taps, IO *gx, IO *gw, void *ws, size_t ws_bytes,
+                               const GeneralGeometry &g, hipStream_t stream);
+
 // ---- dilation and depth multiplier: dwconv_general.hip (T = float, double, half_t or bf16_t) ----
 template <typename T>
 int general_forward(const T *in, const T *taps, T *out, const GeneralGeometry &g, hipStream_t stream);

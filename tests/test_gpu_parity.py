@@ -927,6 +927,59 @@ def test_any_geometry_tiled_kernels(dw, gpu, case, dtype):
     np.testing.assert_allclose(_np(gw.double()), gw_ref.numpy(), rtol=gtol, atol=gtol * float(gw_ref.abs().max()))
 
 
+# (N, C, H, W, dil_h, dil_w): planes that start at every offset from a 16-byte boundary, chains of one to many steps,
+# dilations at and beyond the map, a second round of chains, the largest planes (64 KiB less the zero cell) and one above
+ATROUS = [
+    (3, 5, 7, 9, 3, 3), (2, 3, 5, 5, 4, 4), (2, 3, 6, 11, 6, 11), (2, 2, 9, 13, 40, 50), (5, 3, 33, 35, 6, 12),
+    (2, 7, 64, 64, 18, 18), (3, 2, 65, 65, 12, 12), (2, 3, 97, 97, 18, 6), (1, 2, 127, 129, 6, 6), (1, 2, 130, 131, 5, 5),
+    (40, 2, 20, 17, 3, 5), (1, 1, 3, 40, 3, 2), (1, 2, 1, 37, 2, 5), (2, 2, 41, 1, 6, 3),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=["f32", "f16", "bf16"])
+@pytest.mark.parametrize("case", ATROUS, ids=lambda c: "N%d_C%d_%dx%d_d%dx%d" % c)
+def test_atrous_plane_kernel(dw, gpu, case, dtype):
+    """Dilated 3x3 layers at stride 1 with "same" padding: result and both gradients against fp64 autograd on the rounded
+    inputs (one rounding step of the format on top of the fp32 bounds), bit-identical on a second run; a non-finite input
+    reaches only the sums that torch gives it to."""
+    from torch_dwconv import _C
+    from torch_dwconv.dwconv import depthwise_conv2d_general
+
+    n, c, h, w, dh, dw_ = case
+    step = {torch.float32: 0.0, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dtype]
+    g = torch.Generator("cpu").manual_seed(17)
+    x = torch.randn(n, c, h, w, generator=g).to(dtype)
+    wt = (torch.randn(c, 1, 3, 3, generator=g) / 3).to(dtype)
+    gy = torch.randn(n, c, h, w, generator=g).to(dtype)
+    xr, wr = x.double().requires_grad_(True), wt.double().requires_grad_(True)
+    y_ref = torch.nn.functional.conv2d(xr, wr, padding=(dh, dw_), dilation=(dh, dw_), groups=c)
+    gx_ref, gw_ref = torch.autograd.grad(y_ref, (xr, wr), gy.double())
+    xg, wg, gyg = x.to(gpu), wt.to(gpu), gy.to(gpu)
+    y = depthwise_conv2d_general(xg, wg, padding=(dh, dw_), dilation=(dh, dw_))
+    _announce(case, str(dtype), _C.last_variant())
+    gx, gw = _C.dwconv2d_general_backward(xg, gyg, wg, 1, 1, dh, dw_, dh, dw_)
+    planes = h * w * x.element_size() + 48 <= 64 * 1024
+    assert _C.last_variant().endswith(" plane") == (planes and not (dh == dw_ == 2)), _C.last_variant()
+    gx2, gw2 = _C.dwconv2d_general_backward(xg, gyg, wg, 1, 1, dh, dw_, dh, dw_)
+    assert torch.equal(gx, gx2) and torch.equal(gw, gw2)
+    tol, gtol = 1e-5 + step, 1e-4 + step
+    np.testing.assert_allclose(_np(y.double()), y_ref.detach().numpy(), rtol=tol, atol=tol)
+    np.testing.assert_allclose(_np(gx.double()), gx_ref.numpy(), rtol=tol, atol=tol)
+    np.testing.assert_allclose(_np(gw.double()), gw_ref.numpy(), rtol=gtol, atol=gtol * max(1.0, float(gw_ref.abs().max())))
+    if planes:
+        xg[0, 0, 0, 0] = float("inf")
+        y = depthwise_conv2d_general(xg, wg, padding=(dh, dw_), dilation=(dh, dw_))
+        touched = torch.zeros(n, c, h, w, dtype=torch.bool)
+        touched[0, 0, 0, 0] = True
+        for i in (0, dh):
+            for j in (0, dw_):
+                if i < h and j < w:
+                    touched[0, 0, i, j] = True
+        assert torch.equal(torch.isfinite(y).cpu(), ~touched)
+        _, gw = _C.dwconv2d_general_backward(xg, gyg, wg, 1, 1, dh, dw_, dh, dw_)
+        assert bool(torch.isfinite(gw[1:]).all()) and not bool(torch.isfinite(gw[0, 0, 1, 1]))
+
+
 def test_tuning_overrides_need_the_master_switch(dw, gpu, monkeypatch):
     """DWCONV_* overrides of the planners are ignored unless DWCONV_TUNING=1 is set too, and ill-formed values always."""
     from torch_dwconv import _C
