@@ -86,9 +86,19 @@ __device__ __forceinline__ void nhwc_load_row(__amdgpu_buffer_rsrc_t view, int i
 template <typename IO, int KK, bool FLIP>
 __device__ __forceinline__ void nhwc_stage_taps(const IO *__restrict__ taps, float *lds, int c0, int nch)
 {
-    for (int i = threadIdx.x; i < nch * KK; i += blockDim.x) {
-        const int cl = i / KK, t = i - cl * KK;
-        lds[(FLIP ? KK - 1 - t : t) * nch + cl] = Io<IO>::in(taps[static_cast<long>(c0) * KK + i]);
+    // kTapBatch loads in flight per lane: one at a time, a lane's 6 to 12 taps cost as many memory latencies
+    constexpr int kTapBatch = 8;
+    const IO *src = taps + static_cast<long>(c0) * KK;
+    const int total = nch * KK;
+    for (int i0 = threadIdx.x; i0 < total; i0 += kTapBatch * kNhwcThreads) {
+        IO v[kTapBatch];
+#pragma unroll
+        for (int k = 0; k < kTapBatch; ++k) v[k] = src[min(i0 + k * kNhwcThreads, total - 1)];
+#pragma unroll
+        for (int k = 0; k < kTapBatch; ++k) {
+            const int i = i0 + k * kNhwcThreads, cl = i / KK, t = i - cl * KK;
+            if (i < total) lds[(FLIP ? KK - 1 - t : t) * nch + cl] = Io<IO>::in(v[k]);
+        }
     }
 }
 
