@@ -26,6 +26,15 @@ if not os.path.exists(LIBRARY_PATH):
 
 _lib = ctypes.CDLL(LIBRARY_PATH)
 
+try:
+    from . import _binding
+except ImportError as e:
+    raise ImportError(
+        f"torch_dwconv._binding does not load ({e}): build it with `make -C depthwise-conv-pytorch_amd/csrc`"
+    ) from e
+# Every function below first hands its arguments to its native namesake (csrc/dwconv_binding.cpp), which serves plain
+# GPU tensors and returns None for everything else.  What follows serves the rest and raises the errors.
+
 _i, _p, _z = ctypes.c_int, ctypes.c_void_p, ctypes.c_size_t
 _lib.dwconv_last_error.restype = ctypes.c_char_p
 _lib.dwconv_last_variant.restype = ctypes.c_char_p
@@ -136,6 +145,9 @@ def _stream(t):
 
 def use_dwconv2d_small(input, kernel, up_h, up_w, down_h, down_w, pad_h, pad_w):
     """torch_dwconv/dwconv_kernel.cu:652-662; pure geometry, no device work."""
+    native = _binding.use_small(input, kernel, up_h, up_w, down_h, down_w, pad_h, pad_w)
+    if native is not None:
+        return native
     return bool(
         _lib.dwconv_use_dwconv2d_small(
             input.shape[2], input.shape[3], kernel.shape[2], kernel.shape[3],
@@ -146,6 +158,9 @@ def use_dwconv2d_small(input, kernel, up_h, up_w, down_h, down_w, pad_h, pad_w):
 
 def dwconv2d(input, kernel, up_h, up_w, down_h, down_w, pad_h0, pad_h1, pad_w0, pad_w1, forward):
     """torch_dwconv/dwconv.cpp:27-35: up-sample / filter / down-sample of every plane."""
+    native = _binding.conv(input, kernel, up_h, up_w, down_h, down_w, pad_h0, pad_h1, pad_w0, pad_w1, forward)
+    if native is not None:
+        return native
     _check_cuda(input, "input")
     _check_cuda(kernel, "kernel")
     _check_shapes(input, kernel)
@@ -168,6 +183,9 @@ def dwconv2d(input, kernel, up_h, up_w, down_h, down_w, pad_h0, pad_h1, pad_w0, 
 
 def dwconv2d_small(input, kernel, up_h, up_w, down_h, down_w, pad_h, pad_w, forward):
     """torch_dwconv/dwconv.cpp:37-46: whole-plane stride-1 same-size convolution."""
+    native = _binding.conv_small(input, kernel, up_h, up_w, down_h, down_w, pad_h, pad_w, forward)
+    if native is not None:
+        return native
     _check_cuda(input, "input")
     _check_cuda(kernel, "kernel")
     _check_shapes(input, kernel)
@@ -221,6 +239,9 @@ def dwconv2d_backward(input, out_grad, kernel, stride_h, stride_w, pad_h, pad_w)
     One call for the two the reference's backward makes (torch_dwconv/dwconv.py:56-68); the library reads
     ``out_grad`` once where a fused kernel covers the geometry.  Returns ``(grad_input, grad_kernel)``.
     """
+    native = _binding.backward(input, out_grad, kernel, stride_h, stride_w, pad_h, pad_w)
+    if native is not None:
+        return native
     _check_cuda(input, "input")
     _check_cuda(out_grad, "out_grad")
     _check_cuda(kernel, "kernel")
@@ -277,6 +298,9 @@ def dwconv2d_backward_noalloc(input, out_grad, kernel, in_grad, kernel_grad, str
 # ---- channels-last tensors -----------------------------------------------------------------------------
 def is_channels_last(t):
     """True when ``t`` (logical shape N,C,H,W) is laid out N,H,W,C in memory and not also N,C,H,W."""
+    native = _binding.is_channels_last(t)
+    if native is not None:
+        return native
     return t.dim() == 4 and t.is_contiguous(memory_format=torch.channels_last) and not t.is_contiguous()
 
 
@@ -285,6 +309,9 @@ def dwconv2d_nhwc(input, kernel, stride_h, stride_w, pad_h, pad_w):
 
     The reference has no such path: it makes ``input`` NCHW-contiguous first (torch_dwconv/dwconv_kernel.cu:855).
     """
+    native = _binding.conv_nhwc(input, kernel, stride_h, stride_w, pad_h, pad_w)
+    if native is not None:
+        return native
     _check_cuda(input, "input")
     _check_cuda(kernel, "kernel")
     _check_shapes(input, kernel)
@@ -308,6 +335,10 @@ def dwconv2d_backward_nhwc(input, out_grad, kernel, stride_h, stride_w, pad_h, p
                            need_kernel_grad=True):
     """Both gradients for channels-last ``input`` / ``out_grad``; ``grad_input`` comes back channels-last.  A gradient
     that is not needed is not computed and comes back as ``None``."""
+    native = _binding.backward_nhwc(input, out_grad, kernel, stride_h, stride_w, pad_h, pad_w, need_input_grad,
+                                     need_kernel_grad)
+    if native is not None:
+        return native
     _check_cuda(input, "input")
     _check_cuda(out_grad, "out_grad")
     _check_cuda(kernel, "kernel")
@@ -345,6 +376,10 @@ def dwconv2d_fused(input, kernel, scale, shift, activation, stride_h, stride_w, 
     ``scale`` / ``shift``: per-channel tensors or ``None``; ``activation``: ``None``, ``'relu'``, ``'relu6'`` or
     ``'silu'``.  The reference has no such entry point (it rejects a bias, torch_dwconv/dwconv.py:108-109).
     """
+    if activation in ACTIVATIONS:
+        native = _binding.fused(input, kernel, scale, shift, ACTIVATIONS[activation], stride_h, stride_w, pad_h, pad_w)
+        if native is not None:
+            return native
     _check_cuda(input, "input")
     _check_cuda(kernel, "kernel")
     _check_shapes(input, kernel)
@@ -385,6 +420,10 @@ def dwconv2d_epilogue_backward(conv_out, out_grad, scale, shift, activation):
     channels-last, taken from ``conv_out``): returns ``(conv_out_grad, scale_grad, shift_grad)``.  ``conv_out`` is
     overwritten with ``conv_out_grad`` (the same tensor comes back); the two parameter gradients are float32
     vectors of ``C`` entries.  No counterpart in the reference."""
+    if activation in ACTIVATIONS:
+        native = _binding.epilogue_backward(conv_out, out_grad, scale, shift, ACTIVATIONS[activation])
+        if native is not None:
+            return native
     _check_cuda(conv_out, "conv_out")
     _check_cuda(out_grad, "out_grad")
     sfx = _suffix(conv_out, out_grad)
@@ -436,6 +475,9 @@ def _multiplier(input, kernel):
 
 def dwconv2d_general(input, kernel, stride_h, stride_w, pad_h, pad_w, dil_h, dil_w):
     """``F.conv2d(input, kernel, stride, padding, dilation, groups=C)`` for a kernel of shape (C*M,1,KH,KW)."""
+    native = _binding.general(input, kernel, stride_h, stride_w, pad_h, pad_w, dil_h, dil_w)
+    if native is not None:
+        return native
     _check_cuda(input, "input")
     _check_cuda(kernel, "kernel")
     m = _multiplier(input, kernel)
@@ -458,6 +500,9 @@ def dwconv2d_general(input, kernel, stride_h, stride_w, pad_h, pad_w, dil_h, dil
 
 def dwconv2d_general_backward(input, out_grad, kernel, stride_h, stride_w, pad_h, pad_w, dil_h, dil_w):
     """Both gradients of ``dwconv2d_general``; returns ``(grad_input, grad_kernel)``."""
+    native = _binding.general_backward(input, out_grad, kernel, stride_h, stride_w, pad_h, pad_w, dil_h, dil_w)
+    if native is not None:
+        return native
     _check_cuda(input, "input")
     _check_cuda(out_grad, "out_grad")
     _check_cuda(kernel, "kernel")

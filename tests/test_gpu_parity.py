@@ -927,6 +927,89 @@ def test_any_geometry_tiled_kernels(dw, gpu, case, dtype):
     np.testing.assert_allclose(_np(gw.double()), gw_ref.numpy(), rtol=gtol, atol=gtol * float(gw_ref.abs().max()))
 
 
+NATIVE_CALLS = [
+    ("dwconv2d", "xw", (1, 1, 2, 2, 1, 1, 1, 1, True), False), ("dwconv2d_small", "xw", (1, 1, 1, 1, 1, 1, True), False),
+    ("dwconv2d_backward", "xgw", (1, 1, 1, 1), False), ("dwconv2d_nhwc", "xw", (1, 1, 1, 1), True),
+    ("dwconv2d_backward_nhwc", "xgw", (1, 1, 1, 1), True), ("dwconv2d_backward_nhwc", "xgw", (1, 1, 1, 1, True, False), True),
+    ("dwconv2d_fused", "xwpp", ("silu", 1, 1, 1, 1), False), ("dwconv2d_fused", "xwnp", ("relu", 2, 2, 0, 1), True),
+    ("dwconv2d_epilogue_backward", "xgpn", ("silu",), False), ("dwconv2d_epilogue_backward", "xgpp", ("relu6",), True),
+    ("dwconv2d_general", "xw", (1, 1, 2, 2, 2, 2), False), ("dwconv2d_general_backward", "xgw", (1, 1, 1, 1, 1, 1), False),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64, torch.float16, torch.bfloat16], ids=["f32", "f64", "f16", "bf16"])
+@pytest.mark.parametrize("call", NATIVE_CALLS, ids=lambda c: "%s_%s%s" % (c[0], c[1], "_nhwc" if c[3] else ""))
+def test_native_calls_equal_the_python_ones(dw, gpu, call, dtype, monkeypatch):
+    """Each function of _C through its native namesake and through its Python body: the same bits, strides and types; what
+    the native one does not take (a tensor subclass, functorch wrappers, a dispatch mode, another dtype) it leaves alone."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from torch_dwconv import _C
+
+    name, what, args, nhwc = call
+    g = torch.Generator("cpu").manual_seed(3)
+    fmt = torch.channels_last if nhwc else torch.contiguous_format
+    make = {
+        "x": lambda: torch.randn(2, 8, 9, 11, generator=g).to(gpu, dtype).contiguous(memory_format=fmt),
+        "g": lambda: torch.randn(2, 8, 9, 11, generator=g).to(gpu, dtype).transpose(2, 3).contiguous().transpose(2, 3),
+        "w": lambda: torch.randn(8, 1, 3, 3, generator=g).to(gpu, dtype),
+        "p": lambda: torch.randn(1, 8, 1, 1, generator=g).to(gpu),
+        "n": lambda: None,
+    }
+    given = [make[k]() for k in what]
+    if dtype == torch.float64 and name in ("dwconv2d_backward", "dwconv2d_epilogue_backward"):
+        with pytest.raises(RuntimeError, match="no float64"):
+            getattr(_C, name)(*given, *args)
+        return
+
+    class Nothing:
+        def __getattr__(self, _):
+            return lambda *a: None
+
+    def run():
+        out = getattr(_C, name)(*[t.clone() if t is not None else None for t in given], *args)
+        return out if isinstance(out, tuple) else (out,)
+
+    native, served = _C._binding, []
+
+    class Counting:
+        def __getattr__(self, attr):
+            def f(*a):
+                r = getattr(native, attr)(*a)
+                if attr not in ("is_channels_last", "use_small"):
+                    served.append(r is not None)
+                return r
+            return f
+
+    monkeypatch.setattr(_C, "_binding", Counting())
+    fast = run()
+    assert served == [True]
+    monkeypatch.setattr(_C, "_binding", Nothing())
+    for a, b in zip(fast, run()):
+        assert (a is None and b is None) or (torch.equal(a, b) and a.stride() == b.stride() and a.dtype == b.dtype)
+    monkeypatch.setattr(_C, "_binding", native)
+    x = given[0]
+    assert native.is_channels_last(x) is nhwc and native.is_channels_last(x.cpu()) is None
+
+    class Sub(torch.Tensor):
+        pass
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, a=(), k=None):
+            return func(*a, **(k or {}))
+
+    assert native.is_channels_last(x.as_subclass(Sub)) is None
+    with Mode():
+        assert native.is_channels_last(x) is None
+    seen = []
+    torch.func.vmap(lambda t: (seen.append(native.is_channels_last(t)), t)[1])(x.unsqueeze(0))
+    assert seen == [None]
+    assert native.conv(x, x.double() if dtype != torch.float64 else x.float(), 1, 1, 1, 1, 1, 1, 1, 1, 1) is None
+    w = torch.ones(8, 1, 3, 3, device=gpu, dtype=dtype)
+    assert native.conv(x, w[:7], 1, 1, 1, 1, 1, 1, 1, 1, 1) is None and native.conv(x, w, 1, 1, 1.0, 1, 1, 1, 1, 1, 1) is None
+    assert native.conv(x, w, 1, 1, 1, 1) is None and native.conv(x.int(), w.int(), 1, 1, 1, 1, 1, 1, 1, 1, 1) is None
+
+
 # (N, C, H, W, dil_h, dil_w): planes that start at every offset from a 16-byte boundary, chains of one to many steps,
 # dilations at and beyond the map, a second round of chains, the largest planes (64 KiB less the zero cell) and one above
 ATROUS = [
