@@ -1061,6 +1061,11 @@ def test_atrous_plane_kernel(dw, gpu, case, dtype):
         assert torch.equal(torch.isfinite(y).cpu(), ~touched)
         _, gw = _C.dwconv2d_general_backward(xg, gyg, wg, 1, 1, dh, dw_, dh, dw_)
         assert bool(torch.isfinite(gw[1:]).all()) and not bool(torch.isfinite(gw[0, 0, 1, 1]))
+        # the last element of a plane meets an output through the taps that lead to a row and a column of the map
+        xg[0, 0, 0, 0], xg[0, 0, h - 1, w - 1] = 0.0, float("inf")
+        _, gw = _C.dwconv2d_general_backward(xg, gyg, wg, 1, 1, dh, dw_, dh, dw_)
+        met = torch.outer(torch.tensor([False, True, h > dh]), torch.tensor([False, True, w > dw_]))
+        assert torch.equal(torch.isfinite(gw[0, 0]).cpu(), ~met)
 
 
 def test_tuning_overrides_need_the_master_switch(dw, gpu, monkeypatch):
