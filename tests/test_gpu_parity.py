@@ -1677,6 +1677,32 @@ def test_fused_epilogue_training_path(dw, gpu, case, activation):
             assert (a is None and b is None) or torch.equal(a, b)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=["f32", "f16", "bf16"])
+@pytest.mark.parametrize("channel", [3, 4, 32, 37, 70, 96, 144, 255, 256, 260, 268, 672, 1152])
+@pytest.mark.parametrize("pixels", [(1, 1, 2), (2, 3, 5), (3, 19, 37)], ids=str)
+def test_epilogue_backward_channels_last_lanes(dw, gpu, pixels, channel, dtype):
+    """Every split of a workgroup into pixels and channel lanes (one group, a part of a wavefront, several shares), chunks
+    that end inside a lane's batch of pixels, single elements where four do not divide the channels; against fp64."""
+    import torch.nn.functional as F
+
+    from torch_dwconv import _C
+
+    n, h, w = pixels
+    step = {torch.float32: 1e-6, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dtype]
+    g = torch.Generator("cpu").manual_seed(5)
+    y, gy = (torch.randn(n, channel, h, w, generator=g).to(dtype).contiguous(memory_format=torch.channels_last) for _ in "ab")
+    scale, shift = torch.rand(channel, generator=g) + 0.5, torch.randn(channel, generator=g)
+    conv, sr, br = (t.double().requires_grad_(True) for t in (y, scale, shift))
+    out = F.silu(conv * sr.view(1, -1, 1, 1) + br.view(1, -1, 1, 1))
+    ref = torch.autograd.grad(out, (conv, sr, br), gy.double())
+    got = _C.dwconv2d_epilogue_backward(y.to(gpu), gy.to(gpu), scale.to(gpu), shift.to(gpu), "silu")
+    again = _C.dwconv2d_epilogue_backward(y.to(gpu), gy.to(gpu), scale.to(gpu), shift.to(gpu), "silu")
+    assert all(torch.equal(a, b) for a, b in zip(got, again))
+    np.testing.assert_allclose(_np(got[0].double()), ref[0].numpy(), rtol=1e-5 + step, atol=1e-5)
+    for a, b in zip(got[1:], ref[1:]):  # sums of at most 2109 fp32 terms of about one
+        np.testing.assert_allclose(_np(a.double()), b.numpy(), rtol=1e-5, atol=1e-5 * (n * h * w) ** 0.5)
+
+
 def test_fused_epilogue_training_partial_gradients_and_dtypes(dw, gpu):
     """Only the gradients that are asked for come back; 16-bit tensors train through the same path."""
     from torch_dwconv.dwconv import depthwise_conv2d_fused
