@@ -21,11 +21,17 @@
 // the host takes to make the calls.
 #include "dwconv_tile_common.hpp"
 
+#include <algorithm>
+
 namespace dwconv {
 namespace {
 
 constexpr int kMaxThreads = 512;
+constexpr int kMaxWaves = kMaxThreads / 64;
 constexpr int kAtrousLds = 64 * 1024;
+// 16-byte lines of the next plane that a lane holds at most
+constexpr int kMaxAhead = 8;
+static_assert(kMaxAhead * kMaxThreads * 16 >= kAtrousLds, "every plane that make_plan takes is staged whole");
 
 struct AtrousPlan {
     int batch, channel, h, w;
@@ -213,7 +219,7 @@ bool make_plan(AtrousPlan &p, const GeneralGeometry &g, size_t esize)
     // Three workgroups per CU, all resident, so that every one walks several planes; two where the plane's image is
     // large (backward, us, 512 / 768 workgroups: 65x65 fp32 39 / 36, 97x97 bf16 67 / 58; 80x80 fp32 64 / 71, 97x97
     // fp32 109 / 120, 128x128 bf16 136 / 157).
-    const int want = env_int("DWCONV_ATROUS_WGS", plane_bytes > 24 * 1024 ? 2 * kCus : 3 * kCus);
+    const int want = std::max(1, env_int("DWCONV_ATROUS_WGS", plane_bytes > 24 * 1024 ? 2 * kCus : 3 * kCus));
     const int splits = ceil_div(want, g.channel);
     p.per_split = ceil_div(g.batch, splits < g.batch ? splits : g.batch);
     p.splits = ceil_div(g.batch, p.per_split);
@@ -223,7 +229,7 @@ bool make_plan(AtrousPlan &p, const GeneralGeometry &g, size_t esize)
 // Whole wavefronts of chains, spread evenly over as few rounds as kMaxThreads lanes allow.
 int threads_for(const AtrousPlan &p)
 {
-    const int waves = ceil_div(p.chains, 64), most = env_int("DWCONV_ATROUS_WAVES", kMaxThreads / 64);
+    const int waves = ceil_div(p.chains, 64), most = std::clamp(env_int("DWCONV_ATROUS_WAVES", kMaxWaves), 1, kMaxWaves);
     return 64 * ceil_div(waves, ceil_div(waves, most));
 }
 
@@ -238,7 +244,7 @@ template <typename IO, bool FUSED>
 int launch(const AtrousPlan &p, const IO *in, const IO *x, const IO *taps, IO *out, float *partial, hipStream_t stream)
 {
     const int lines = (p.h * p.w * static_cast<int>(sizeof(IO)) + 15 + 15) / 16;
-    const int most = env_int("DWCONV_ATROUS_AHEAD", 8);
+    const int most = std::clamp(env_int("DWCONV_ATROUS_AHEAD", kMaxAhead), ceil_div(lines, kMaxThreads), kMaxAhead);
     // as many wavefronts as the chains keep busy, more where the plane's lines need them
     int threads = threads_for(p);
     while (threads * most < lines) threads += 64;
@@ -246,7 +252,7 @@ int launch(const AtrousPlan &p, const IO *in, const IO *x, const IO *taps, IO *o
     const size_t bytes = lds_for(p, sizeof(IO));
     if (lines <= 3 * threads) hipLaunchKernelGGL((atrous_kernel<IO, FUSED, 3>), grid, block, bytes, stream, p, in, x, taps, out, partial);
     else if (lines <= 5 * threads) hipLaunchKernelGGL((atrous_kernel<IO, FUSED, 5>), grid, block, bytes, stream, p, in, x, taps, out, partial);
-    else hipLaunchKernelGGL((atrous_kernel<IO, FUSED, 8>), grid, block, bytes, stream, p, in, x, taps, out, partial);
+    else hipLaunchKernelGGL((atrous_kernel<IO, FUSED, kMaxAhead>), grid, block, bytes, stream, p, in, x, taps, out, partial);
     return check_launch("atrous_kernel");
 }
 

@@ -1068,6 +1068,34 @@ def test_atrous_plane_kernel(dw, gpu, case, dtype):
         assert torch.equal(torch.isfinite(gw[0, 0]).cpu(), ~met)
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("value", [0, 1, 2, 8, 9, 1 << 24])
+@pytest.mark.parametrize("switch", ["DWCONV_ATROUS_AHEAD", "DWCONV_ATROUS_WAVES", "DWCONV_ATROUS_WGS"])
+def test_atrous_tuning_switches_are_bounded(dw, gpu, switch, value, dtype, monkeypatch):
+    """Any value of the plane kernel's switches that the planners read gives a launch that stages whole planes within its
+    launch bounds: result and grad-input bit for bit (they do not depend on the split), grad-weight to fp32 rounding."""
+    from torch_dwconv import _C
+
+    for n, c, h, w, d in [(3, 2, 127, 128, 6), (5, 3, 21, 19, 3)]:
+        g = torch.Generator("cpu").manual_seed(23)
+        x, gy = (torch.randn(n, c, h, w, generator=g).to(gpu, dtype) for _ in "ab")
+        wt = torch.randn(c, 1, 3, 3, generator=g).to(gpu, dtype)
+
+        def run():
+            y = _C.dwconv2d_general(x, wt, 1, 1, d, d, d, d)
+            return (y, *_C.dwconv2d_general_backward(x, gy, wt, 1, 1, d, d, d, d))
+
+        monkeypatch.delenv("DWCONV_TUNING", raising=False)
+        y, gx, gw = run()
+        monkeypatch.setenv("DWCONV_TUNING", "1")
+        monkeypatch.setenv(switch, str(value))
+        y2, gx2, gw2 = run()
+        assert torch.equal(y, y2) and torch.equal(gx, gx2)
+        # sums of at most 48768 products of unit variance: 2^-24 a step in 32 bits, and one rounding of the format
+        step = 2.0 ** -8 if dtype == torch.bfloat16 else 0.0
+        np.testing.assert_allclose(_np(gw2.double()), _np(gw.double()), rtol=1e-4 + step, atol=1e-4 * (n * h * w) ** 0.5)
+
+
 def test_tuning_overrides_need_the_master_switch(dw, gpu, monkeypatch):
     """DWCONV_* overrides of the planners are ignored unless DWCONV_TUNING=1 is set too, and ill-formed values always."""
     from torch_dwconv import _C
