@@ -150,7 +150,7 @@ __global__ __launch_bounds__(kEpiThreads) void epilogue_bwd_nhwc_kernel(const Ep
     const int pixels = kEpiThreads / p.lanes;
     const int c0 = (blockIdx.x * p.lanes + cl) * CV;
     const int chunk = blockIdx.y;
-    const int o0 = chunk * p.outer_per_chunk, o1 = min(p.outer, o0 + p.outer_per_chunk);
+    const int o0 = chunk * p.outer_per_chunk, o1 = o0 + min(p.outer - o0, p.outer_per_chunk);  // o0 + a chunk may pass 2^31
     const bool live = pl < pixels && c0 < p.channel;
     const IO *const conv = static_cast<const IO *>(p.conv);
     const IO *const gy = static_cast<const IO *>(p.out_grad);
@@ -238,7 +238,7 @@ bool make_plan(EpiBwdPlan &p, int batch, int channel, int out_h, int out_w, bool
         while (static_cast<long>(p.outer_per_chunk) * plane >= (1l << 31)) p.outer_per_chunk = ceil_div(p.outer_per_chunk, 2);
         if (ceil_div(batch, p.outer_per_chunk) > 65535) return false;
     }
-    p.chunks = ceil_div(p.outer, p.outer_per_chunk);
+    p.chunks = static_cast<int>((static_cast<long>(p.outer) + p.outer_per_chunk - 1) / p.outer_per_chunk);  // the sum may pass 2^31
     return true;
 }
 

@@ -1731,6 +1731,19 @@ def test_epilogue_backward_channels_last_lanes(dw, gpu, pixels, channel, dtype):
         np.testing.assert_allclose(_np(a.double()), b.numpy(), rtol=1e-5, atol=1e-5 * (n * h * w) ** 0.5)
 
 
+def test_epilogue_backward_channels_last_near_two_to_the_31_pixels(dw, gpu):
+    """2^31 - 32768 pixels: the last chunk starts below 2^31 and its nominal end lies past it; its pixels are worked on."""
+    from torch_dwconv import _C
+
+    h, w = 65535, 32768
+    y, gy = (torch.zeros(1, h, w, 2, dtype=torch.bfloat16, device=gpu).permute(0, 3, 1, 2) for _ in "ab")
+    y[:, :, -1], gy[:, :, -1] = 2.0, 1.0
+    scale = torch.tensor([3.0, 4.0], device=gpu)
+    got, scale_grad, shift_grad = _C.dwconv2d_epilogue_backward(y, gy, scale, None, None)
+    assert torch.equal(got[0, :, -1].float(), scale.view(2, 1).expand(2, w)) and not bool(got[0, :, -3:-1].any())
+    assert shift_grad.tolist() == [w, w] and scale_grad.tolist() == [2 * w, 2 * w]
+
+
 def test_fused_epilogue_training_partial_gradients_and_dtypes(dw, gpu):
     """Only the gradients that are asked for come back; 16-bit tensors train through the same path."""
     from torch_dwconv.dwconv import depthwise_conv2d_fused
