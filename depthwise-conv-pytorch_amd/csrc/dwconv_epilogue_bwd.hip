@@ -34,7 +34,11 @@ struct EpiBwdPlan {
     int chunks;
     int outer_per_chunk;
     int vec;              // groups of four elements may be moved with one access
-    int lanes;            // channels-last: lanes that one pixel takes in a workgroup
+    // channels-last
+    int lanes;            // lanes that one pixel takes in a workgroup
+    unsigned lanes_magic; // lane / lanes
+    int pixels;           // pixels that a workgroup takes at a time
+    int half;             // the largest power of two below pixels: the first step of the sum over them
 };
 
 // out_grad * d act(z) / dz.  Boundaries as PyTorch's own backward formulas: ReLU passes z > 0, ReLU6 passes 0 < z < 6.
@@ -76,9 +80,8 @@ __device__ __forceinline__ void epi_store(IO *to, const float (&v)[CV])
     else *to = Io<IO>::out(v[0]);
 }
 
-// Accesses to both tensors that a lane of the channels-last kernel has in flight: conv_grad may lie over conv, so the
-// compiler moves no load across a store.
-constexpr int kEpiBatch = 4;
+// Rows of pixels that the end of the channels-last kernel adds in one go, and that a long chunk is a multiple of.
+constexpr int kEpiRows = 4;
 
 // Sum of v over the workgroup, in a fixed order, valid in lane 0.
 __device__ __forceinline__ float block_sum(float v, float *red)
@@ -137,21 +140,26 @@ __global__ __launch_bounds__(kEpiThreads) void epilogue_bwd_nchw_kernel(const Ep
 
 // Channels-last: workgroup (p.lanes lanes of CV channels each, chunk of pixels).  The sweep is bound by HBM when every
 // lane has work: with a wavefront per pixel whatever the channel count, 32 channels kept 8 lanes of 64 busy.  So a
-// workgroup takes 256 / p.lanes pixels at a time, consecutive lanes consecutive addresses across pixels as well, and a
-// lane keeps kEpiBatch pixels in flight.  Batch 128, SiLU, us, a wavefront per pixel / this (TB/s of the three sweeps):
-//   C=32 112x112 fp32 312 / 144 (4.3), bf16 342 / 83 (3.7)    C=96 56x56 fp32 118 / 113 (4.1), bf16 102 / 70 (3.3)
-//   C=144 56x56 fp32 167 / 162 (4.3), bf16 107 / 95 (3.7)     C=1152 7x7 fp32 26.8 / 25.7, bf16 24.2 / 21.2
-// The lanes that share channels are added in order at the end.
+// workgroup takes 256 / p.lanes pixels at a time, consecutive lanes consecutive addresses across pixels as well.  A lane
+// has B pixels of both tensors in flight (conv_grad may lie over conv, so the compiler moves no load across a store): 32
+// bytes of each, more is code that a small pass fetches and runs once (batch 64, C=768, 7x7, fp32: B=4 13.6 us, 2 12.5;
+// batch 128, C=672, 14x14: 52.1 / 51.7, bf16 31.4 / 32.5).  Small passes are bound by latency, of the sum at the end too:
+// the rows of lanes that share channels are halved in LDS down to kEpiRows, which all lanes then add, channel by channel.
+// us, SiLU, a wavefront per pixel / this (TB/s of the three sweeps):
+//   batch 128  C=32 112x112 fp32 312 / 142 (4.4), bf16 344 / 85 (3.6)   C=96 56x56 119 / 113 (4.1), bf16 102 / 71 (3.3)
+//              C=144 56x56 167 / 163 (4.3), bf16 108 / 96 (3.6)         C=240 14x14 31.6 / 31.0, bf16 28.8 / 28.0
+//              C=672 14x14 55.1 / 52.6, bf16 32.5 / 31.5                C=1152 7x7 25.8 / 25.5, bf16 21.0 / 20.3
+//   batch 8    C=4 14x14 8.1 / 6.8    C=32 56x56 22 / 9.2   C=240 28x28 12.4 / 12.4, bf16 11.7 / 12.0   C=1152 7x7 7.6 / 7.6
 template <typename IO, int CV>
 __global__ __launch_bounds__(kEpiThreads) void epilogue_bwd_nhwc_kernel(const EpiBwdPlan p)
 {
+    constexpr int B = CV == 1 ? 1 : 8 / sizeof(IO);
     __shared__ float red[2 * CV][kEpiThreads];
-    const int pl = threadIdx.x / p.lanes, cl = threadIdx.x - pl * p.lanes;
-    const int pixels = kEpiThreads / p.lanes;
+    const int pl = fast_div(threadIdx.x, p.lanes_magic), cl = threadIdx.x - pl * p.lanes;
     const int c0 = (blockIdx.x * p.lanes + cl) * CV;
     const int chunk = blockIdx.y;
     const int o0 = chunk * p.outer_per_chunk, o1 = o0 + min(p.outer - o0, p.outer_per_chunk);  // o0 + a chunk may pass 2^31
-    const bool live = pl < pixels && c0 < p.channel;
+    const bool live = pl < p.pixels && c0 < p.channel;
     const IO *const conv = static_cast<const IO *>(p.conv);
     const IO *const gy = static_cast<const IO *>(p.out_grad);
     IO *const g0 = static_cast<IO *>(p.conv_grad);
@@ -163,19 +171,27 @@ __global__ __launch_bounds__(kEpiThreads) void epilogue_bwd_nhwc_kernel(const Ep
         s_scale[v] = s_shift[v] = 0.f;
     }
     if (live) {
-        const long step = static_cast<long>(pixels) * p.channel;
+        const long step = static_cast<long>(p.pixels) * p.channel;
         long off = static_cast<long>(o0 + pl) * p.channel + c0;
-        for (int left = o1 - o0 - pl; left > 0; left -= kEpiBatch * pixels, off += kEpiBatch * step) {
-            float y[kEpiBatch][CV], g[kEpiBatch][CV];
+        for (int left = o1 - o0 - pl; left > 0; left -= B * p.pixels, off += B * step) {
+            float y[B][CV], g[B][CV];
+            if ((B - 1) * p.pixels < left) {
 #pragma unroll
-            for (int u = 0; u < kEpiBatch; ++u) {
-                const long at = u * pixels < left ? off + u * step : off;  // past the chunk: this lane's own first pixel again
-                epi_load<IO, CV>(conv + at, y[u]);
-                epi_load<IO, CV>(gy + at, g[u]);
+                for (int u = 0; u < B; ++u) {
+                    epi_load<IO, CV>(conv + off + u * step, y[u]);
+                    epi_load<IO, CV>(gy + off + u * step, g[u]);
+                }
+            } else {
+#pragma unroll
+                for (int u = 0; u < B - 1; ++u) {
+                    if (u * p.pixels >= left) break;
+                    epi_load<IO, CV>(conv + off + u * step, y[u]);
+                    epi_load<IO, CV>(gy + off + u * step, g[u]);
+                }
             }
 #pragma unroll
-            for (int u = 0; u < kEpiBatch; ++u) {
-                if (u * pixels >= left) break;
+            for (int u = 0; u < B; ++u) {
+                if (u * p.pixels >= left) break;
                 float out[CV];
 #pragma unroll
                 for (int v = 0; v < CV; ++v) out[v] = epi_element(y[u][v], g[u][v], sc[v], sh[v], p.act, s_scale[v], s_shift[v]);
@@ -189,17 +205,33 @@ __global__ __launch_bounds__(kEpiThreads) void epilogue_bwd_nhwc_kernel(const Ep
         red[2 * v + 1][threadIdx.x] = s_shift[v];
     }
     __syncthreads();
-    if (pl == 0 && live) {
+    int rows = p.pixels;
+    for (int half = p.half; half >= kEpiRows; half >>= 1) {
+        if (pl < half && pl + half < rows) {
 #pragma unroll
-        for (int v = 0; v < CV; ++v) {
-            float a = red[2 * v][cl], b = red[2 * v + 1][cl];
-            for (int w = 1; w < pixels; ++w) {
-                a += red[2 * v][w * p.lanes + cl];
-                b += red[2 * v + 1][w * p.lanes + cl];
-            }
-            float *dst = p.partial + (static_cast<long>(c0 + v) * p.chunks + chunk) * 2;
-            dst[0] = a;
-            dst[1] = b;
+            for (int v = 0; v < 2 * CV; ++v) red[v][threadIdx.x] += red[v][threadIdx.x + half * p.lanes];
+        }
+        rows = half;
+        __syncthreads();
+    }
+    for (int i = threadIdx.x; i < CV * p.lanes; i += kEpiThreads) {
+        const int v = fast_div(i, p.lanes_magic), lane = i - v * p.lanes, c = (blockIdx.x * p.lanes + lane) * CV + v;
+        float a[kEpiRows], b[kEpiRows];
+#pragma unroll
+        for (int r = 0; r < kEpiRows; ++r) {
+            const int at = min(r, rows - 1) * p.lanes + lane;
+            a[r] = red[2 * v][at];
+            b[r] = red[2 * v + 1][at];
+        }
+#pragma unroll
+        for (int r = 1; r < kEpiRows; ++r) {
+            a[0] += r < rows ? a[r] : 0.f;
+            b[0] += r < rows ? b[r] : 0.f;
+        }
+        if (c < p.channel) {
+            float *dst = p.partial + (static_cast<long>(c) * p.chunks + chunk) * 2;
+            dst[0] = a[0];
+            dst[1] = b[0];
         }
     }
 }
@@ -223,10 +255,16 @@ bool make_plan(EpiBwdPlan &p, int batch, int channel, int out_h, int out_w, bool
         int chunks = ceil_div(2048, groups);
         chunks = std::max(1, std::min(chunks, std::min(ceil_div(p.outer, 16), 65535)));
         p.outer_per_chunk = ceil_div(p.outer, chunks);
-        // whole batches of pixels: a chunk that ends inside one issues its loads and works on a part of them
-        // (batch 128, C=480, 14x14, us: bf16 29.6 without / 28.1 with, fp32 43.8 / 42.3)
-        const int batch_pixels = kEpiBatch * (kEpiThreads / lanes_for(channel % 4 == 0 ? channel / 4 : channel));
-        if (p.outer_per_chunk > batch_pixels) p.outer_per_chunk = ceil_div(p.outer_per_chunk, batch_pixels) * batch_pixels;
+        // A chunk takes the pixels that a workgroup works on at a time, or whole multiples of them, and up to kEpiRows times
+        // as many where that leaves 128 chunks or more: partial sums are the larger part of a small pass (batch 8, fp32,
+        // C=8 56x56: chunks of 16 pixels 26.7 us, of a workgroup's 128 and more 7.3).  Longer chunks are whole batches of four
+        // (batch 128, 28x28, C=80 bf16: multiples of one 28.7, of four 24.9; batch 100, 50x50, C=36 30.0 / 25.8), except
+        // where lanes hold single elements and the workgroups' balance counts for more (128x255x14x14 bf16 21.2 / 24.0).
+        const bool quads = channel % 4 == 0;
+        const int pixels = kEpiThreads / lanes_for(quads ? channel / 4 : channel), batch_pixels = kEpiRows * pixels;
+        p.outer_per_chunk = std::max(p.outer_per_chunk, std::min(batch_pixels, ceil_div(p.outer, 128)));
+        const int unit = quads && p.outer_per_chunk > batch_pixels ? batch_pixels : pixels;
+        p.outer_per_chunk = ceil_div(p.outer_per_chunk, unit) * unit;
     } else {
         if (plane >= (1l << 30)) return false;
         p.outer = batch;
@@ -274,6 +312,9 @@ int epilogue_backward(const IO *conv, const IO *out_grad, const float *scale, co
         p.vec = aligned && channel % 4 == 0;
         const int groups = p.vec ? channel / 4 : channel;
         p.lanes = lanes_for(groups);
+        p.lanes_magic = magic_u16(static_cast<unsigned>(p.lanes));
+        p.pixels = kEpiThreads / p.lanes;
+        for (p.half = 1; 2 * p.half < p.pixels;) p.half *= 2;
         const dim3 grid(ceil_div(groups, p.lanes), p.chunks);
         if (p.vec) hipLaunchKernelGGL((epilogue_bwd_nhwc_kernel<IO, 4>), grid, dim3(kEpiThreads), 0, stream, p);
         else hipLaunchKernelGGL((epilogue_bwd_nhwc_kernel<IO, 1>), grid, dim3(kEpiThreads), 0, stream, p);

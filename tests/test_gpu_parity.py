@@ -1731,6 +1731,44 @@ def test_epilogue_backward_channels_last_lanes(dw, gpu, pixels, channel, dtype):
         np.testing.assert_allclose(_np(a.double()), b.numpy(), rtol=1e-5, atol=1e-5 * (n * h * w) ** 0.5)
 
 
+# (channel, N, H, W, lanes of a pixel): chunks of several batches of pixels, the last one ending inside a batch; channels in
+# fours (one lane to several shares) and singly
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=["f32", "f16", "bf16"])
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("case", [(4, 3, 839, 839, 1), (32, 5, 231, 229, 8), (96, 3, 165, 167, 24), (260, 2, 111, 113, 40),
+                                  (1152, 7, 31, 31, 64), (37, 3, 129, 129, 37), (255, 3, 53, 53, 64)], ids=str)
+def test_epilogue_backward_channels_last_long_chunks(dw, gpu, case, offset, dtype):
+    """More pixels than 2048 workgroups take in one go, in place, also from a storage offset that leaves only accesses of
+    single elements; against fp64 torch, bit-identical on a second run."""
+    import torch.nn.functional as F
+
+    from torch_dwconv import _C
+
+    channel, n, h, w, lanes = case
+    step = {torch.float32: 1e-6, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dtype]
+    g = torch.Generator(gpu).manual_seed(7)
+
+    def activations():
+        flat = torch.randn(n * h * w * channel + offset, generator=g, device=gpu).to(dtype)
+        return flat[offset:].view(n, h, w, channel).permute(0, 3, 1, 2)
+
+    y, gy = activations(), activations()
+    scale, shift = torch.rand(channel, generator=g, device=gpu) + 0.5, torch.randn(channel, generator=g, device=gpu)
+    conv, sr, br = (t.double().requires_grad_(True) for t in (y, scale, shift))
+    ref = torch.autograd.grad(F.silu(conv * sr.view(1, -1, 1, 1) + br.view(1, -1, 1, 1)), (conv, sr, br), gy.double())
+    first = [t.clone() for t in _C.dwconv2d_epilogue_backward(y.clone(), gy, scale, shift, "silu")]
+    got = _C.dwconv2d_epilogue_backward(y, gy, scale, shift, "silu")
+    variant = _C.last_variant()
+    _announce(case, str(dtype), variant)
+    assert got[0] is y and ("v4>" in variant) == (channel % 4 == 0 and offset == 0), variant
+    assert n * h * w / int(variant.rsplit("chunks", 1)[1]) > 4 * (256 // lanes), variant
+    if offset == 0:
+        assert all(torch.equal(a, b) for a, b in zip(got, first))
+    assert bool(((got[0].double() - ref[0]).abs() <= (1e-5 + step) * ref[0].abs() + 1e-5).all())
+    for a, b in zip(got[1:], ref[1:]):  # sums of fp32 terms of about one
+        assert bool(((a.double() - b).abs() <= 1e-5 * b.abs() + 1e-5 * (n * h * w) ** 0.5).all())
+
+
 def test_epilogue_backward_channels_last_near_two_to_the_31_pixels(dw, gpu):
     """2^31 - 32768 pixels: the last chunk starts below 2^31 and its nominal end lies past it; its pixels are worked on."""
     from torch_dwconv import _C
