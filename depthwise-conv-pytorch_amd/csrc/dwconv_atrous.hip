@@ -1,4 +1,4 @@
-// Dilated 3x3 layers at stride 1 with "same" padding (pad == dilation), any dilation: forward, and both gradients in one
+// Dilated 3x3 layers at stride 1 with "same" padding (pad == dilation), any dilation (make_plan says where): forward, and both gradients in one
 // sweep over out_grad.
 //
 // What bounds them is how much is moved per useful byte: with rates of 6 to 18 on maps of 33 to 97 columns the zero
@@ -199,7 +199,8 @@ __global__ __launch_bounds__(kMaxThreads) void atrous_kernel(const AtrousPlan p,
     }
 }
 
-bool make_plan(AtrousPlan &p, const GeneralGeometry &g, size_t esize)
+// fused: for the backward kernel.
+bool make_plan(AtrousPlan &p, const GeneralGeometry &g, size_t esize, bool fused)
 {
     if (g.multiplier != 1 || g.kernel_h != 3 || g.kernel_w != 3 || g.stride_h != 1 || g.stride_w != 1) return false;
     if (g.pad_h != g.dil_h || g.pad_w != g.dil_w || g.batch < 1 || g.channel < 1 || g.in_h < 1 || g.in_w < 1) return false;
@@ -216,10 +217,38 @@ bool make_plan(AtrousPlan &p, const GeneralGeometry &g, size_t esize)
     p.chains = p.dh * p.w;
     p.steps = ceil_div(p.h, p.dh);
     p.w_magic = magic_u16(static_cast<unsigned>(p.w));
-    // Three workgroups per CU, all resident, so that every one walks several planes; two where the plane's image is
-    // large (backward, us, 512 / 768 workgroups: 65x65 fp32 39 / 36, 97x97 bf16 67 / 58; 80x80 fp32 64 / 71, 97x97
-    // fp32 109 / 120, 128x128 bf16 136 / 157).
-    const int want = std::max(1, env_int("DWCONV_ATROUS_WGS", plane_bytes > 24 * 1024 ? 2 * kCus : 3 * kCus));
+    // Workgroups per CU: two or three walk several planes each where a plane's image or chains fill the CU (backward, us,
+    // 512 / 768 workgroups: 65x65 fp32 39 / 36, 97x97 bf16 67 / 58; 80x80 fp32 64 / 71, 97x97 fp32 109 / 120, 128x128 bf16
+    // 136 / 157).  Small planes are bound by the latency of a step, so up to 16 wavefronts of them, 24 of one each, and
+    // eight in the forward pass once their bytes count (forward and backward, us, three a CU / these: batch 128, C=960 7x7
+    // rate 3 fp32 86 and 129 / 31 and 42, C=480 14x14 56 and 88 / 24 and 36; batch 64, C=256 33x33 rate 6 30 and 44 / 27
+    // and 42; with 12 a CU, batch 171, C=164 39x39 rate 3 forward 68 / 76).
+    const int lanes = std::min(round_up(p.chains, 64), kMaxThreads);
+    int per_cu = plane_bytes > 24 * 1024 ? 2 : 3;
+    if (plane_bytes <= 12 * 1024) {
+        const int waves = lanes == 64 ? 24 : fused || plane_bytes <= 4 * 1024 ? 16 : 8;
+        per_cu = std::max(per_cu, std::min(waves * 64 / lanes, static_cast<int>(2 * kAtrousLds / (plane_bytes + 48))));
+    }
+    // A chain is walked row by row and a plane is never split, so a long chain takes as long as it takes whatever else the
+    // CU does.  The any-geometry kernels split planes into bands: better where too few columns are in flight for the rows
+    // there are, and the less so the more of their staging is padding or rows that are not a multiple of four long.  us,
+    // any-geometry / this, fp32, rates vertical x horizontal:
+    //   forward   batch 16, C=64: 400x40 1x2 34 / 68, 1000x16 1x3 57 / 227, 80x80 1x2 14 / 18; batch 4, C=32 97x97 1x2 7.8 / 10
+    //             but 65x130 1x3 25 / 18, 120x60 2x3 21 / 15, 200x60 3x3 32 / 23; batch 7, C=712 278x26 3x3 106 / 80
+    //   backward  batch 16, C=64: 400x40 1x2 88 / 133; batch 1, C=52 639x14 3x6 20 / 27
+    //             but 120x120 1x2 79 / 52; batch 3, C=778 555x8 3x3 155 / 96
+    const int serial = p.steps * ceil_div(p.chains, kMaxThreads);
+    if (serial > 48) {
+        const float planes = 1.f * g.batch * g.channel / kCus, ragged = p.w % 4 != 0 ? 1.4f : 1.f;
+        const float padded = (1.f + 2.f * p.dh / p.h) * (1.f + 2.f * p.dw / p.w);
+        const float columns = std::min<float>(per_cu, planes) * std::min(p.chains, kMaxThreads) * padded * ragged;
+        if (fused) {
+            if (serial > 160 && columns < 110.f) return false;
+        } else if (p.dh > 2) {
+            if (serial > 64 && planes < 1.f && columns < 140.f) return false;
+        } else if (columns < (p.dh == 2 ? 125.f : p.dw > 3 ? 200.f : 265.f)) return false;
+    }
+    const int want = std::max(1, env_int("DWCONV_ATROUS_WGS", per_cu * kCus));
     const int splits = ceil_div(want, g.channel);
     p.per_split = ceil_div(g.batch, splits < g.batch ? splits : g.batch);
     p.splits = ceil_div(g.batch, p.per_split);
@@ -261,14 +290,14 @@ int launch(const AtrousPlan &p, const IO *in, const IO *x, const IO *taps, IO *o
 size_t atrous_workspace(const GeneralGeometry &g, size_t esize)
 {
     AtrousPlan p;
-    return make_plan(p, g, esize) ? static_cast<size_t>(p.channel) * p.splits * 9 * sizeof(float) : 0;
+    return make_plan(p, g, esize, true) ? static_cast<size_t>(p.channel) * p.splits * 9 * sizeof(float) : 0;
 }
 
 template <typename IO>
 int try_launch_atrous_forward(const IO *in, const IO *taps, IO *out, const GeneralGeometry &g, hipStream_t stream)
 {
     AtrousPlan p;
-    if (!make_plan(p, g, sizeof(IO))) return -1;
+    if (!make_plan(p, g, sizeof(IO), false)) return -1;
     note_variant("tile_any%s<k3x3,s1x1,d%dx%d,fwd> plane", sizeof(IO) == 2 ? "16" : "", g.dil_h, g.dil_w);
     return launch<IO, false>(p, in, in, taps, out, nullptr, stream);
 }
@@ -278,7 +307,7 @@ int try_launch_atrous_backward(const IO *in, const IO *gy, const IO *taps, IO *g
                                const GeneralGeometry &g, hipStream_t stream)
 {
     AtrousPlan p;
-    if (!make_plan(p, g, sizeof(IO))) return -1;
+    if (!make_plan(p, g, sizeof(IO), true)) return -1;
     const size_t need = static_cast<size_t>(p.channel) * p.splits * 9 * sizeof(float);
     if (ws == nullptr || ws_bytes < need)
         return fail(DWCONV_ERR_WORKSPACE, "grad-weight needs a workspace of %zu bytes, got %zu", need, ws_bytes);

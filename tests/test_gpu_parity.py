@@ -1042,7 +1042,7 @@ def test_atrous_plane_kernel(dw, gpu, case, dtype):
     _announce(case, str(dtype), _C.last_variant())
     gx, gw = _C.dwconv2d_general_backward(xg, gyg, wg, 1, 1, dh, dw_, dh, dw_)
     planes = h * w * x.element_size() + 48 <= 64 * 1024
-    assert _C.last_variant().endswith(" plane") == (planes and not (dh == dw_ == 2)), _C.last_variant()
+    assert (" plane" in _C.last_variant()) == (planes and not (dh == dw_ == 2)), _C.last_variant()
     gx2, gw2 = _C.dwconv2d_general_backward(xg, gyg, wg, 1, 1, dh, dw_, dh, dw_)
     assert torch.equal(gx, gx2) and torch.equal(gw, gw2)
     tol, gtol = 1e-5 + step, 1e-4 + step
@@ -1066,6 +1066,40 @@ def test_atrous_plane_kernel(dw, gpu, case, dtype):
         _, gw = _C.dwconv2d_general_backward(xg, gyg, wg, 1, 1, dh, dw_, dh, dw_)
         met = torch.outer(torch.tensor([False, True, h > dh]), torch.tensor([False, True, w > dw_]))
         assert torch.equal(torch.isfinite(gw[0, 0]).cpu(), ~met)
+
+
+# (N, C, H, W, dil_h, dil_w), forward and backward through the plane kernel: either side of the rule on long chains
+ATROUS_RULE = [
+    ((2, 3, 48, 20, 1, 2), (True, True)), ((2, 3, 49, 20, 1, 2), (False, True)), ((2, 3, 161, 20, 1, 2), (False, False)),
+    ((2, 3, 66, 33, 3, 2), (True, True)), ((2, 3, 195, 7, 3, 2), (False, True)), ((2, 3, 486, 7, 3, 2), (False, False)),
+    ((1, 64, 97, 48, 2, 3), (False, True)), ((3, 256, 64, 64, 1, 2), (False, True)), ((3, 256, 49, 131, 1, 2), (True, True)),
+    ((3, 256, 110, 60, 2, 3), (True, True)), ((3, 257, 162, 21, 1, 2), (False, False)), ((3, 257, 162, 60, 1, 2), (False, True)),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("case,plane", ATROUS_RULE, ids=str)
+def test_atrous_long_chains(dw, gpu, case, plane, dtype):
+    """Long chains with few columns in flight stay with the any-geometry kernels, per direction; against fp64 on the rounded
+    inputs whichever runs."""
+    from torch_dwconv import _C
+
+    n, c, h, w, dh, dw_ = case
+    g = torch.Generator("cpu").manual_seed(29)
+    x, gy = (torch.randn(n, c, h, w, generator=g).to(dtype) for _ in "ab")
+    wt = (torch.randn(c, 1, 3, 3, generator=g) / 3).to(dtype)
+    xr, wr = x.double().requires_grad_(True), wt.double().requires_grad_(True)
+    y_ref = torch.nn.functional.conv2d(xr, wr, padding=(dh, dw_), dilation=(dh, dw_), groups=c)
+    gx_ref, gw_ref = torch.autograd.grad(y_ref, (xr, wr), gy.double())
+    y = _C.dwconv2d_general(x.to(gpu), wt.to(gpu), 1, 1, dh, dw_, dh, dw_)
+    forward = " plane" in _C.last_variant()
+    gx, gw = _C.dwconv2d_general_backward(x.to(gpu), gy.to(gpu), wt.to(gpu), 1, 1, dh, dw_, dh, dw_)
+    assert (forward, " plane" in _C.last_variant()) == plane, (forward, _C.last_variant())
+    step = 2.0 ** -8 if dtype == torch.bfloat16 else 0.0
+    np.testing.assert_allclose(_np(y.double()), y_ref.detach().numpy(), rtol=1e-5 + step, atol=1e-5 + step)
+    np.testing.assert_allclose(_np(gx.double()), gx_ref.numpy(), rtol=1e-5 + step, atol=1e-5 + step)
+    gtol = 1e-4 + step
+    np.testing.assert_allclose(_np(gw.double()), gw_ref.numpy(), rtol=gtol, atol=gtol * float(gw_ref.abs().max()))
 
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
