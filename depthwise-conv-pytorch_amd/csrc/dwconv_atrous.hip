@@ -150,14 +150,17 @@ __global__ __launch_bounds__(kMaxThreads) void atrous_kernel(const AtrousPlan p,
                     view_put<IO>(outs, s + k > 0 ? at + k * step - step : kOob, done);
                     if constexpr (FUSED) {
                         const float x_after = k == 0 ? x_now[1] : x_next[0];
-                        // a position past the plane meets no input: the row above it may hold one that is not finite
+                        // Padding meets nothing, so that a value that is not finite stays out of the sums it has no part in:
+                        // a position past the plane meets no input of the row before, the first row has none before it
+                        // and the last one none after it.
                         const float x_before = at + k * step < plane_bytes ? x_prev : 0.f;
+                        const bool has_after = at + (k + 1) * step < plane_bytes;
 #pragma unroll
                         for (int j = 0; j < 3; ++j) {
                             // out_grad at column col + (j - 1) * dw meets input column col through tap column 2 - j
-                            acc[2 - j] = fmaf(x_before, v[k][j], acc[2 - j]);
+                            if (s + k > 0) acc[2 - j] = fmaf(x_before, v[k][j], acc[2 - j]);
                             acc[3 + 2 - j] = fmaf(x_now[k], v[k][j], acc[3 + 2 - j]);
-                            acc[6 + 2 - j] = fmaf(x_after, v[k][j], acc[6 + 2 - j]);
+                            acc[6 + 2 - j] = fmaf(x_after, has_after ? v[k][j] : 0.f, acc[6 + 2 - j]);
                         }
                         x_prev = x_now[k];
                     }

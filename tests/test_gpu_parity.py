@@ -1066,6 +1066,15 @@ def test_atrous_plane_kernel(dw, gpu, case, dtype):
         _, gw = _C.dwconv2d_general_backward(xg, gyg, wg, 1, 1, dh, dw_, dh, dw_)
         met = torch.outer(torch.tensor([False, True, h > dh]), torch.tensor([False, True, w > dw_]))
         assert torch.equal(torch.isfinite(gw[0, 0]).cpu(), ~met)
+        # nor does an out_grad that is not finite meet the padding: every corner reaches the taps that lead into the map
+        xg[0, 0, h - 1, w - 1] = 0.0
+        for r, q in {(0, 0), (0, w - 1), (h - 1, 0), (h - 1, w - 1)}:
+            gyi = gyg.clone()
+            gyi[0, 0, r, q] = float("inf")
+            _, gw = _C.dwconv2d_general_backward(xg, gyi, wg, 1, 1, dh, dw_, dh, dw_)
+            met = torch.outer(torch.tensor([0 <= r + i * dh < h for i in (-1, 0, 1)]),
+                              torch.tensor([0 <= q + j * dw_ < w for j in (-1, 0, 1)]))
+            assert torch.equal(torch.isfinite(gw[0, 0]).cpu(), ~met), (r, q)
 
 
 # (N, C, H, W, dil_h, dil_w), forward and backward through the plane kernel: either side of the rule on long chains
