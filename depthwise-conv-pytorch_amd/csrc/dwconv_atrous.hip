@@ -301,7 +301,7 @@ int try_launch_atrous_forward(const IO *in, const IO *taps, IO *out, const Gener
 {
     AtrousPlan p;
     if (!make_plan(p, g, sizeof(IO), false)) return -1;
-    note_variant("tile_any%s<k3x3,s1x1,d%dx%d,fwd> plane", sizeof(IO) == 2 ? "16" : "", g.dil_h, g.dil_w);
+    note_variant("atrous%s<k3x3,d%dx%d,fwd> splits%d images%d", sizeof(IO) == 2 ? "16" : "", g.dil_h, g.dil_w, p.splits, p.per_split);
     return launch<IO, false>(p, in, in, taps, out, nullptr, stream);
 }
 
@@ -314,9 +314,7 @@ int try_launch_atrous_backward(const IO *in, const IO *gy, const IO *taps, IO *g
     const size_t need = static_cast<size_t>(p.channel) * p.splits * 9 * sizeof(float);
     if (ws == nullptr || ws_bytes < need)
         return fail(DWCONV_ERR_WORKSPACE, "grad-weight needs a workspace of %zu bytes, got %zu", need, ws_bytes);
-    const char *sfx = sizeof(IO) == 2 ? "16" : "";
-    note_variant("tile_any%s<k3x3,s1x1,d%dx%d,rot> + wgrad_any%s<k3x3,s1x1,d%dx%d> passes1 plane", sfx, g.dil_h, g.dil_w, sfx,
-                 g.dil_h, g.dil_w);
+    note_variant("atrous_bwd%s<k3x3,d%dx%d> splits%d images%d", sizeof(IO) == 2 ? "16" : "", g.dil_h, g.dil_w, p.splits, p.per_split);
     const int rc = launch<IO, true>(p, gy, in, taps, gx, static_cast<float *>(ws), stream);
     if (rc != DWCONV_OK) return rc;
     return launch_wgrad_final(static_cast<const float *>(ws), gw, p.channel, 9, p.splits, stream);

@@ -876,12 +876,16 @@ def any_geometry_walks(kh, kw, sh, sw, dh, dw_):
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=["f32", "f16", "bf16"])
 @pytest.mark.parametrize("case", ANY_GEOMETRY, ids=lambda c: "N%d_C%d_%dx%d_k%dx%d_s%dx%d_p%dx%d_d%dx%d" % c)
-def test_any_geometry_tiled_kernels(dw, gpu, case, dtype):
+def test_any_geometry_tiled_kernels(dw, gpu, case, dtype, monkeypatch):
     """Rectangular, even-sized and strip filters, strides above 2 and dilations above 2: forward, grad-input (the
     correlation with the rotated taps where the stride is 1) and grad-weight through the tiled kernels that loop over
-    their taps at run time, against fp64 autograd on the rounded inputs; bit-identical grad-weight."""
+    their taps at run time, against fp64 autograd on the rounded inputs; bit-identical grad-weight.  The plane kernel,
+    which takes the dilated 3x3 cases with "same" padding, is off."""
     from torch_dwconv import _C
     from torch_dwconv.dwconv import depthwise_conv2d_general
+
+    monkeypatch.setenv("DWCONV_TUNING", "1")
+    monkeypatch.setenv("DWCONV_ATROUS", "0")
 
     n, c, h, w, kh, kw, sh, sw, ph, pw, dh, dw_ = case
     step = {torch.float32: 0.0, torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dtype]
@@ -1016,6 +1020,8 @@ ATROUS = [
     (3, 5, 7, 9, 3, 3), (2, 3, 5, 5, 4, 4), (2, 3, 6, 11, 6, 11), (2, 2, 9, 13, 40, 50), (5, 3, 33, 35, 6, 12),
     (2, 7, 64, 64, 18, 18), (3, 2, 65, 65, 12, 12), (2, 3, 97, 97, 18, 6), (1, 2, 127, 129, 6, 6), (1, 2, 130, 131, 5, 5),
     (40, 2, 20, 17, 3, 5), (1, 1, 3, 40, 3, 2), (1, 2, 1, 37, 2, 5), (2, 2, 41, 1, 6, 3),
+    # several planes to a workgroup, the last workgroup of a channel with fewer
+    (7, 256, 33, 35, 6, 12), (7, 256, 65, 65, 12, 12), (67, 256, 13, 11, 3, 4), (11, 130, 47, 31, 5, 5),
 ]
 
 
@@ -1039,10 +1045,18 @@ def test_atrous_plane_kernel(dw, gpu, case, dtype):
     gx_ref, gw_ref = torch.autograd.grad(y_ref, (xr, wr), gy.double())
     xg, wg, gyg = x.to(gpu), wt.to(gpu), gy.to(gpu)
     y = depthwise_conv2d_general(xg, wg, padding=(dh, dw_), dilation=(dh, dw_))
-    _announce(case, str(dtype), _C.last_variant())
+    v_fwd = _C.last_variant()
     gx, gw = _C.dwconv2d_general_backward(xg, gyg, wg, 1, 1, dh, dw_, dh, dw_)
+    v_bwd = _C.last_variant()
+    _announce(case, str(dtype), v_fwd, v_bwd)
     planes = h * w * x.element_size() + 48 <= 64 * 1024
-    assert (" plane" in _C.last_variant()) == (planes and not (dh == dw_ == 2)), _C.last_variant()
+    sfx = "" if dtype == torch.float32 else "16"
+    assert v_fwd.startswith("atrous%s<k3x3,d%dx%d,fwd>" % (sfx, dh, dw_)) == planes, v_fwd
+    assert v_bwd.startswith("atrous_bwd%s<k3x3,d%dx%d>" % (sfx, dh, dw_)) == planes, v_bwd
+    if c >= 130:
+        for v in (v_fwd, v_bwd):
+            splits, images = (int(v.split(key)[1].split()[0]) for key in ("splits", "images"))
+            assert images >= 2 and (splits - 1) * images < n < splits * images, v
     gx2, gw2 = _C.dwconv2d_general_backward(xg, gyg, wg, 1, 1, dh, dw_, dh, dw_)
     assert torch.equal(gx, gx2) and torch.equal(gw, gw2)
     tol, gtol = 1e-5 + step, 1e-4 + step
@@ -1101,9 +1115,9 @@ def test_atrous_long_chains(dw, gpu, case, plane, dtype):
     y_ref = torch.nn.functional.conv2d(xr, wr, padding=(dh, dw_), dilation=(dh, dw_), groups=c)
     gx_ref, gw_ref = torch.autograd.grad(y_ref, (xr, wr), gy.double())
     y = _C.dwconv2d_general(x.to(gpu), wt.to(gpu), 1, 1, dh, dw_, dh, dw_)
-    forward = " plane" in _C.last_variant()
+    forward = _C.last_variant().startswith("atrous")
     gx, gw = _C.dwconv2d_general_backward(x.to(gpu), gy.to(gpu), wt.to(gpu), 1, 1, dh, dw_, dh, dw_)
-    assert (forward, " plane" in _C.last_variant()) == plane, (forward, _C.last_variant())
+    assert (forward, _C.last_variant().startswith("atrous_bwd")) == plane, (forward, _C.last_variant())
     step = 2.0 ** -8 if dtype == torch.bfloat16 else 0.0
     np.testing.assert_allclose(_np(y.double()), y_ref.detach().numpy(), rtol=1e-5 + step, atol=1e-5 + step)
     np.testing.assert_allclose(_np(gx.double()), gx_ref.numpy(), rtol=1e-5 + step, atol=1e-5 + step)
@@ -2061,7 +2075,9 @@ def test_dilation_and_depth_multiplier(dw, gpu, case, dtype):
     elif plain:
         assert not v_fwd.startswith("general_fwd"), v_fwd  # the plain case runs the tuned kernels
     elif m == 1 and dtype != torch.float64:
-        assert v_fwd.startswith("tile_any<k%dx%d,s%dx%d,d%dx%d" % (kh, kw, s, s, d, d)), v_fwd  # any other dilation / stride
+        plane = (kh, kw, s, p) == (3, 3, 1, d)  # "same" 3x3 layers; else any other dilation / stride
+        name = "atrous<k3x3,d%dx%d,fwd>" % (d, d) if plane else "tile_any<k%dx%d,s%dx%d,d%dx%d" % (kh, kw, s, s, d, d)
+        assert v_fwd.startswith(name), v_fwd
     elif m == 1:
         # double tensors: the fp64 tiled kernels, with dilated taps; backward as two passes (grad-input of a stride-1
         # layer through the same kernel with rotated taps)
