@@ -117,6 +117,7 @@ void input_and_kernel(const Tensor &input, const Tensor &kernel)
     together(input, kernel);
 }
 
+// An uninitialised result; at::empty_like where it takes the strides of an argument (those of axes of one element are free).
 Tensor empty_like_format(const Tensor &t, at::IntArrayRef sizes, at::MemoryFormat format)
 {
     return at::empty(sizes, t.options().requires_grad(false), format);
@@ -220,7 +221,7 @@ PyObject *conv_small(Args a)
     const Type type = type_of(input);
     const Tensor x = input.contiguous(), k = kernel.contiguous();
     const int n = extent(x, 0), c = extent(x, 1), h = extent(x, 2), w = extent(x, 3), kh = extent(k, 2), kw = extent(k, 3);
-    const Tensor y = empty_like_format(x, x.sizes(), at::MemoryFormat::Contiguous);
+    const Tensor y = at::empty_like(x);
 #define DWCONV_CALL(T, FN)                                                                                            \
     call(x, [&](void *s) {                                                                                            \
         return FN(in<T>(x), in<T>(k), out<T>(y), n, c, h, w, kh, kw, v[0], v[1], v[2], v[3], v[4], v[5], forward, s); \
@@ -244,8 +245,8 @@ PyObject *backward(Args a)
     const Tensor x = input.contiguous(), gy = grad.contiguous(), k = kernel.contiguous();
     const int n = extent(x, 0), c = extent(x, 1), h = extent(x, 2), w = extent(x, 3), oh = extent(gy, 2), ow = extent(gy, 3);
     const int kh = extent(k, 2), kw = extent(k, 3);
-    const Tensor gx = empty_like_format(x, x.sizes(), at::MemoryFormat::Contiguous);
-    const Tensor gw = empty_like_format(k, k.sizes(), at::MemoryFormat::Contiguous);
+    const Tensor gx = at::empty_like(x);
+    const Tensor gw = at::empty_like(k);
     const size_t bytes = dwconv2d_backward_kernel_workspace_bytes(n, c, h, w, oh, ow, kh, kw, sh, sw, ph, pw,
                                                                   static_cast<int>(x.element_size()));
     const Tensor ws = workspace(x, bytes);
@@ -301,7 +302,7 @@ PyObject *backward_nhwc(Args a)
     const int kh = extent(k, 2), kw = extent(k, 3);
     Tensor gx, gw;
     if (need_x) gx = empty_like_format(x, x.sizes(), at::MemoryFormat::ChannelsLast);
-    if (need_w) gw = empty_like_format(k, k.sizes(), at::MemoryFormat::Contiguous);
+    if (need_w) gw = at::empty_like(k);
     const size_t bytes = dwconv2d_backward_nhwc_workspace_bytes(n, c, h, w, kh, kw, sh, sw, ph, pw, static_cast<int>(x.element_size()));
     const Tensor ws = workspace(x, bytes);
 #define DWCONV_CALL(T, FN)                                                                                                  \
@@ -436,8 +437,8 @@ PyObject *general_backward(Args a)
     const Tensor x = input.contiguous(), gy = grad.contiguous(), k = kernel.contiguous();
     const int n = extent(x, 0), c = extent(x, 1), h = extent(x, 2), w = extent(x, 3), oh = extent(gy, 2), ow = extent(gy, 3);
     const int kh = extent(k, 2), kw = extent(k, 3);
-    const Tensor gx = empty_like_format(x, x.sizes(), at::MemoryFormat::Contiguous);
-    const Tensor gw = empty_like_format(k, k.sizes(), at::MemoryFormat::Contiguous);
+    const Tensor gx = at::empty_like(x);
+    const Tensor gw = at::empty_like(k);
     const size_t bytes = dwconv2d_general_backward_workspace_bytes(n, c, h, w, m, kh, kw, v[0], v[1], v[2], v[3], v[4], v[5],
                                                                    static_cast<int>(x.element_size()));
     const Tensor ws = workspace(x, bytes);

@@ -1014,6 +1014,33 @@ def test_native_calls_equal_the_python_ones(dw, gpu, call, dtype, monkeypatch):
     assert native.conv(x, w, 1, 1, 1, 1) is None and native.conv(x.int(), w.int(), 1, 1, 1, 1, 1, 1, 1, 1, 1) is None
 
 
+@pytest.mark.parametrize("shape", [(2, 1, 9, 11), (1, 8, 9, 11), (2, 8, 1, 11), (1, 1, 9, 11)], ids=str)
+@pytest.mark.parametrize("call", NATIVE_CALLS, ids=lambda c: "%s_%s%s" % (c[0], c[1], "_nhwc" if c[3] else ""))
+def test_native_calls_keep_strides_of_single_elements(dw, gpu, call, shape, monkeypatch):
+    """Tensors that are dense NCHW and channels-last at once (one channel, filters of (C,1,K,K) moved to channels-last):
+    the strides of the results, which memory_format and suggest_memory_format go by, as the Python functions give them."""
+    from torch_dwconv import _C
+
+    name, what, args, nhwc = call
+    n, c, h, w = shape
+    make = {"x": lambda: torch.ones(n, h, w, c, device=gpu).permute(0, 3, 1, 2), "g": lambda: torch.ones(n, c, h, w, device=gpu),
+            "w": lambda: torch.ones(c, 3, 3, 1, device=gpu).permute(0, 3, 1, 2), "p": lambda: torch.ones(c, device=gpu),
+            "n": lambda: None}
+    given = [make[k]() for k in what]
+
+    class Nothing:
+        def __getattr__(self, _):
+            return lambda *a: None
+
+    def strides():
+        out = getattr(_C, name)(*given, *args)
+        return [t.stride() if t is not None else None for t in (out if isinstance(out, tuple) else (out,))]
+
+    native = strides()
+    monkeypatch.setattr(_C, "_binding", Nothing())
+    assert native == strides()
+
+
 # (N, C, H, W, dil_h, dil_w): planes that start at every offset from a 16-byte boundary, chains of one to many steps,
 # dilations at and beyond the map, a second round of chains, the largest planes (64 KiB less the zero cell) and one above
 ATROUS = [
