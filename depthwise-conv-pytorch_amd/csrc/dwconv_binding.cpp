@@ -128,15 +128,28 @@ void *stream_of(const Tensor &t)
     return c10::hip::getCurrentHIPStream(t.device().index()).stream();
 }
 
-// Runs one library call with the GIL released, as ctypes does (a full launch queue may block it).
+// The GIL is free from the parsed arguments to the results, as it is in torch's own functions and in ctypes: an allocation
+// may wait for the device, a launch for room in a queue.
+class NoGil {
+  public:
+    NoGil() : state_(PyEval_SaveThread()) {}
+    ~NoGil() { PyEval_RestoreThread(state_); }
+    NoGil(const NoGil &) = delete;
+    NoGil &operator=(const NoGil &) = delete;
+
+  private:
+    PyThreadState *state_;
+};
+
+// What a function returns: one tensor, or several as a tuple (an undefined one is None).
+using Results = c10::SmallVector<Tensor, 3>;
+
 template <typename F>
 void call(const Tensor &on, F &&f)
 {
     const c10::DeviceGuard guard(on.device());
-    void *stream = stream_of(on);
-    int rc;
-    Py_BEGIN_ALLOW_THREADS rc = f(stream);
-    Py_END_ALLOW_THREADS if (rc != 0) throw std::runtime_error("libdwconv_hip error " + std::to_string(rc) + ": " + dwconv_last_error());
+    const int rc = f(stream_of(on));
+    if (rc != 0) throw std::runtime_error("libdwconv_hip error " + std::to_string(rc) + ": " + dwconv_last_error());
 }
 
 Tensor workspace(const Tensor &on, size_t bytes)
@@ -165,33 +178,39 @@ using Half = unsigned short;  // 16-bit elements at the C boundary
         default: NAME(Half, FN##_bf16) break;                     \
     }
 
-PyObject *wrap3(PyObject *a, PyObject *b, PyObject *c)
+PyObject *wrap(const Tensor &t)
 {
-    PyObject *t = PyTuple_New(3);
-    PyTuple_SET_ITEM(t, 0, a);
-    PyTuple_SET_ITEM(t, 1, b);
-    PyTuple_SET_ITEM(t, 2, c);
-    return t;
+    if (t.defined()) return THPVariable_Wrap(t);
+    Py_RETURN_NONE;
 }
 
-PyObject *wrap2(const Tensor &a, const Tensor &b)
+PyObject *wrap(const Results &results)
 {
-    PyObject *x = a.defined() ? THPVariable_Wrap(a) : (Py_INCREF(Py_None), Py_None);
-    PyObject *y = b.defined() ? THPVariable_Wrap(b) : (Py_INCREF(Py_None), Py_None);
-    PyObject *pair = PyTuple_New(2);
-    PyTuple_SET_ITEM(pair, 0, x);
-    PyTuple_SET_ITEM(pair, 1, y);
-    return pair;
+    if (results.size() == 1) return wrap(results[0]);
+    PyObject *tuple = PyTuple_New(static_cast<Py_ssize_t>(results.size()));
+    if (tuple == nullptr) return nullptr;
+    for (size_t i = 0; i < results.size(); ++i) {
+        PyObject *o = wrap(results[i]);
+        if (o == nullptr) {
+            Py_DECREF(tuple);
+            return nullptr;
+        }
+        PyTuple_SET_ITEM(tuple, static_cast<Py_ssize_t>(i), o);
+    }
+    return tuple;
 }
+
+PyObject *wrap(bool b) { return PyBool_FromLong(b); }
 
 // (input, kernel, up_h, up_w, down_h, down_w, pad_h0, pad_h1, pad_w0, pad_w1, forward)
-PyObject *conv(Args a)
+Results conv(Args a)
 {
     const Tensor input = a.tensor(), kernel = a.tensor();
     int v[8];
     for (int &e : v) e = a.integer();
     const int forward = a.integer() != 0;
     a.done();
+    const NoGil nogil;
     input_and_kernel(input, kernel);
     const Type type = type_of(input);
     const Tensor x = input.contiguous(), k = kernel.contiguous();
@@ -206,17 +225,18 @@ PyObject *conv(Args a)
     });
     DWCONV_BY_TYPE(type, DWCONV_CALL, dwconv2d)
 #undef DWCONV_CALL
-    return THPVariable_Wrap(y);
+    return {y};
 }
 
 // (input, kernel, up_h, up_w, down_h, down_w, pad_h, pad_w, forward)
-PyObject *conv_small(Args a)
+Results conv_small(Args a)
 {
     const Tensor input = a.tensor(), kernel = a.tensor();
     int v[6];
     for (int &e : v) e = a.integer();
     const int forward = a.integer() != 0;
     a.done();
+    const NoGil nogil;
     input_and_kernel(input, kernel);
     const Type type = type_of(input);
     const Tensor x = input.contiguous(), k = kernel.contiguous();
@@ -228,15 +248,16 @@ PyObject *conv_small(Args a)
     });
     DWCONV_BY_TYPE(type, DWCONV_CALL, dwconv2d_small)
 #undef DWCONV_CALL
-    return THPVariable_Wrap(y);
+    return {y};
 }
 
 // (input, out_grad, kernel, stride_h, stride_w, pad_h, pad_w) -> (in_grad, kernel_grad)
-PyObject *backward(Args a)
+Results backward(Args a)
 {
     const Tensor input = a.tensor(), grad = a.tensor(), kernel = a.tensor();
     const int sh = a.integer(), sw = a.integer(), ph = a.integer(), pw = a.integer();
     a.done();
+    const NoGil nogil;
     input_and_kernel(input, kernel);
     together(input, grad);
     if (grad.dim() != 4 || grad.size(0) != input.size(0) || grad.size(1) != input.size(1)) throw NotHere{};
@@ -261,15 +282,16 @@ PyObject *backward(Args a)
         default: DWCONV_CALL(Half, dwconv2d_backward_bf16) break;
     }
 #undef DWCONV_CALL
-    return wrap2(gx, gw);
+    return {gx, gw};
 }
 
 // (input, kernel, stride_h, stride_w, pad_h, pad_w), input channels-last or made so
-PyObject *conv_nhwc(Args a)
+Results conv_nhwc(Args a)
 {
     const Tensor input = a.tensor(), kernel = a.tensor();
     const int sh = a.integer(), sw = a.integer(), ph = a.integer(), pw = a.integer();
     a.done();
+    const NoGil nogil;
     input_and_kernel(input, kernel);
     const Type type = type_of(input);
     if (sh < 1 || sw < 1) throw NotHere{};
@@ -281,16 +303,17 @@ PyObject *conv_nhwc(Args a)
     call(x, [&](void *s) { return FN(in<T>(x), in<T>(k), out<T>(y), n, c, h, w, kh, kw, sh, sw, ph, pw, s); });
     DWCONV_BY_TYPE(type, DWCONV_CALL, dwconv2d_nhwc)
 #undef DWCONV_CALL
-    return THPVariable_Wrap(y);
+    return {y};
 }
 
 // (input, out_grad, kernel, stride_h, stride_w, pad_h, pad_w, need_input_grad, need_kernel_grad)
-PyObject *backward_nhwc(Args a)
+Results backward_nhwc(Args a)
 {
     const Tensor input = a.tensor(), grad = a.tensor(), kernel = a.tensor();
     const int sh = a.integer(), sw = a.integer(), ph = a.integer(), pw = a.integer();
     const bool need_x = a.integer() != 0, need_w = a.integer() != 0;
     a.done();
+    const NoGil nogil;
     if (!need_x && !need_w) throw NotHere{};
     input_and_kernel(input, kernel);
     together(input, grad);
@@ -312,7 +335,7 @@ PyObject *backward_nhwc(Args a)
     });
     DWCONV_BY_TYPE(type, DWCONV_CALL, dwconv2d_backward_nhwc)
 #undef DWCONV_CALL
-    return wrap2(gx, gw);
+    return {gx, gw};
 }
 
 // A per-channel vector as the library reads it: fp32 (fp64 beside fp64 tensors), dense, on the tensor's device.
@@ -326,12 +349,13 @@ c10::optional<Tensor> per_channel(const c10::optional<Tensor> &t, const Tensor &
 }
 
 // (input, kernel, scale | None, shift | None, activation, stride_h, stride_w, pad_h, pad_w)
-PyObject *fused(Args a)
+Results fused(Args a)
 {
     const Tensor input = a.tensor(), kernel = a.tensor();
     const c10::optional<Tensor> scale_ = a.optional_tensor(), shift_ = a.optional_tensor();
     const int act = a.integer(), sh = a.integer(), sw = a.integer(), ph = a.integer(), pw = a.integer();
     a.done();
+    const NoGil nogil;
     input_and_kernel(input, kernel);
     const Type type = type_of(input);
     if (sh < 1 || sw < 1) throw NotHere{};
@@ -355,16 +379,17 @@ PyObject *fused(Args a)
         DWCONV_BY_TYPE(type, DWCONV_CALL, dwconv2d_fused)
     }
 #undef DWCONV_CALL
-    return THPVariable_Wrap(y);
+    return {y};
 }
 
 // (conv_out, out_grad, scale | None, shift | None, activation) -> (conv_out overwritten, scale_grad, shift_grad)
-PyObject *epilogue_backward(Args a)
+Results epilogue_backward(Args a)
 {
     const Tensor conv_out = a.tensor(), grad = a.tensor();
     const c10::optional<Tensor> scale_ = a.optional_tensor(), shift_ = a.optional_tensor();
     const int act = a.integer();
     a.done();
+    const NoGil nogil;
     together(conv_out, grad);
     if (conv_out.dim() != 4 || grad.sizes() != conv_out.sizes()) throw NotHere{};
     const Type type = type_of(conv_out);
@@ -378,14 +403,18 @@ PyObject *epilogue_backward(Args a)
     const size_t bytes = dwconv2d_epilogue_backward_workspace_bytes(n, c, oh, ow, nhwc);
     const Tensor ws = workspace(conv_out, bytes);
     const float *sc = scale ? in<float>(*scale) : nullptr, *sf = shift ? in<float>(*shift) : nullptr;
-#define DWCONV_CALL(T, FN)                                                                                                     call(conv_out, [&](void *s) {                                                                                                  return FN(in<T>(conv_out), in<T>(gy), sc, sf, out<T>(conv_out), out<float>(grads), ws.mutable_data_ptr(), bytes, n, c,                   oh, ow, act, nhwc, s);                                                                                       });
+#define DWCONV_CALL(T, FN)                                                                                            \
+    call(conv_out, [&](void *s) {                                                                                     \
+        return FN(in<T>(conv_out), in<T>(gy), sc, sf, out<T>(conv_out), out<float>(grads), ws.mutable_data_ptr(), bytes, n, c, \
+                  oh, ow, act, nhwc, s);                                                                              \
+    });
     switch (type) {
         case F32: DWCONV_CALL(float, dwconv2d_epilogue_backward_f32) break;
         case F16: DWCONV_CALL(Half, dwconv2d_epilogue_backward_f16) break;
         default: DWCONV_CALL(Half, dwconv2d_epilogue_backward_bf16) break;
     }
 #undef DWCONV_CALL
-    return wrap3(THPVariable_Wrap(conv_out), THPVariable_Wrap(grads.select(1, 0)), THPVariable_Wrap(grads.select(1, 1)));
+    return {conv_out, grads.select(1, 0), grads.select(1, 1)};
 }
 
 // Input and a kernel of shape (C * M, 1, KH, KW); returns M.
@@ -404,12 +433,13 @@ int dilated_out(int in, int k, int stride, int pad, int dil)
 }
 
 // (input, kernel, stride_h, stride_w, pad_h, pad_w, dil_h, dil_w)
-PyObject *general(Args a)
+Results general(Args a)
 {
     const Tensor input = a.tensor(), kernel = a.tensor();
     int v[6];
     for (int &e : v) e = a.integer();
     a.done();
+    const NoGil nogil;
     const int m = multiplier(input, kernel);
     const Type type = type_of(input);
     if (v[0] < 1 || v[1] < 1) throw NotHere{};
@@ -417,19 +447,23 @@ PyObject *general(Args a)
     const int n = extent(x, 0), c = extent(x, 1), h = extent(x, 2), w = extent(x, 3), kh = extent(k, 2), kw = extent(k, 3);
     const Tensor y = empty_like_format(x, {n, static_cast<int64_t>(c) * m, dilated_out(h, kh, v[0], v[2], v[4]),
                                            dilated_out(w, kw, v[1], v[3], v[5])}, at::MemoryFormat::Contiguous);
-#define DWCONV_CALL(T, FN)                                                                                                   call(x, [&](void *s) {                                                                                                       return FN(in<T>(x), in<T>(k), out<T>(y), n, c, h, w, m, kh, kw, v[0], v[1], v[2], v[3], v[4], v[5], s);              });
+#define DWCONV_CALL(T, FN)                                                                                            \
+    call(x, [&](void *s) {                                                                                            \
+        return FN(in<T>(x), in<T>(k), out<T>(y), n, c, h, w, m, kh, kw, v[0], v[1], v[2], v[3], v[4], v[5], s);       \
+    });
     DWCONV_BY_TYPE(type, DWCONV_CALL, dwconv2d_general)
 #undef DWCONV_CALL
-    return THPVariable_Wrap(y);
+    return {y};
 }
 
 // (input, out_grad, kernel, stride_h, stride_w, pad_h, pad_w, dil_h, dil_w) -> (in_grad, kernel_grad)
-PyObject *general_backward(Args a)
+Results general_backward(Args a)
 {
     const Tensor input = a.tensor(), grad = a.tensor(), kernel = a.tensor();
     int v[6];
     for (int &e : v) e = a.integer();
     a.done();
+    const NoGil nogil;
     const int m = multiplier(input, kernel);
     together(input, grad);
     if (grad.dim() != 4 || grad.size(0) != input.size(0) || grad.size(1) != input.size(1) * m) throw NotHere{};
@@ -442,30 +476,34 @@ PyObject *general_backward(Args a)
     const size_t bytes = dwconv2d_general_backward_workspace_bytes(n, c, h, w, m, kh, kw, v[0], v[1], v[2], v[3], v[4], v[5],
                                                                    static_cast<int>(x.element_size()));
     const Tensor ws = workspace(x, bytes);
-#define DWCONV_CALL(T, FN)                                                                                                       call(x, [&](void *s) {                                                                                                           return FN(in<T>(x), in<T>(gy), in<T>(k), out<T>(gx), out<T>(gw), ws.mutable_data_ptr(), bytes, n, c, h, w, oh, ow, m,                   kh, kw, v[0], v[1], v[2], v[3], v[4], v[5], s);                                                                });
+#define DWCONV_CALL(T, FN)                                                                                            \
+    call(x, [&](void *s) {                                                                                            \
+        return FN(in<T>(x), in<T>(gy), in<T>(k), out<T>(gx), out<T>(gw), ws.mutable_data_ptr(), bytes, n, c, h, w, oh, ow, m, \
+                  kh, kw, v[0], v[1], v[2], v[3], v[4], v[5], s);                                                     \
+    });
     DWCONV_BY_TYPE(type, DWCONV_CALL, dwconv2d_general_backward)
 #undef DWCONV_CALL
-    return wrap2(gx, gw);
+    return {gx, gw};
 }
 
 // (tensor): channels-last and not also dense NCHW
-PyObject *is_channels_last(Args a)
+bool is_channels_last(Args a)
 {
     const Tensor t = a.tensor();
     a.done();
-    return PyBool_FromLong(channels_last(t));
+    return channels_last(t);
 }
 
 // (input, kernel, up_h, up_w, down_h, down_w, pad_h, pad_w)
-PyObject *use_small(Args a)
+bool use_small(Args a)
 {
     const Tensor input = a.tensor(), kernel = a.tensor();
     int v[6];
     for (int &e : v) e = a.integer();
     a.done();
     if (input.dim() != 4 || kernel.dim() != 4) throw NotHere{};
-    return PyBool_FromLong(dwconv_use_dwconv2d_small(extent(input, 2), extent(input, 3), extent(kernel, 2), extent(kernel, 3), v[0],
-                                                     v[1], v[2], v[3], v[4], v[5]));
+    return dwconv_use_dwconv2d_small(extent(input, 2), extent(input, 3), extent(kernel, 2), extent(kernel, 3), v[0], v[1], v[2],
+                                     v[3], v[4], v[5]) != 0;
 }
 
 // Modes under which tensor functions are not simply run: the Python functions, which call them one by one, serve then.
@@ -477,12 +515,12 @@ bool observed()
            c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::Functionalize);
 }
 
-template <PyObject *(*F)(Args)>
+template <auto F>
 PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t n)
 {
     HANDLE_TH_ERRORS
     try {
-        if (!observed()) return F(Args(args, n));
+        if (!observed()) return wrap(F(Args(args, n)));
     } catch (const NotHere &) {
     }
     Py_RETURN_NONE;

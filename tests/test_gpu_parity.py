@@ -1041,6 +1041,67 @@ def test_native_calls_keep_strides_of_single_elements(dw, gpu, call, shape, monk
     assert native == strides()
 
 
+POOL = r"""
+#include <stddef.h>
+int PyGILState_Check(void);
+static char *base;
+static size_t used = 4096, size; /* never the address of the tensor itself, which torch knows it by */
+static int calls, held;
+void pool_give(void *p, size_t n) { base = p; size = n; }
+int pool_calls(void) { return calls; }
+int pool_held(void) { return held; }
+void *pool_alloc(ptrdiff_t n, int device, void *stream)
+{
+    (void)device, (void)stream;
+    char *p = base + used;
+    calls += 1;
+    held += PyGILState_Check();
+    used += (n + 511) / 512 * 512;
+    return used <= size ? p : 0;
+}
+void pool_free(void *p, ptrdiff_t n, int device, void *stream) { (void)p, (void)n, (void)device, (void)stream; }
+"""
+
+
+def test_native_calls_allocate_without_the_gil(dw, gpu, tmp_path):
+    """No native call holds the GIL while it allocates: seen by an allocator of the test's own, which hands out pieces of a
+    tensor and looks whether its caller's thread holds the GIL."""
+    import ctypes
+    import subprocess
+
+    from torch_dwconv import _C
+
+    (tmp_path / "pool.c").write_text(POOL)
+    path = str(tmp_path / "pool.so")
+    subprocess.run(["gcc", "-O1", "-shared", "-fPIC", str(tmp_path / "pool.c"), "-o", path], check=True)
+    lib = ctypes.PyDLL(path)
+    backing = torch.empty(512 << 20, dtype=torch.uint8, device=gpu)
+    lib.pool_give(ctypes.c_void_p(backing.data_ptr()), ctypes.c_size_t(backing.numel()))
+    # results of 19 MB: above 10 MB every tensor is a piece of memory of its own, so that each call needs the allocator
+    x, g = (torch.ones(600, 8, 32, 31, device=gpu) for _ in "ab")
+    w, p = torch.ones(8, 1, 3, 3, device=gpu), torch.ones(8, device=gpu)
+    xl, yl, gl = (x.contiguous(memory_format=torch.channels_last) for _ in "abc")
+    calls = [
+        lambda: _C.dwconv2d(x, w, 1, 1, 1, 1, 1, 1, 1, 1, True), lambda: _C.dwconv2d_small(x, w, 1, 1, 1, 1, 1, 1, True),
+        lambda: _C.dwconv2d_backward(x, g, w, 1, 1, 1, 1), lambda: _C.dwconv2d_nhwc(xl, w, 1, 1, 1, 1),
+        lambda: _C.dwconv2d_backward_nhwc(xl, gl, w, 1, 1, 1, 1), lambda: _C.dwconv2d_fused(x, w, p, p, "silu", 1, 1, 1, 1),
+        lambda: _C.dwconv2d_general(x, w, 1, 1, 3, 3, 3, 3), lambda: _C.dwconv2d_general_backward(x, g, w, 1, 1, 3, 3, 3, 3),
+        lambda: _C.dwconv2d_epilogue_backward(yl, g, p, p, "silu"),  # its copy of g is free again afterwards
+    ]
+    allocator = torch.cuda.memory.CUDAPluggableAllocator(path, "pool_alloc", "pool_free")
+    pool = torch.cuda.MemPool(allocator.allocator())
+    kept, seen = [], []
+    with torch.cuda.use_mem_pool(pool):
+        for call in calls:
+            before = lib.pool_calls()
+            kept.append(call())
+            seen.append(lib.pool_calls() - before)
+    torch.cuda.synchronize()
+    kept.clear()  # before the pool
+    assert min(seen) >= 1 and lib.pool_held() == 0, (seen, lib.pool_held())
+    del pool
+
+
 # (N, C, H, W, dil_h, dil_w): planes that start at every offset from a 16-byte boundary, chains of one to many steps,
 # dilations at and beyond the map, a second round of chains, the largest planes (64 KiB less the zero cell) and one above
 ATROUS = [
