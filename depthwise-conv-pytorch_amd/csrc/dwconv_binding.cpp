@@ -9,6 +9,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/csrc/jit/frontend/tracer.h>
+#include <torch/version.h>
 
 #include <ATen/ATen.h>
 #include <ATen/PythonTorchFunctionTLS.h>
@@ -537,4 +538,10 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_binding", "Native calls behind to
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__binding(void) { return PyModule_Create(&module); }
+PyMODINIT_FUNC PyInit__binding(void)
+{
+    PyObject *m = PyModule_Create(&module);
+    // torch's C++ interface holds for one release: _C.py uses the module under that one only
+    if (m != nullptr && PyModule_AddStringConstant(m, "torch_version", TORCH_VERSION) != 0) Py_CLEAR(m);
+    return m;
+}

@@ -11,7 +11,9 @@ There is no CPU implementation behind this module: if the shared library is
 missing, importing it raises ImportError.
 """
 import ctypes
+import importlib
 import os
+import warnings
 
 import torch
 
@@ -26,14 +28,36 @@ if not os.path.exists(LIBRARY_PATH):
 
 _lib = ctypes.CDLL(LIBRARY_PATH)
 
-try:
-    from . import _binding
-except ImportError as e:
-    raise ImportError(
-        f"torch_dwconv._binding does not load ({e}): build it with `make -C depthwise-conv-pytorch_amd/csrc`"
-    ) from e
+class _NoBinding:
+    """Stands where there is no native module: serves no call."""
+
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
+def _load_binding():
+    """The native module, if it was built for this Python and this release of torch."""
+    try:
+        module = importlib.import_module("._binding", __package__)
+    except ModuleNotFoundError:
+        return _NoBinding()
+    except ImportError as e:
+        reason = str(e)
+    else:
+        built_for = getattr(module, "torch_version", "of another release")
+        if built_for == torch.__version__.split("+")[0]:
+            return module
+        reason = f"it was built against torch {built_for}, this is {torch.__version__}"
+    warnings.warn(f"torch_dwconv._binding is not used ({reason}): calls cost 10 us more each. "
+                  "Build it with `make -C depthwise-conv-pytorch_amd/csrc`.", RuntimeWarning, stacklevel=3)
+    return _NoBinding()
+
+
 # Every function below first hands its arguments to its native namesake (csrc/dwconv_binding.cpp), which serves plain
-# GPU tensors and returns None for everything else.  What follows serves the rest and raises the errors.
+# GPU tensors and returns None for everything else.  What follows serves the rest, and everything where the module is
+# missing or was built for another Python or torch, and raises the errors.  A function or dispatch mode counts as the rest,
+# also the one that torch.set_default_device installs: under it calls take the longer way.
+_binding = _load_binding()
 
 _i, _p, _z = ctypes.c_int, ctypes.c_void_p, ctypes.c_size_t
 _lib.dwconv_last_error.restype = ctypes.c_char_p

@@ -4,6 +4,9 @@ import ctypes
 import itertools
 import os
 import re
+import shutil
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -27,6 +30,44 @@ def lib():
     from torch_dwconv import _C
 
     return _C._lib
+
+
+@pytest.mark.parametrize("native", ["missing", "broken", "other_torch", "unversioned"])
+def test_package_serves_without_its_native_module(native, tmp_path):
+    """The module of native calls missing, not loadable, or built against another torch: the package imports and serves
+    through ctypes (here: geometry, layout and the error of a tensor that is not on a GPU), with a warning unless missing."""
+    from torch_dwconv import _C
+
+    package = tmp_path / "torch_dwconv"
+    package.mkdir()
+    here = os.path.dirname(_C.__file__)
+    for name in os.listdir(here):
+        if name.endswith(".py"):
+            shutil.copy(os.path.join(here, name), package)
+    os.symlink(_C.LIBRARY_PATH, package / "libdwconv_hip.so")
+    if native == "broken":
+        (package / "_binding.so").write_bytes(b"not a shared object")
+    elif native == "other_torch":
+        (package / "_binding.py").write_text("torch_version = '1.13.1'\n")
+    elif native == "unversioned":
+        (package / "_binding.py").write_text("")
+    code = """if True:
+        import warnings
+        import torch
+        with warnings.catch_warnings(record=True) as seen:
+            warnings.simplefilter("always")
+            from torch_dwconv import _C
+        assert [w.category for w in seen if "_binding" in str(w.message)] == [RuntimeWarning] * %d, seen
+        assert _C.use_dwconv2d_small(torch.zeros(1, 2, 14, 14), torch.zeros(2, 1, 3, 3), 1, 1, 1, 1, 1, 1) is True
+        assert _C.is_channels_last(torch.zeros(1, 5, 5, 2).permute(0, 3, 1, 2)) is True
+        try:
+            _C.dwconv2d(torch.zeros(1, 2, 5, 5), torch.zeros(2, 1, 3, 3), 1, 1, 1, 1, 1, 1, 1, 1, True)
+        except RuntimeError as e:
+            assert "must be a CUDA tensor" in str(e)
+            print("served")
+    """ % (native != "missing")
+    run = subprocess.run([sys.executable, "-c", code], cwd=tmp_path, capture_output=True, text=True, timeout=300)
+    assert run.returncode == 0 and run.stdout.strip() == "served", run.stderr
 
 
 def test_library_exports_every_declared_symbol():
