@@ -7,6 +7,7 @@ import re
 import shutil
 import subprocess
 import sys
+import sysconfig
 
 import pytest
 import torch
@@ -243,3 +244,15 @@ def test_product_code_never_reaches_for_the_oracle_or_working_files():
     start = bench.index("def cpu_baseline")
     end = bench.index("\ndef ", start + 1)
     assert uses and all(start < u < end for u in uses), "bench.py touches the oracle outside cpu_baseline()"
+
+
+@pytest.mark.parametrize("given, native", [((), True), (("OUT=/tmp/elsewhere/libdwconv_hip.so",), False), (("PYTHON=false",), False)],
+                         ids=["package", "elsewhere", "no_torch"])
+def test_make_builds_the_library_alone(given, native):
+    """The library needs neither torch nor Python and may be built anywhere; the native module only goes with the package."""
+    csrc = os.path.join(ROOT, "depthwise-conv-pytorch_amd", "csrc")
+    run = subprocess.run(["make", "-n", "-B", "-C", csrc, *(given or ("PYTHON=" + sys.executable,))], capture_output=True, text=True)
+    assert run.returncode == 0, run.stderr
+    assert ("dwconv_binding.cpp" in run.stdout) == native and "-shared -fPIC -o" in run.stdout
+    if native:
+        assert "_binding" + sysconfig.get_config_var("EXT_SUFFIX") in run.stdout
