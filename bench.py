@@ -461,6 +461,7 @@ def main():
                 "bwd_tile": "wgrad_tile_kernel + wgrad_tile_final_kernel",
                 "wgrad_tile": "wgrad_tile_kernel + wgrad_tile_final_kernel",
                 "bwd_tile_s2": "bwd_s2_kernel + wgrad_tile_final_kernel",
+                "atrous": "atrous_kernel", "atrous_bwd": "atrous_kernel + wgrad_tile_final_kernel",
                 "tile_stack": "stack_kernel", "bwd_stack": "stack_kernel + wgrad_tile_final_kernel",
                 "nhwc_bwd": "nhwc_bwd_fused_kernel + nhwc_wgrad_final_kernel"}.get(family, family)
     roofline = {"bound": "hbm", "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
