@@ -17,8 +17,7 @@
 // 65x65).  Batch 16, 256 channels, us, the any-geometry kernels before / this one:
 //   65x65 fp32, rate 6:  forward 44 / 26, backward 127 / 36      rate 18: forward 55 / 26, backward 148 / 37
 //   97x97 fp32, rate 18: forward 129 / 73, backward 293 / 109    65x65 bf16, rate 6: forward 44 / 18, backward 138 / 27
-// (the 65x65 fp32 pair moves 138 and 208 MB: 5.3 and 5.7 TB/s).  Maps of 9 to 24 columns: 13 / 13 and 24 / 20, the time
-// the host takes to make the calls.
+// (the 65x65 fp32 pair moves 138 and 208 MB: 5.3 and 5.7 TB/s).
 #include "dwconv_tile_common.hpp"
 
 #include <algorithm>

@@ -236,7 +236,8 @@ __global__ __launch_bounds__(kEpiThreads) void epilogue_bwd_nhwc_kernel(const Ep
     }
 }
 
-// Lanes for `groups` channel groups: all of them where a wavefront holds them, else equal shares of whole 128-byte lines.
+// Lanes for `groups` channel groups: all of them where a wavefront holds them, else equal shares of whole eights of lanes
+// (a 128-byte line where a lane moves four fp32 channels).
 int lanes_for(int groups)
 {
     const int blocks = ceil_div(groups, 64), share = ceil_div(groups, blocks);

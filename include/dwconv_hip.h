@@ -336,8 +336,10 @@ int dwconv2d_epilogue_backward_bf16(const unsigned short *conv_out, const unsign
  * (C*multiplier,1,KH,KW); out and out_grad (N,C*multiplier,OH,OW) with
  * OH = (H + 2*pad_h - dil_h*(KH-1) - 1) / stride_h + 1:
  *   out[n, c*M+j, oy, ox] = sum_{ty,tx} input[n, c, oy*stride - pad + ty*dil, ox*stride - pad + tx*dil] * kernel[c*M+j, ty, tx]
- * i.e. F.conv2d(groups=C, dilation=dil).  With multiplier 1 and dilation 1 the call is served by the tuned
- * kernels behind dwconv2d_* / dwconv2d_backward_*; otherwise by per-element kernels (correct, not tuned).
+ * i.e. F.conv2d(groups=C, dilation=dil).  With multiplier 1 and dilation 1 the call is served by the
+ * kernels behind dwconv2d_* / dwconv2d_backward_*, with multiplier 1 and any other dilation by tiled kernels, with a
+ * multiplier and square 3x3 / 5x5 / 7x7 filters by tiled kernels on larger maps; what is left (multipliers on small maps,
+ * the input gradient of dilated layers above stride 1, multipliers of double tensors) by per-element kernels.
  * kernel_grad is bit-identical from run to run. */
 size_t dwconv2d_general_backward_workspace_bytes(int batch, int channel, int in_h, int in_w,
                                                  int multiplier, int kernel_h, int kernel_w,
