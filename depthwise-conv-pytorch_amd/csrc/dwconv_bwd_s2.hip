@@ -97,7 +97,8 @@ __global__ __launch_bounds__(kThreads) void bwd_s2_kernel(const BwdS2Plan p)
     // (the epilogue's x image starts at the window of gy row q0 - M + E, the first one that in_grad depends on)
     const float *base_x = lds + ((EPI ? qb + M - E : qb) * 2) * p.sx.pitch + kSlack + 4 * cb;
     const float *base_g = lds + p.g_base + qb * p.sg.pitch + kSlack + 2 * cb;
-    float s_scale = 0.f, s_shift = 0.f, e_scale = 1.f, e_shift = 0.f;
+    EpilogueSums sums;
+    float e_scale = 1.f, e_shift = 0.f;
     if constexpr (EPI) p.epi.load(c, e_scale, e_shift);
 
     float rot[KK];
@@ -174,6 +175,7 @@ __global__ __launch_bounds__(kThreads) void bwd_s2_kernel(const BwdS2Plan p)
                 pin_registers(z);
             }
             float *gp = lds + p.g_base + (rb * BQ + E) * p.sg.pitch + kSlack + 2 * cb + M;
+            float s_scale = 0.f, s_shift = 0.f;
             p.epi.slopes([&](auto act) {
 #pragma unroll
                 for (int b = 0; b < BQ; ++b) {
@@ -190,6 +192,7 @@ __global__ __launch_bounds__(kThreads) void bwd_s2_kernel(const BwdS2Plan p)
                     }
                 }
             });
+            sums.add(s_scale, s_shift);
             __syncthreads();
         }
 
@@ -336,7 +339,7 @@ __global__ __launch_bounds__(kThreads) void bwd_s2_kernel(const BwdS2Plan p)
     constexpr int SUMS = EPI ? KK + 2 : KK;
 #pragma unroll
     for (int t = 0; t < SUMS; ++t) {
-        const float s = wave_sum_to_last_lane(t < KK ? wacc[t < KK ? t : 0] : (t == KK ? s_scale : s_shift));
+        const float s = wave_sum_to_last_lane(t < KK ? wacc[t < KK ? t : 0] : static_cast<float>(t == KK ? sums.scale : sums.shift));
         if ((threadIdx.x & 63) == 63) lds[(threadIdx.x >> 6) * SUMS + t] = s;
     }
     __syncthreads();

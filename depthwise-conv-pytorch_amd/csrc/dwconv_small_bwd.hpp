@@ -160,7 +160,8 @@ __global__ __launch_bounds__(kWave, EPI ? 2 : 1) void small_bwd_kernel(const Sma
 #pragma unroll
     for (int t = 0; t < KK; ++t) wacc[t] = 0.f;
     static_assert(!EPI || (GX && D == 1), "the epilogue's instances make all gradients");
-    float s_scale = 0.f, s_shift = 0.f, e_scale = 1.f, e_shift = 0.f;
+    EpilogueSums sums;
+    float e_scale = 1.f, e_shift = 0.f;
     if constexpr (EPI) p.epi.load(c0 + pl, e_scale, e_shift);
     float tapv[GX ? KK : 1];
     if constexpr (GX) load_taps<KK, true>(static_cast<const IO *>(p.taps), c0 + pl, tapv);
@@ -239,6 +240,8 @@ __global__ __launch_bounds__(kWave, EPI ? 2 : 1) void small_bwd_kernel(const Sma
                     lds_load_row_w<OW, RAG>(ok ? grow + b * lp_out : zrow, g[b], w_out);
                 }
                 // (rows and columns past the plane keep their zeros whatever the convolution is there)
+                constexpr int PARTS = BH * OW > 16 ? 2 : 1;
+                float s_scale[PARTS] = {}, s_shift[PARTS] = {};
                 p.epi.slopes([&](auto act) {
 #pragma unroll
                     for (int b = 0; b < BH; ++b) {
@@ -247,12 +250,14 @@ __global__ __launch_bounds__(kWave, EPI ? 2 : 1) void small_bwd_kernel(const Sma
                         for (int o = 0; o < OW; ++o) {
                             const bool in = ok && (!RAG || o < w_out);
                             const float ga = EpilogueBackward::slope<decltype(act)::value>(fmaf(z[b][o], e_scale, e_shift), g[b][o]);
-                            s_scale = fmaf(in ? ga : 0.f, in ? z[b][o] : 0.f, s_scale);
-                            s_shift += in ? ga : 0.f;
+                            s_scale[o % PARTS] = fmaf(in ? ga : 0.f, in ? z[b][o] : 0.f, s_scale[o % PARTS]);
+                            s_shift[o % PARTS] += in ? ga : 0.f;
                             g[b][o] = in ? ga * e_scale : 0.f;
                         }
                     }
                 });
+#pragma unroll
+                for (int q = 0; q < PARTS; ++q) sums.add(s_scale[q], s_shift[q]);
 #pragma unroll
                 for (int b = 0; b < BH; ++b)
                     if (active && oy0 + b < p.out_h) lds_store_row_w<OW, RAG>(grow + b * lp_out, g[b], w_out);
@@ -379,16 +384,16 @@ __global__ __launch_bounds__(kWave, EPI ? 2 : 1) void small_bwd_kernel(const Sma
     for (int t = 0; t < KK; ++t) lds[t * kSmallRedPitch + threadIdx.x] = wacc[t];
     constexpr int SUMS = EPI ? KK + 2 : KK;
     if constexpr (EPI) {
-        lds[KK * kSmallRedPitch + threadIdx.x] = s_scale;
-        lds[(KK + 1) * kSmallRedPitch + threadIdx.x] = s_shift;
+        lds[KK * kSmallRedPitch + threadIdx.x] = static_cast<float>(sums.scale);
+        lds[(KK + 1) * kSmallRedPitch + threadIdx.x] = static_cast<float>(sums.shift);
     }
     __syncthreads();
     for (int e = threadIdx.x; e < nplanes * SUMS; e += kWave) {
         const int q = e / SUMS, t = e - q * SUMS;
         const float *col = lds + t * kSmallRedPitch + q * p.lanes_per_plane;
-        float s = 0.f;
+        typename std::conditional<EPI, double, float>::type s = 0;
         for (int i = 0; i < p.lanes_per_plane; ++i) s += col[i];
-        p.partial[(static_cast<long>(c0 + q) * p.chunks + chunk) * SUMS + t] = s;
+        p.partial[(static_cast<long>(c0 + q) * p.chunks + chunk) * SUMS + t] = static_cast<float>(s);
     }
 }
 

@@ -113,7 +113,8 @@ __global__ __launch_bounds__(kThreads) void wgrad_tile_kernel(const WgradPlan p)
     const float *base = lds + pl * p.st.plane_pitch + (row0 * S + HALO) * p.st.pitch + kSlack + 4 * cb * S;
     const float *base_g = EPI ? lds + p.g_base + pl * p.sg.plane_pitch + row0 * p.sg.pitch + kSlack + 4 * cb : base + p.g_base;
     static_assert(!EPI || GX, "the epilogue's instances make all gradients");
-    float s_scale = 0.f, s_shift = 0.f, e_scale = 1.f, e_shift = 0.f;
+    EpilogueSums sums;
+    float e_scale = 1.f, e_shift = 0.f;
     if constexpr (EPI) p.epi.load(c0 + pl, e_scale, e_shift);
 
     float rot[GX ? KK : 1];
@@ -201,6 +202,7 @@ __global__ __launch_bounds__(kThreads) void wgrad_tile_kernel(const WgradPlan p)
                 pin_registers(z);
             }
             float *gp = lds + p.g_base + pl * p.sg.plane_pitch + rb * BH * p.sg.pitch + kSlack + 4 * cb + HALO;
+            float s_scale = 0.f, s_shift = 0.f;
             p.epi.slopes([&](auto act) {
 #pragma unroll
                 for (int b = 0; b < BH; ++b) {
@@ -217,6 +219,7 @@ __global__ __launch_bounds__(kThreads) void wgrad_tile_kernel(const WgradPlan p)
                     }
                 }
             });
+            sums.add(s_scale, s_shift);
             __syncthreads();
         }
 
@@ -352,7 +355,7 @@ __global__ __launch_bounds__(kThreads) void wgrad_tile_kernel(const WgradPlan p)
         // every lane worked on the same channel: wavefront sums, then the four wavefronts in order
 #pragma unroll
         for (int t = 0; t < SUMS; ++t) {
-            const float s = wave_sum_to_last_lane(t < KK ? acc[t < KK ? t : 0] : (t == KK ? s_scale : s_shift));
+            const float s = wave_sum_to_last_lane(t < KK ? acc[t < KK ? t : 0] : static_cast<float>(t == KK ? sums.scale : sums.shift));
             if ((threadIdx.x & 63) == 63) lds[(threadIdx.x >> 6) * SUMS + t] = s;
         }
         __syncthreads();
@@ -367,16 +370,16 @@ __global__ __launch_bounds__(kThreads) void wgrad_tile_kernel(const WgradPlan p)
 #pragma unroll
         for (int t = 0; t < KK; ++t) lds[t * kRedPitch + threadIdx.x] = acc[t];
         if constexpr (EPI) {
-            lds[KK * kRedPitch + threadIdx.x] = s_scale;
-            lds[(KK + 1) * kRedPitch + threadIdx.x] = s_shift;
+            lds[KK * kRedPitch + threadIdx.x] = static_cast<float>(sums.scale);
+            lds[(KK + 1) * kRedPitch + threadIdx.x] = static_cast<float>(sums.shift);
         }
         __syncthreads();
         for (int e = threadIdx.x; e < nplanes * SUMS; e += blockDim.x) {
             const int pl = e / SUMS, t = e - pl * SUMS;
             const float *col = lds + t * kRedPitch + pl * p.items_per_plane;
-            float s = 0.f;
+            typename std::conditional<EPI, double, float>::type s = 0;
             for (int i = 0; i < p.items_per_plane; ++i) s += col[i];
-            out[static_cast<long>(pl) * p.chunks * SUMS + t] = s;
+            out[static_cast<long>(pl) * p.chunks * SUMS + t] = static_cast<float>(s);
         }
     }
 }

@@ -62,6 +62,36 @@ def test_one_sweep(gpu, case, dtype):
     assert all(torch.equal(a, b) for a, b in zip(grads, again))
 
 
+# Grids capped to one workgroup a channel group: every workgroup walks all images.
+ONE_WORKGROUP = ("DWCONV_SMALL_WGRAD_WAVES", "DWCONV_EPI_WGS", "DWCONV_S2_WGS_K3", "DWCONV_WGRAD_WGS")
+
+
+def cap_grids(monkeypatch):
+    monkeypatch.setenv("DWCONV_TUNING", "1")
+    for name in ONE_WORKGROUP:
+        monkeypatch.setenv(name, "1")
+
+
+@pytest.mark.parametrize("shape", [(96, 16, 28, 28, 5, 1, 2), (96, 16, 7, 7, 3, 1, 1), (96, 16, 14, 14, 5, 2, 2), (96, 16, 13, 13, 3, 1, 1),
+                                   (96, 16, 56, 56, 3, 1, 1), (96, 16, 36, 36, 3, 1, 1), (192, 16, 56, 56, 3, 2, 1)], ids=shape_id)
+def test_scale_and_shift_sums_over_many_images(gpu, monkeypatch, shape):
+    """fp32 sums over up to 3e5 elements, every workgroup on all images.  With u = 2^-24 and random signs: sums of 16 elements are off
+    by sqrt(17 / 6) u of their size, images are added up in fp64, the tree over the lanes adds sqrt(10 / 3) u and the convolution
+    under scale's gradient sqrt(25 / 6) u: 3.3 u together, u / 2 more for the results.  One fp32 sum over all images would be off
+    by sqrt(n / 6) u, 16 to 21 u for 1344 to 2688 elements a lane (7x7 and 13x13: 8 to 15).  The bound is 6 u."""
+    from torch_dwconv import _C
+
+    cap_grids(monkeypatch)
+    n, c, h, w, k, s, p = shape
+    x, wt, gy = (t.to(gpu) for t in make_inputs(shape, seed=13))
+    scale, shift = params(c, gpu)
+    grads = _C.dwconv2d_fused_backward(x, gy, wt, scale, shift, None, s, s, p, p)
+    assert " chunks1" in _C.last_variant(), _C.last_variant()
+    for got, ref in zip(grads[2:], reference(x, wt, gy, scale, shift, None, s, p)[2:]):
+        error = float((got.cpu().double() - ref).norm() / ref.norm())
+        assert error <= 6 * 2.0 ** -24, (_C.last_variant(), error)
+
+
 @pytest.mark.parametrize("act", [None, "relu", "relu6"])
 @pytest.mark.parametrize("shape", [(2, 6, 14, 14, 3, 1, 1), (2, 3, 38, 38, 3, 2, 1), (2, 3, 56, 56, 5, 1, 2)], ids=shape_id)
 def test_activations(gpu, shape, act):
