@@ -176,7 +176,7 @@ __global__ __launch_bounds__(kThreads) void bwd_s2_kernel(const BwdS2Plan p)
             }
             float *gp = lds + p.g_base + (rb * BQ + E) * p.sg.pitch + kSlack + 2 * cb + M;
             float s_scale = 0.f, s_shift = 0.f;
-            p.epi.slopes([&](auto act) {
+            p.epi.slopes(z, e_scale, e_shift, [&](auto act) {
 #pragma unroll
                 for (int b = 0; b < BQ; ++b) {
                     const int r = rb * BQ + b + E - M;  // row of the tile

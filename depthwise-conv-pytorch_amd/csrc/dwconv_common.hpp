@@ -116,19 +116,41 @@ struct EpilogueBackward {
     {
         if constexpr (ACT == DWCONV_ACT_RELU) return z > 0.f ? g : 0.f;
         else if constexpr (ACT == DWCONV_ACT_RELU6) return (z > 0.f && z < 6.f) ? g : 0.f;
-        else if constexpr (ACT == DWCONV_ACT_SILU) {
-            const float s = __builtin_amdgcn_rcpf(1.f + __expf(-z));
+        else if constexpr (ACT == DWCONV_ACT_SILU || ACT == kSiluNear) {
+            const float d = 1.f + __expf(-z);
+            float s;
+            if constexpr (ACT == kSiluNear) {
+                const float r = __builtin_amdgcn_rcpf(d);
+                s = fmaf(fmaf(-d, r, 1.f), r, r);
+            } else {
+                s = 1.f / d;
+            }
             return g * s * (1.f + z * (1.f - s));
         } else return g;
     }
-    // body(std::integral_constant<int, activation>): the test on the (uniform) activation is made once for a block
-    template <typename F>
-    __device__ __forceinline__ void slopes(F &&body) const
+    // SiLU where z is at least kNear, so that 1 / (1 + exp(-z)) is no subnormal number: the hardware's reciprocal, which is off by
+    // one unit in the last place, and one step of Newton's method make the rounded quotient (P. Markstein, IBM Journal of Research and
+    // Development 34, 1990; significands of all ones excepted) in three instructions instead of ten.  With the division the
+    // fused backward passes of EfficientNet-B0 (batch 128, fp32 and bf16) take 2244 us, with this 2162, with the bare reciprocal 2132.
+    static constexpr int kSiluNear = -1;
+    static constexpr float kNear = -87.f;
+    // body(std::integral_constant<int, activation>) for a lane's block conv: the tests on the (uniform) activation and on the
+    // range are made once for the block
+    template <int R, int C, typename F>
+    __device__ __forceinline__ void slopes(const float (&conv)[R][C], float sc, float sh, F &&body) const
     {
         if (act == DWCONV_ACT_RELU) body(std::integral_constant<int, DWCONV_ACT_RELU>{});
         else if (act == DWCONV_ACT_RELU6) body(std::integral_constant<int, DWCONV_ACT_RELU6>{});
-        else if (act == DWCONV_ACT_SILU) body(std::integral_constant<int, DWCONV_ACT_SILU>{});
-        else body(std::integral_constant<int, DWCONV_ACT_NONE>{});
+        else if (act == DWCONV_ACT_SILU) {
+            float lo = conv[0][0], hi = conv[0][0];
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+#pragma unroll
+                for (int c = 0; c < C; ++c) lo = fminf(lo, conv[r][c]), hi = fmaxf(hi, conv[r][c]);
+            // (z is a monotonic function of the convolution; a NaN stays one either way)
+            if (__any(fminf(fmaf(lo, sc, sh), fmaf(hi, sc, sh)) < kNear)) body(std::integral_constant<int, DWCONV_ACT_SILU>{});
+            else body(std::integral_constant<int, kSiluNear>{});
+        } else body(std::integral_constant<int, DWCONV_ACT_NONE>{});
     }
 };
 

@@ -41,15 +41,12 @@ struct EpiBwdPlan {
     int half;             // the largest power of two below pixels: the first step of the sum over them
 };
 
-// out_grad * d act(z) / dz.  Boundaries as PyTorch's own backward formulas: ReLU passes z > 0, ReLU6 passes 0 < z < 6.
+// out_grad * d act(z) / dz.
 __device__ __forceinline__ float act_backward(float z, float g, int act)
 {
-    if (act == DWCONV_ACT_RELU) return z > 0.f ? g : 0.f;
-    if (act == DWCONV_ACT_RELU6) return (z > 0.f && z < 6.f) ? g : 0.f;
-    if (act == DWCONV_ACT_SILU) {
-        const float s = 1.f / (1.f + __expf(-z));
-        return g * s * (1.f + z * (1.f - s));
-    }
+    if (act == DWCONV_ACT_RELU) return EpilogueBackward::slope<DWCONV_ACT_RELU>(z, g);
+    if (act == DWCONV_ACT_RELU6) return EpilogueBackward::slope<DWCONV_ACT_RELU6>(z, g);
+    if (act == DWCONV_ACT_SILU) return EpilogueBackward::slope<DWCONV_ACT_SILU>(z, g);
     return g;
 }
 

@@ -242,7 +242,7 @@ __global__ __launch_bounds__(kWave, EPI ? 2 : 1) void small_bwd_kernel(const Sma
                 // (rows and columns past the plane keep their zeros whatever the convolution is there)
                 constexpr int PARTS = BH * OW > 16 ? 2 : 1;
                 float s_scale[PARTS] = {}, s_shift[PARTS] = {};
-                p.epi.slopes([&](auto act) {
+                p.epi.slopes(z, e_scale, e_shift, [&](auto act) {
 #pragma unroll
                     for (int b = 0; b < BH; ++b) {
                         const bool ok = active && oy0 + b < p.out_h;

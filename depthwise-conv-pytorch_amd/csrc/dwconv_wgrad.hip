@@ -203,7 +203,7 @@ __global__ __launch_bounds__(kThreads) void wgrad_tile_kernel(const WgradPlan p)
             }
             float *gp = lds + p.g_base + pl * p.sg.plane_pitch + rb * BH * p.sg.pitch + kSlack + 4 * cb + HALO;
             float s_scale = 0.f, s_shift = 0.f;
-            p.epi.slopes([&](auto act) {
+            p.epi.slopes(z, e_scale, e_shift, [&](auto act) {
 #pragma unroll
                 for (int b = 0; b < BH; ++b) {
                     const int r = rb * BH + b - HALO;  // row of the tile; the first and last HALO rows are the neighbours'

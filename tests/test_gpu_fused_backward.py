@@ -92,6 +92,25 @@ def test_scale_and_shift_sums_over_many_images(gpu, monkeypatch, shape):
         assert error <= 6 * 2.0 ** -24, (_C.last_variant(), error)
 
 
+@pytest.mark.parametrize("shape", [(2, 4, 14, 14, 3, 1, 1), (1, 3, 29, 28, 5, 1, 2), (2, 2, 56, 56, 3, 1, 1), (1, 2, 75, 75, 3, 1, 1),
+                                   (1, 2, 56, 56, 5, 2, 2)], ids=shape_id)
+def test_silu_slope_is_that_of_the_separate_sweep(gpu, shape):
+    """A filter that is one at its centre and zero elsewhere: the convolution is the input's elements, in_grad the slopes, both without
+    a rounding.  The sigmoid is the rounded quotient in both, so the bits are those of the epilogue's own sweep, also where it is subnormal."""
+    from torch_dwconv import _C
+
+    n, c, h, w, k, s, p = shape
+    x, _, gy = (t.to(gpu) for t in make_inputs(shape, seed=17))
+    x[:, 0] = x[:, 0].clamp(-1, 1) * 89
+    wt = torch.zeros(c, 1, k, k, device=gpu)
+    wt[:, :, p, p] = 1
+    gx = _C.dwconv2d_fused_backward(x, gy, wt, None, None, "silu", s, s, p, p)[0]
+    assert ",epi>" in _C.last_variant(), _C.last_variant()
+    want = torch.zeros_like(x)
+    want[:, :, ::s, ::s] = _C.dwconv2d_epilogue_backward(x[:, :, ::s, ::s].contiguous(), gy, None, None, "silu")[0]
+    assert torch.equal(gx, want), float((gx - want).abs().max())
+
+
 @pytest.mark.parametrize("act", [None, "relu", "relu6"])
 @pytest.mark.parametrize("shape", [(2, 6, 14, 14, 3, 1, 1), (2, 3, 38, 38, 3, 2, 1), (2, 3, 56, 56, 5, 1, 2)], ids=shape_id)
 def test_activations(gpu, shape, act):
