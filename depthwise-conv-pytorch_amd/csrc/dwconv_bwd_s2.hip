@@ -326,10 +326,14 @@ __global__ __launch_bounds__(kThreads) void bwd_s2_kernel(const BwdS2Plan p)
             for (int bq = 0; bq < BQ; ++bq) {
                 const int ty = wr - 2 * bq;
                 if (ty < 0 || ty >= K) continue;
+                // (with the epilogue a tile hangs over the plane by other rows than the plain kernel's: those past it meet no x)
+                if (EPI && !(has_item && 2 * cb < p.out_w && bq >= skip && q0 + qb + bq < p.out_h)) continue;
 #pragma unroll
-                for (int tx = 0; tx < K; ++tx)
+                for (int o = 0; o < 2; ++o) {
+                    if (EPI && o > 0 && 2 * cb + o >= p.out_w) continue;
 #pragma unroll
-                    for (int o = 0; o < 2; ++o) wacc[ty * K + tx] = fmaf(g[bq][o], win[2 * o + tx], wacc[ty * K + tx]);
+                    for (int tx = 0; tx < K; ++tx) wacc[ty * K + tx] = fmaf(g[bq][o], win[2 * o + tx], wacc[ty * K + tx]);
+                }
             }
             pin_registers(wacc);
         }

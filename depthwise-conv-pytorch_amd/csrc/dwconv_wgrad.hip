@@ -312,11 +312,15 @@ __global__ __launch_bounds__(kThreads) void wgrad_tile_kernel(const WgradPlan p)
             for (int b = 0; b < BH; ++b) {
                 const int ty = wr - b * S;
                 if (ty < 0 || ty >= K) continue;
+                // (with the epilogue the tiles hang over the plane where the plain kernels' do not: their rows and columns past it
+                // meet no x, so that one that is not finite stays out of the taps it has no part in)
+                if (EPI && !(has_item && b >= skip && oy0 + row0 + b < p.out_h)) continue;
 #pragma unroll
-                for (int tx = 0; tx < K; ++tx)
+                for (int o = 0; o < 4; ++o) {
+                    if (EPI && ANY_WIDTH && o > 0 && ox + o >= p.out_w) continue;
 #pragma unroll
-                    for (int o = 0; o < 4; ++o)
-                        acc[ty * K + tx] = fmaf(g[b][o], win[o * S + tx], acc[ty * K + tx]);
+                    for (int tx = 0; tx < K; ++tx) acc[ty * K + tx] = fmaf(g[b][o], win[o * S + tx], acc[ty * K + tx]);
+                }
             }
             pin_registers(acc);
         }

@@ -138,12 +138,33 @@ def test_non_finite_inputs_stay_where_they_are(gpu, shape):
     x, wt, gy = (t.to(gpu) for t in make_inputs(shape, seed=9))
     scale, shift = params(c, gpu)
     x[:, :, -1, -1] = float("inf")
-    gx, _, s_scale, s_shift = _C.dwconv2d_fused_backward(x, gy, wt, scale, shift, "silu", s, s, p, p)
+    gx, gw, s_scale, s_shift = _C.dwconv2d_fused_backward(x, gy, wt, scale, shift, "silu", s, s, p, p)
     conv_grad, *sums = _C.dwconv2d_epilogue_backward(_C.dwconv2d(x, wt, 1, 1, s, s, p, p, p, p, True), gy, scale, shift, "silu")
-    want, _ = _C.dwconv2d_backward(x, conv_grad, wt, s, s, p, p)
+    want, gw_want = _C.dwconv2d_backward(x, conv_grad, wt, s, s, p, p)
     assert torch.equal(torch.isfinite(gx), torch.isfinite(want)) and not bool(torch.isfinite(want).all())
+    assert not bool((torch.isfinite(gw_want) & ~torch.isfinite(gw)).any())
     assert torch.equal(torch.isfinite(s_scale), torch.isfinite(sums[0]))
     assert torch.equal(torch.isfinite(s_shift), torch.isfinite(sums[1]))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16], ids=["f32", "bf16"])
+@pytest.mark.parametrize("shape", [(1, 2, 40, 36, 3, 1, 1), (1, 2, 56, 56, 3, 1, 1), (1, 2, 75, 75, 3, 1, 1), (1, 2, 75, 75, 5, 1, 2), (1, 2, 64, 129, 5, 1, 2),
+                                   (1, 2, 112, 112, 3, 2, 1), (1, 2, 64, 64, 3, 2, 1), (1, 2, 75, 75, 5, 2, 2), (1, 2, 57, 64, 5, 2, 2)], ids=shape_id)
+def test_infinite_input_reaches_its_own_taps_only(gpu, shape, dtype):
+    """The tiled kernels: blocks that hang over the plane, or repeat a neighbour's rows, add nothing to the filter's gradient.  One
+    infinite element of x, at either end of the plane or inside: the taps whose sums hold it are not finite, the others are."""
+    from torch_dwconv import _C
+
+    n, c, h, w, k, s, p = shape
+    x, wt, gy = (t.to(dtype).to(gpu) for t in make_inputs(shape, seed=19))
+    for iy, ix in ((h - 1, w - 1), (0, 0), (h - 1, w // 2), (h // 2, w - 1), (h // 2, w // 2)):
+        xi = x.clone()
+        xi[:, :, iy, ix] = float("inf")
+        gw = _C.dwconv2d_fused_backward(xi, gy, wt, None, None, None, s, s, p, p)[1]
+        assert _C.last_variant().startswith("bwd_tile"), _C.last_variant()
+        rows, cols = ([(i + p - t) % s == 0 and 0 <= (i + p - t) // s < e for t in range(k)] for i, e in ((iy, gy.shape[2]), (ix, gy.shape[3])))
+        want = torch.tensor([[r and q for q in cols] for r in rows])
+        assert torch.equal(~torch.isfinite(gw).cpu(), want.expand(c, 1, k, k)), (iy, ix, gw)
 
 
 def test_the_rest_takes_the_separate_calls(gpu):
