@@ -402,10 +402,10 @@ def test_rows_of_any_width_fp32(dw, gpu, shape):
     ow = gy.shape[3]
     _C.dwconv2d_backward(xg, gg, wg, s, s, p, p)
     fused = _C.last_variant()
-    if fused.startswith("bwd_stack"):  # (5x5 / 7x7 stride-1 "same" layers: the stacked kernel's own any-width instance)
-        assert fused.endswith(" anywidth"), fused
+    if s == 1 and k >= 5 and p == k // 2:  # 5x5 / 7x7 "same" layers: the stacked kernel's own any-width instance
+        assert fused.startswith("bwd_stack<") and fused.endswith(" anywidth"), fused
     else:
-        assert "vin3" in fused and ("vgy3" in fused or ow % 4 == 0), fused
+        assert not fused.startswith("bwd_stack") and "vin3" in fused and ("vgy3" in fused or ow % 4 == 0), fused
     if s == 2:
         assert "vgx3" in fused, fused
     _C.dwconv2d_backward_kernel(xg, gg, wg, 1, 1, s, s, p, p)
@@ -462,7 +462,16 @@ def test_rows_of_any_width_half_precision(dw, gpu, dtype):
 def test_rows_of_any_width_full_batch(dw, gpu, shape):
     """Layers of the 300-pixel stack (150x150 3x3 stride 1 and 2, 75x75 5x5 stride 2, 38x38 5x5) at batch 128: whole
     tensors against the fp64 reference, outputs start as NaN."""
-    check_full_size(dw, gpu, shape, seed=64, expect=("tile_down<", "bwd_tile"))
+    backward = {(3, 1): "bwd_tile<k3", (3, 2): "bwd_tile_s2<k3", (5, 2): "bwd_tile_s2<k5", (5, 1): "bwd_stack<k5"}[shape[4:6]]
+    check_full_size(dw, gpu, shape, seed=64, expect=("tile_down<", backward))
+
+
+def test_rows_of_any_width_full_batch_general_tiled_kernel(dw, gpu, monkeypatch):
+    """The 38x38 5x5 layer through the general tiled kernel (two planes a workgroup, rows of any width), which serves what
+    the stacked-image kernel refuses."""
+    monkeypatch.setenv("DWCONV_TUNING", "1")
+    monkeypatch.setenv("DWCONV_STACK", "0")
+    check_full_size(dw, gpu, effnet_layers_at(300)[4], seed=64, expect=("tile_down<", "bwd_tile<k5"))
 
 
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
@@ -517,7 +526,7 @@ def test_half_precision_full_batch_stacked_forward(dw, gpu, dtype):
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=["f16", "bf16"])
 def test_half_precision_full_batch_general_tiled_kernels(dw, gpu, dtype, monkeypatch):
     """The 16-bit instances of the general tiled kernels on the 56x56 3x3 layer (they serve what the stacked-image
-    kernel does not take: rows of odd width, tensors off a 32-bit boundary, small planes)."""
+    kernel does not take, planes of fewer than eight rows among it)."""
     monkeypatch.setenv("DWCONV_TUNING", "1")
     monkeypatch.setenv("DWCONV_STACK_K3_16", "0")
     check_full_size(dw, gpu, effnet_layers()[2], seed=41, dtype=dtype, expect=("tile_down16<", "bwd_tile16<"))
@@ -767,7 +776,8 @@ def test_half_precision_uses_the_fast_kernels(dw, gpu):
                             ((2, 8, 56, 56, 3, 1, 1), "tile_down16<", "bwd_stack16<k3"),
                             ((2, 8, 48, 48, 3, 1, 1), "tile_stack16<k3", "bwd_stack16<k3"),
                             ((2, 8, 56, 54, 3, 1, 1), "tile_down16<", "bwd_stack16<k3"),
-                            ((2, 8, 56, 55, 3, 1, 1), "tile_down16<", "bwd_tile16<"),
+                            ((2, 8, 56, 55, 3, 1, 1), "tile_down16<", "bwd_stack16<k3"),
+                            ((2, 8, 7, 55, 3, 1, 1), "tile_down16<", "bwd_tile16<"),
                             ((2, 8, 14, 14, 5, 1, 2), "small_down16", "small_bwd16"),
                             ((2, 8, 28, 28, 3, 1, 1), "small_down16", "small_bwd16")]:
         n, c, h, w, k, s, p = shape
