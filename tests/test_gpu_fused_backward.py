@@ -12,7 +12,7 @@ pytestmark = pytest.mark.gpu
 ACT = {None: lambda z: z, "relu": F.relu, "relu6": F.relu6, "silu": F.silu}
 
 CASES = [
-    # whole planes: exact and ragged widths, one image a chunk and several, channels that do not fill a wavefront
+    # whole planes: exact and ragged widths, channels that do not fill a wavefront (several images a workgroup: below)
     ((3, 12, 7, 7, 3, 1, 1), "small_bwd"), ((2, 5, 14, 14, 5, 1, 2), "small_bwd"), ((2, 7, 11, 13, 3, 1, 1), "small_bwd"),
     ((1, 3, 31, 29, 5, 1, 2), "small_bwd"), ((2, 6, 32, 32, 3, 2, 1), "small_bwd"), ((3, 4, 15, 15, 5, 2, 2), "small_bwd"),
     ((2, 3, 4, 1, 3, 1, 1), "small_bwd"), ((2, 4, 22, 22, 5, 1, 2), "small_bwd"),
@@ -90,6 +90,69 @@ def test_scale_and_shift_sums_over_many_images(gpu, monkeypatch, shape):
     for got, ref in zip(grads[2:], reference(x, wt, gy, scale, shift, None, s, p)[2:]):
         error = float((got.cpu().double() - ref).norm() / ref.norm())
         assert error <= 6 * 2.0 ** -24, (_C.last_variant(), error)
+
+
+def check_against_64_bits(gpu, shape, dtype, seed):
+    """As test_one_sweep; returns the variant."""
+    from torch_dwconv import _C
+
+    n, c, h, w, k, s, p = shape
+    x, wt, gy = (t.to(dtype).to(gpu) for t in make_inputs(shape, seed=seed))
+    scale, shift = params(c, gpu)
+    grads = _C.dwconv2d_fused_backward(x, gy, wt, scale, shift, "silu", s, s, p, p)
+    assert grads is not None
+    variant = _C.last_variant()
+    u = {torch.float32: 0.0, torch.bfloat16: 2.0 ** -8, torch.float16: 2.0 ** -11}[dtype]
+    for got, ref, rounded in zip(grads, reference(x, wt, gy, scale, shift, "silu", s, p), (True, True, False, False)):
+        err = (got.cpu().double() - ref).abs()
+        bound = (u if rounded else 0.0) * ref.abs() + 2e-5 * ref.abs().max()
+        assert bool((err <= bound).all()), (variant, float(err.max()), float(ref.abs().max()))
+    return variant
+
+
+# (shape, family): whole planes on and off 4-element boundaries, with and without the prefetch of the next image;
+# tiles whose in_grad leaves through LDS (fp32 3x3, 56 and 60 columns), rows of any width, two planes a workgroup, two bands
+SEVERAL = [((7, 5, 7, 7, 3, 1, 1), "small_bwd"), ((5, 4, 14, 14, 5, 1, 2), "small_bwd"), ((5, 3, 13, 11, 5, 1, 2), "small_bwd"),
+           ((5, 3, 28, 28, 5, 1, 2), "small_bwd"), ((5, 3, 28, 28, 3, 2, 1), "small_bwd"), ((5, 3, 15, 15, 5, 2, 2), "small_bwd"),
+           ((5, 2, 56, 56, 3, 1, 1), "bwd_tile"), ((3, 2, 130, 60, 3, 1, 1), "bwd_tile"), ((5, 3, 38, 38, 5, 1, 2), "bwd_tile"),
+           ((5, 5, 33, 35, 3, 1, 1), "bwd_tile"), ((3, 1, 75, 75, 3, 1, 1), "bwd_tile"), ((3, 2, 64, 129, 5, 1, 2), "bwd_tile"),
+           ((5, 3, 38, 38, 3, 2, 1), "bwd_tile_s2"), ((3, 1, 75, 75, 5, 2, 2), "bwd_tile_s2"), ((3, 2, 112, 112, 3, 2, 1), "bwd_tile_s2"),
+           ((5, 1, 47, 57, 5, 2, 2), "bwd_tile_s2")]
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16, torch.float16], ids=["f32", "bf16", "f16"])
+@pytest.mark.parametrize("case", SEVERAL, ids=lambda c: shape_id(c[0]))
+def test_several_tiles_a_workgroup(gpu, monkeypatch, case, dtype):
+    """One workgroup a channel group, so that it walks every image and band: LDS whose gy was replaced in place is staged again, the
+    next image is prefetched, sums and results leave between tiles."""
+    shape, family = case
+    cap_grids(monkeypatch)
+    variant = check_against_64_bits(gpu, shape, dtype, seed=29)
+    assert variant.startswith(family) and ",epi>" in variant and variant.split(" chunks")[1].split(" ")[0] == "1", variant
+    assert shape[0] >= 3
+
+
+# Layers of 4 Mi elements and more, on both sides of the rules that send some of them to three calls; the same planes with fewer
+# elements always take one sweep.
+@pytest.mark.parametrize("shape,dtype,one_sweep", [
+    ((9, 144, 64, 64, 3, 1, 1), torch.bfloat16, False), ((10, 144, 56, 56, 3, 1, 1), torch.bfloat16, True),
+    ((9, 144, 64, 64, 5, 1, 2), torch.float32, False), ((9, 144, 64, 64, 3, 1, 1), torch.float32, True),
+    ((9, 144, 64, 64, 5, 1, 2), torch.bfloat16, False), ((3, 144, 112, 112, 5, 1, 2), torch.bfloat16, False),
+    ((5, 144, 80, 80, 5, 1, 2), torch.bfloat16, True), ((21, 144, 38, 38, 3, 2, 1), torch.bfloat16, False),
+    ((19, 144, 40, 40, 3, 2, 1), torch.bfloat16, True), ((8, 144, 64, 64, 5, 2, 2), torch.bfloat16, False),
+    ((10, 144, 56, 56, 5, 2, 2), torch.bfloat16, True), ((8, 144, 64, 64, 5, 2, 2), torch.float32, True)],
+    ids=lambda v: shape_id(v) if isinstance(v, tuple) else str(v).split(".")[-1])
+def test_which_large_layers_take_one_sweep(gpu, shape, dtype, one_sweep):
+    from torch_dwconv import _C
+
+    n, c, h, w, k, s, p = shape
+    assert n * c * h * w >= 4 << 20 and (n // 2) * c * h * w < 4 << 20
+    x, wt, gy = (t.to(dtype).to(gpu) for t in make_inputs(shape, seed=31))
+    grads = _C.dwconv2d_fused_backward(x, gy, wt, None, None, "silu", s, s, p, p)
+    assert (grads is not None) == one_sweep
+    assert _C.dwconv2d_fused_backward(x[:n // 2], gy[:n // 2], wt, None, None, "silu", s, s, p, p) is not None
+    if one_sweep:
+        check_against_64_bits(gpu, shape, dtype, seed=31)
 
 
 @pytest.mark.parametrize("shape", [(2, 4, 14, 14, 3, 1, 1), (1, 3, 29, 28, 5, 1, 2), (2, 2, 56, 56, 3, 1, 1), (1, 2, 75, 75, 3, 1, 1),
