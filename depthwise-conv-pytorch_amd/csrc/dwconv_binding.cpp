@@ -30,7 +30,8 @@ namespace {
 
 using at::Tensor;
 
-struct NotHere {};  // the call is one for the Python function
+struct NotHere {};   // the call is one for the Python function
+struct NoKernel {};  // (fused_backward) a call to serve here, but no kernel makes it: False
 
 // The arguments of one call, taken from left to right.
 class Args {
@@ -420,7 +421,7 @@ Results epilogue_backward(Args a)
 }
 
 // (input, out_grad, kernel, scale | None, shift | None, activation, stride_h, stride_w, pad_h, pad_w)
-//   -> (in_grad, kernel_grad, scale_grad, shift_grad), or not here where no kernel makes them in one sweep
+//   -> (in_grad, kernel_grad, scale_grad, shift_grad), or False where no kernel makes them in one sweep
 Results fused_backward(Args a)
 {
     const Tensor input = a.tensor(), grad = a.tensor(), kernel = a.tensor();
@@ -432,12 +433,12 @@ Results fused_backward(Args a)
     together(input, grad);
     if (grad.dim() != 4 || grad.size(0) != input.size(0) || grad.size(1) != input.size(1)) throw NotHere{};
     const Type type = type_of(input);
-    if (type == F64 || channels_last(input)) throw NotHere{};
+    if (type == F64 || channels_last(input)) throw NoKernel{};
     const int n = extent(input, 0), c = extent(input, 1), h = extent(input, 2), w = extent(input, 3), oh = extent(grad, 2), ow = extent(grad, 3);
     const int kh = extent(kernel, 2), kw = extent(kernel, 3);
     const size_t bytes = dwconv2d_fused_backward_workspace_bytes(n, c, h, w, oh, ow, kh, kw, sh, sw, ph, pw,
                                                                  static_cast<int>(input.element_size()));
-    if (bytes == 0) throw NotHere{};
+    if (bytes == 0) throw NoKernel{};
     const c10::optional<Tensor> scale = per_channel(scale_, input), shift = per_channel(shift_, input);
     const Tensor x = input.contiguous(), gy = grad.contiguous(), k = kernel.contiguous();
     const Tensor gx = at::empty_like(x);
@@ -449,7 +450,7 @@ Results fused_backward(Args a)
     call(x, [&](void *s) {                                                                                                     \
         const int rc = FN(in<T>(x), in<T>(gy), in<T>(k), sc, sf, out<T>(gx), out<T>(gw), out<float>(grads),                    \
                           ws.mutable_data_ptr(), bytes, n, c, h, w, oh, ow, kh, kw, sh, sw, ph, pw, act, s);                   \
-        if (rc == DWCONV_ERR_UNSUPPORTED) throw NotHere{};                                                                     \
+        if (rc == DWCONV_ERR_UNSUPPORTED) throw NoKernel{};                                                                     \
         return rc;                                                                                                             \
     });
     switch (type) {
@@ -566,6 +567,8 @@ PyObject *entry(PyObject *, PyObject *const *args, Py_ssize_t n)
     try {
         if (!observed()) return wrap(F(Args(args, n)));
     } catch (const NotHere &) {
+    } catch (const NoKernel &) {
+        Py_RETURN_FALSE;
     }
     Py_RETURN_NONE;
     END_HANDLE_TH_ERRORS

@@ -110,6 +110,12 @@ for _sfx in ("f32", "f16", "bf16"):
     getattr(_lib, "dwconv2d_epilogue_backward_" + _sfx).restype = _i
     getattr(_lib, "dwconv2d_epilogue_backward_" + _sfx).argtypes = [_p] * 7 + [_z] + [_i] * 6 + [_p]
 
+_lib.dwconv2d_fused_backward_workspace_bytes.restype = _z
+_lib.dwconv2d_fused_backward_workspace_bytes.argtypes = [_i] * 13
+for _sfx in ("f32", "f16", "bf16"):
+    getattr(_lib, "dwconv2d_fused_backward_" + _sfx).restype = _i
+    getattr(_lib, "dwconv2d_fused_backward_" + _sfx).argtypes = [_p] * 9 + [_z] + [_i] * 13 + [_p]
+
 _lib.dwconv2d_general_backward_workspace_bytes.restype = _z
 _lib.dwconv2d_general_backward_workspace_bytes.argtypes = [_i] * 14
 for _sfx in ("f32", "f64", "f16", "bf16"):
@@ -117,6 +123,8 @@ for _sfx in ("f32", "f64", "f16", "bf16"):
     getattr(_lib, "dwconv2d_general_" + _sfx).argtypes = [_p, _p, _p] + [_i] * 13 + [_p]
     getattr(_lib, "dwconv2d_general_backward_" + _sfx).restype = _i
     getattr(_lib, "dwconv2d_general_backward_" + _sfx).argtypes = [_p, _p, _p, _p, _p, _p, _z] + [_i] * 15 + [_p]
+
+_ERR_UNSUPPORTED = 2  # DWCONV_ERR_UNSUPPORTED
 
 ACTIVATIONS = {None: 0, "none": 0, "relu": 1, "relu6": 2, "silu": 3}
 
@@ -488,12 +496,44 @@ def dwconv2d_epilogue_backward(conv_out, out_grad, scale, shift, activation):
 
 def dwconv2d_fused_backward(input, out_grad, kernel, scale, shift, activation, stride_h, stride_w, pad_h, pad_w):
     """All gradients of ``dwconv2d_fused`` in one sweep over an NCHW ``input`` and ``out_grad``:
-    ``(input_grad, kernel_grad, scale_grad, shift_grad)``, or ``None`` where no kernel makes them together (and where
-    there is no native module): the convolution, ``dwconv2d_epilogue_backward`` and ``dwconv2d_backward`` then do."""
+    ``(input_grad, kernel_grad, scale_grad, shift_grad)``, or ``None`` where no kernel makes them together: the
+    convolution, ``dwconv2d_epilogue_backward`` and ``dwconv2d_backward`` then do (and raise the errors)."""
     if activation not in ACTIVATIONS:
         return None
-    return _binding.fused_backward(input, out_grad, kernel, scale, shift, ACTIVATIONS[activation], stride_h, stride_w,
-                                   pad_h, pad_w)
+    native = _binding.fused_backward(input, out_grad, kernel, scale, shift, ACTIVATIONS[activation], stride_h, stride_w,
+                                     pad_h, pad_w)
+    if native is not None:
+        return native or None
+    same = [input, out_grad, kernel]
+    if any(t.dim() != 4 or not t.is_cuda or t.dtype != input.dtype or t.device != input.device for t in same) or \
+            _SUFFIX.get(input.dtype, "f64") == "f64" or is_channels_last(input):
+        return None
+    n, c, h, w = input.shape
+    oh, ow = out_grad.shape[2:]
+    kh, kw = kernel.shape[2:]
+    if kernel.shape[:2] != (c, 1) or out_grad.shape[:2] != (n, c) or \
+            any(t is not None and (not t.is_cuda or t.numel() != c) for t in (scale, shift)):
+        return None
+    geometry = (n, c, h, w, oh, ow, kh, kw, stride_h, stride_w, pad_h, pad_w)
+    ws_bytes = _lib.dwconv2d_fused_backward_workspace_bytes(*geometry, input.element_size())
+    if ws_bytes == 0:
+        return None
+    params = [t if t is None else t.detach().reshape(-1).to(device=input.device, dtype=torch.float32).contiguous()
+              for t in (scale, shift)]
+    x, gy, k = input.contiguous(), out_grad.contiguous(), kernel.contiguous()
+    gx, gw = torch.empty_like(x), torch.empty_like(k)
+    grads = torch.empty((c, 2), dtype=torch.float32, device=x.device)
+    ws = torch.empty(ws_bytes, dtype=torch.uint8, device=x.device)
+    with torch.cuda.device(x.device):
+        rc = getattr(_lib, "dwconv2d_fused_backward_" + _SUFFIX[x.dtype])(
+            x.data_ptr(), gy.data_ptr(), k.data_ptr(), *(t if t is None else t.data_ptr() for t in params), gx.data_ptr(),
+            gw.data_ptr(), grads.data_ptr(), ws.data_ptr(), ws_bytes, *geometry, ACTIVATIONS[activation], _stream(x),
+        )
+    if rc == _ERR_UNSUPPORTED:
+        return None
+    if rc != 0:
+        _raise(rc)
+    return gx, gw, grads[:, 0], grads[:, 1]
 
 
 # ---- dilation and depth multiplier -----------------------------------------------------------------------

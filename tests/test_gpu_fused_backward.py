@@ -230,9 +230,12 @@ def test_infinite_input_reaches_its_own_taps_only(gpu, shape, dtype):
         assert torch.equal(~torch.isfinite(gw).cpu(), want.expand(c, 1, k, k)), (iy, ix, gw)
 
 
-def test_the_rest_takes_the_separate_calls(gpu):
+@pytest.mark.parametrize("native", [True, False], ids=["native", "ctypes"])
+def test_the_rest_takes_the_separate_calls(gpu, monkeypatch, native):
     from torch_dwconv import _C
 
+    if not native:
+        monkeypatch.setattr(_C, "_binding", _C._NoBinding())
     x, w = torch.randn(2, 4, 20, 20, device=gpu), torch.randn(4, 1, 7, 7, device=gpu)
     assert _C.dwconv2d_fused_backward(x, x, w, None, None, "silu", 1, 1, 3, 3) is None  # 7x7
     w = torch.randn(4, 1, 3, 3, device=gpu)
@@ -240,3 +243,29 @@ def test_the_rest_takes_the_separate_calls(gpu):
     assert _C.dwconv2d_fused_backward(x.double(), x.double(), w.double(), None, None, "silu", 1, 1, 1, 1) is None
     y = x.contiguous(memory_format=torch.channels_last)
     assert _C.dwconv2d_fused_backward(y, y, w, None, None, "silu", 1, 1, 1, 1) is None
+    for bad in (x[:1], x[:, :3], x.half(), x.cpu(), x[0]):
+        assert _C.dwconv2d_fused_backward(x, bad, w, None, None, "silu", 1, 1, 1, 1) is None
+    for bad in (torch.ones(3, device=gpu), torch.ones(4)):
+        assert _C.dwconv2d_fused_backward(x, x, w, bad, None, "silu", 1, 1, 1, 1) is None
+    assert _C.dwconv2d_fused_backward(x, x, w[:3], None, None, "silu", 1, 1, 1, 1) is None
+    assert _C.dwconv2d_fused_backward(x, x, w, None, None, "gelu", 1, 1, 1, 1) is None
+    assert _C.dwconv2d_fused_backward(x, x, w, None, None, "silu", 1, 1, 1, 1) is not None
+
+
+def test_a_dispatch_mode_changes_nothing(gpu):
+    """Under a mode the calls go through their Python forms: the same kernel, the same bits."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from torch_dwconv import _C
+
+    class Mode(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            return func(*args, **(kwargs or {}))
+
+    n, c, h, w, k, s, p = shape = (2, 6, 28, 28, 5, 1, 2)
+    x, wt, gy = (t.to(gpu) for t in make_inputs(shape, seed=37))
+    scale, shift = params(c, gpu)
+    plain = _C.dwconv2d_fused_backward(x, gy, wt, scale, shift, "silu", s, s, p, p)
+    with Mode():
+        moded = _C.dwconv2d_fused_backward(x, gy, wt, scale, shift, "silu", s, s, p, p)
+    assert all(torch.equal(a, b) and a.stride() == b.stride() for a, b in zip(plain, moded))

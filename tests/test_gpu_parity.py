@@ -947,6 +947,7 @@ NATIVE_CALLS = [
     ("dwconv2d_backward_nhwc", "xgw", (1, 1, 1, 1), True), ("dwconv2d_backward_nhwc", "xgw", (1, 1, 1, 1, True, False), True),
     ("dwconv2d_fused", "xwpp", ("silu", 1, 1, 1, 1), False), ("dwconv2d_fused", "xwnp", ("relu", 2, 2, 0, 1), True),
     ("dwconv2d_epilogue_backward", "xgpn", ("silu",), False), ("dwconv2d_epilogue_backward", "xgpp", ("relu6",), True),
+    ("dwconv2d_fused_backward", "xgwpp", ("silu", 1, 1, 1, 1), False), ("dwconv2d_fused_backward", "xgwnp", ("relu", 1, 1, 1, 1), False),
     ("dwconv2d_general", "xw", (1, 1, 2, 2, 2, 2), False), ("dwconv2d_general_backward", "xgw", (1, 1, 1, 1, 1, 1), False),
 ]
 
