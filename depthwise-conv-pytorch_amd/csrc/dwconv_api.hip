@@ -315,12 +315,12 @@ size_t fused_backward_workspace(const WgradGeometry &g, size_t esize)
 }
 
 // One sweep instead of three (the convolution again, its result and out_grad into its gradient, that through the backward
-// kernels): 2 |x| + |y| elements are moved instead of 3 |x| + 6 |y|, and the added multiply-adds are those of the convolution.
+// kernels): 2 |x| + |y| elements are moved instead of 3 |x| + 5 |y|, and the added multiply-adds are those of the convolution.
 // Measured at batch 128 with SiLU, us, three calls / one:
-//   fp32  3x3 C=32 112x112 317 / 159   C=96 112x112 stride 2 491 / 297   C=144 56x56 359 / 180   C=480 14x14 79 / 37   C=1152 7x7 65 / 27
-//         5x5 C=144 56x56 stride 2 193 / 128   C=240 28x28 145 / 118   C=672 14x14 110 / 62   C=1152 7x7 75 / 36
-//   bf16  177 / 154, 266 / 238, 224 / 172, 56 / 31, 54 / 24; 142 / 125, 105 / 107, 88 / 57, 64 / 35
-//   batch 64, 300 pixels: fp32 5x5 75x75 C=144 stride 2 230 / 160, bf16 3x3 150x150 C=32 241 / 170, 38x38 C=240 5x5 175 / 154
+//   fp32  3x3 C=32 112x112 303 / 157   C=96 112x112 stride 2 483 / 299   C=144 56x56 343 / 184   C=480 14x14 73 / 33   C=1152 7x7 63 / 27
+//         5x5 C=144 56x56 stride 2 180 / 125   C=240 28x28 141 / 82   C=672 14x14 104 / 60   C=1152 7x7 71 / 36
+//   bf16  163 / 140, 265 / 247, 207 / 156, 53 / 31, 53 / 24; 131 / 114, 103 / 75, 88 / 55, 63 / 35
+//   batch 64, 300 pixels: fp32 5x5 75x75 C=144 stride 2 190 / 145, bf16 3x3 150x150 C=32 173 / 166, 75x75 C=144 295 / 249
 template <typename T>
 int fused_backward_any(const T *in, const T *gy, const T *taps, T *gx, T *gw, float *param_grad, const EpilogueBackward &epi, void *ws,
                        size_t ws_bytes, const WgradGeometry &g, hipStream_t stream)

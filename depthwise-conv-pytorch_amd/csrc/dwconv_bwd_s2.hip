@@ -20,8 +20,6 @@ namespace dwconv {
 
 namespace {
 
-constexpr long kFusedFewElements = 4l << 20;  // of the input: below, one launch instead of four is what counts
-
 // Both images of a tile.  At 36 KiB the 5x5 kernels on 75- to 80-wide maps get one band more, which is nearly empty: bf16,
 // batch 64, 75x75 C=144 219 us against 162 at 40 KiB, 80x80 106 / 80; fp32 75x75 148 / 138; every other layer of 185- to
 // 320-pixel EfficientNets within 2 %.  48 KiB leaves three workgroups per CU: 117x117 C=96 3x3 5 % slower.

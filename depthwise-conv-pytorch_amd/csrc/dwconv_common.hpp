@@ -342,6 +342,8 @@ template <typename IO>
 int launch_fused_final(const float *partial, IO *gw, float *param_grad, int channel, int taps, int chunks, hipStream_t stream);
 
 // ---- backward of act(conv(x, w) * scale + shift) in one sweep (the convolution is recomputed in LDS) ----
+// Elements of the input below which such a layer always takes it: two launches instead of five are what counts there.
+constexpr long kFusedFewElements = 4l << 20;
 // Workspace bytes (0: the kernels do not cover g) and launch (-1 likewise).
 size_t fused_small_workspace(const WgradGeometry &g, size_t esize);
 template <typename IO>

@@ -1033,7 +1033,7 @@ bool plan_nhwc(NhwcPlan &p, const NhwcGeometry &g, int bh, int tw, int blocks_h,
     p.blocks_y = ceil_div(blocks_h, bh);
     p.blocks_x = ceil_div(blocks_w, tw);
     const long blocks = static_cast<long>(g.batch) * p.blocks_y * p.blocks_x;
-    if (blocks <= 0 || blocks >= (1l << 31) - kNhwcThreads) return false;  // (of four channels or more: far past the GPU's memory)
+    if (blocks <= 0 || blocks >= (1l << 31) - kNhwcThreads) return false;  // (the direct kernels take those)
     p.blocks_total = static_cast<int>(blocks);
     p.per_image_div = exact_div(static_cast<unsigned>(p.blocks_y) * p.blocks_x);
     p.blocks_x_div = exact_div(p.blocks_x);

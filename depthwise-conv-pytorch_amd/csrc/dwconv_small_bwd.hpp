@@ -113,8 +113,9 @@ constexpr bool fused_prefetch(int w, int k, int s)
 // PAD: LDS rows of 8, 16 or 32 floats get four spare floats (see lds_row_pitch)
 // D: dilation of the taps (stride 1 only; the padding is then D * (K/2)).
 // EPI (with GX): gy is the gradient of act(conv * scale + shift).  The same three tensors are moved; the convolution and the
-// activation's slope add a third of the multiply-adds and a walk over the x rows in LDS (batch 128, fp32, us without it / with
-// it, against the two launches that it saves: 14x14 C=480 3x3 26 / 37 (47), 5x5 33 / 50 (47); 7x7 C=1152 5x5 24 / 36 (41)).
+// activation's slope add half as many multiply-adds again and a walk over the x rows in LDS (batch 128, fp32, us without it / with
+// it, and the convolution and the sweep that it saves: 14x14 C=480 3x3 28 / 33 (46), 5x5 32 / 48 (49); 7x7 C=1152 5x5 25 / 36 (41);
+// 28x28 C=240 5x5 53 / 82 (89)).
 template <typename IO, int W, bool RAG, int K, int S, int BH, bool GX, bool PAD, int D = 1, bool EPI = false,
           bool PF = EPI ? fused_prefetch<IO>(W, K, S) : (sizeof(IO) == 2 || (K < 7 && (RAG || W <= 28 || K == 3)))>
 __global__ __launch_bounds__(kWave, EPI ? 2 : 1) void small_bwd_kernel(const SmallBwdPlan p)
@@ -475,16 +476,16 @@ long small_bwd_case(int mode, const SmallBwdArgs &a, const WgradGeometry &g, hip
                      PAD ? ",pad" : "", p.planes_per_run, p.chunks);
         return launch_fused_final(p.partial, static_cast<IO *>(a.gw), a.param_grad, g.channel, K * K, p.chunks, stream);
     } else {
-    if (mode == 2)
-        hipLaunchKernelGGL((small_bwd_kernel<IO, W, RAG, K, S, BH, true, PAD, D>), dim3(groups * p.chunks), dim3(kWave), shmem, stream, p);
-    else
-        hipLaunchKernelGGL((small_bwd_kernel<IO, W, RAG, K, S, BH, false, PAD, D>), dim3(groups * p.chunks), dim3(kWave), shmem, stream, p);
-    const int rc = check_launch("small_bwd_kernel");
-    if (rc != DWCONV_OK) return rc;
-    note_variant("%s%s<%s%d,k%d,s%d,bh%d%s%s> P%d chunks%d", mode == 2 ? "small_bwd" : "small_wgrad",
-                 sizeof(IO) == 2 ? "16" : "", RAG ? "r" : "w", W, K, S, BH, PAD ? ",pad" : "", D == 2 ? ",d2" : "",
-                 p.planes_per_run, p.chunks);
-    return launch_wgrad_final(p.partial, static_cast<IO *>(a.gw), g.channel, K * K, p.chunks, stream);
+        if (mode == 2)
+            hipLaunchKernelGGL((small_bwd_kernel<IO, W, RAG, K, S, BH, true, PAD, D>), dim3(groups * p.chunks), dim3(kWave), shmem, stream, p);
+        else
+            hipLaunchKernelGGL((small_bwd_kernel<IO, W, RAG, K, S, BH, false, PAD, D>), dim3(groups * p.chunks), dim3(kWave), shmem, stream, p);
+        const int rc = check_launch("small_bwd_kernel");
+        if (rc != DWCONV_OK) return rc;
+        note_variant("%s%s<%s%d,k%d,s%d,bh%d%s%s> P%d chunks%d", mode == 2 ? "small_bwd" : "small_wgrad",
+                     sizeof(IO) == 2 ? "16" : "", RAG ? "r" : "w", W, K, S, BH, PAD ? ",pad" : "", D == 2 ? ",d2" : "",
+                     p.planes_per_run, p.chunks);
+        return launch_wgrad_final(p.partial, static_cast<IO *>(a.gw), g.channel, K * K, p.chunks, stream);
     }
 }
 

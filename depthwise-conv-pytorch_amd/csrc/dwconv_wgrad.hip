@@ -56,7 +56,6 @@ struct WgradPlan {
     EpilogueBackward epi;
 };
 
-constexpr long kFusedFewElements = 4l << 20;  // of the input: below, one launch instead of four is what counts
 constexpr int kFusedRows = 4;                 // rows per lane with the epilogue's backward
 constexpr int kFusedEpilogueLds = 48 * 1024;  // both images of a tile with the epilogue's backward
 
@@ -68,8 +67,8 @@ constexpr int kFusedEpilogueLds = 48 * 1024;  // both images of a tile with the 
 // EPI (with GX): gy is the gradient of act(conv * scale + shift).  The x image reaches K/2 rows further up and down, so that
 // the convolution of every row of the gy image can be recomputed from it; each lane does so for the BH x 4 block at its place
 // in the gy image and replaces gy there by the gradient of the convolution.  A tile is then units * BH - 2 (K/2) rows, and the
-// last lane of a column takes the last BH of them, of which it owns those no other lane has.  Bound by HBM and, at a third
-// more multiply-adds than without it, by its instructions; 2 |x| + |y| elements are moved where the separate calls move 3 |x| + 6 |y|.
+// last lane of a column takes the last BH of them, of which it owns those no other lane has.  Bound by HBM and, with half
+// again the multiply-adds of the plain kernel, by its instructions; 2 |x| + |y| elements are moved where the separate calls move 3 |x| + 5 |y|.
 // ANY_WIDTH: the instance for rows that are not whole, aligned groups of four elements (a mode 3 among st.vec_in,
 // vec_gy, vec_gx); the other instance carries none of it.
 template <typename IO, int K, int S, int BH, bool GX, bool ANY_WIDTH = false, bool EPI = false>

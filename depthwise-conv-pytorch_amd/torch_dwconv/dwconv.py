@@ -200,11 +200,14 @@ class DepthwiseConv2dFusedFunction(Function):
     into the gradient of the convolution result plus the gradients of ``scale`` and ``shift``
     (``_C.dwconv2d_epilogue_backward``), and that goes through the ordinary backward kernels.  NCHW layers with 3x3 and
     5x5 filters and "same" padding take one kernel for all of it (``_C.dwconv2d_fused_backward``), which recomputes the
-    convolution from the input tile that it holds for the filter's gradient.
+    convolution from the input tile that it holds for the filter's gradient, where both ``input`` and ``kernel`` need a
+    gradient and where that is faster: float16 / bfloat16 layers (and float32 5x5 ones) of 4 Mi input elements and more
+    take either way by the extent of their maps.
 
     Corner behaviour with float16 / bfloat16 tensors and ReLU / ReLU6: the forward kernel applies the activation to
-    its fp32 sum, the backward pass (but for that one kernel) takes the mask from the recomputed result after that was
-    rounded to 16 bits.
+    its fp32 sum, the backward pass takes the mask from the recomputed result after that was rounded to 16 bits, or,
+    in that one kernel, before.  Which of the two follows the rules above, so the mask of one layer may change with the
+    batch and with the gradients asked for.
     An output whose pre-activation lies within one 16-bit rounding step of 0 (or of 6) can therefore get the slope
     of the other side of the corner; no other output is affected (with fp32 tensors the window shrinks to the last
     bit of the fp32 sum)."""
