@@ -527,7 +527,8 @@ long bwd_s2_case(int mode, const IO *x, const IO *gy, const IO *taps, IO *gx, IO
 // Whether one sweep beats the three calls.  It does with fp32 tensors (0.6 to 0.9 of their time) and with 16-bit ones of few
 // elements, where launches count (batch 4, C=144: 0.5 to 0.9).  Else their two-step staging makes up for the extra passes in
 // part: time of one sweep to three calls at C = 144, batch 96, bf16, by columns: 3x3 34 1.08, 38 1.08, 40 0.87, 56 0.72, 80 0.90,
-// 112 0.91, 150 0.78; 5x5 34 1.11, 40 0.97, 48 0.92, 56 0.85, 60 0.90, 64 1.10, 75 1.01, 90 1.13, 112 1.20, 150 1.12.
+// 112 0.91, 150 0.78 (rows of any width, 41 to 106, 0.67 to 0.99, 117 1.09); 5x5 34 1.11, 40 0.97, 48 0.92, 56 0.85, 60 0.90,
+// 64 1.10, 75 1.01, 90 1.13, 112 1.20, 150 1.12 (rows of any width, 41 to 59, 0.84 to 1.04, 61 1.29).
 bool fused_s2_pays(const WgradGeometry &g, size_t esize)
 {
     const long elements = static_cast<long>(g.batch) * g.channel * g.in_h * g.in_w;

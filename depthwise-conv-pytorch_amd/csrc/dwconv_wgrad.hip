@@ -1096,7 +1096,9 @@ size_t fused_tiled_bytes(const WgradPlan &p)
 // time of one sweep to three calls at C = 144, batch 96, by columns: bf16 3x3 56 (0.77) 0.74, 64 (0.50) 1.07, 44 (0.47) 1.02,
 // 112 (0.77) 0.79; bf16 5x5 40 (0.78) 0.95, 48 (0.56) 1.11, 60 (0.88) 0.87, 64 (0.50) 1.31, 72 (0.63) 1.07, 80 (0.78) 0.95, 112 (0.77)
 // 1.07; fp32 5x5 44 (0.47) 1.06, 64 (0.50) 0.96 (batch 32: 1.18), 68 (0.56) 0.84; fp32 3x3 is faster in one sweep everywhere.
-// Small tensors take it too: launches count there.
+// Small tensors take it too: launches count there.  Rows of any width are not told apart, though their plain backward (stacked, loads behind the
+// arithmetic) is faster than that of the tiled kernel: bf16 3x3 33 to 150 columns 0.75 to 0.95, but 34 1.06, 46 1.13, 66 1.10; bf16 5x5 38 1.12, 54 to 59 1.05 to
+// 1.10, 75 1.09, 93 1.15; fp32 5x5 33 to 150 0.73 to 1.04; fp32 3x3 0.50 to 0.76.
 template <int K>
 bool fused_tiled_pays(const WgradPlan &p, size_t esize)
 {
