@@ -61,7 +61,7 @@ struct BwdS2Plan {
 // EPI (padding K/2): gy is the gradient of act(conv * scale + shift).  The x image covers every gy row that a tile's in_grad
 // depends on, K/2 more than its own, so each lane recomputes the convolution of a BQ x 2 block of them and replaces gy in LDS
 // by the gradient of the convolution; two more sums are the gradients of scale and shift.  A tile is units * BQ - K/2 rows, and
-// the last lane of a column takes the last BQ of them, of which it owns those no other lane has.
+// the last lanes of a column take the last BQ of them, of which they own those no other lane has.
 constexpr int kPrefetchSlots = 8;  // loads per lane and image at most (the planner checks rows_fit)
 
 template <typename IO, int K, int E, int BQ, bool VIEWS, bool PF = false, bool EPI = false>
@@ -90,11 +90,6 @@ __global__ __launch_bounds__(kThreads) void bwd_s2_kernel(const BwdS2Plan p)
     const int cb = item - rb * p.ncb;
     static_assert(!EPI || !PF, "the epilogue's instances stage in one step");
     constexpr int M = (K - 1 - K / 2 + E) / 2;  // p.m of the epilogue's instances
-    const int qb = EPI ? min(rb * BQ, p.rows_per_tile - BQ) : rb * BQ;  // first gy row of this lane's block in the tile ...
-    const int skip = EPI ? rb * BQ - qb : 0;                            // ... whose first rows belong to another lane
-    // (the epilogue's x image starts at the window of gy row q0 - M + E, the first one that in_grad depends on)
-    const float *base_x = lds + ((EPI ? qb + M - E : qb) * 2) * p.sx.pitch + kSlack + 4 * cb;
-    const float *base_g = lds + p.g_base + qb * p.sg.pitch + kSlack + 2 * cb;
     EpilogueSums sums;
     float e_scale = 1.f, e_shift = 0.f;
     if constexpr (EPI) p.epi.load(c, e_scale, e_shift);
@@ -131,6 +126,13 @@ __global__ __launch_bounds__(kThreads) void bwd_s2_kernel(const BwdS2Plan p)
         const int n = tile / p.row_tiles, rt = tile - n * p.row_tiles;
         const long plane0 = static_cast<long>(n) * p.channel + c;
         const int q0 = rt * p.rows_per_tile;
+        // The first gy row of this lane's block in the tile, and how many of its first rows belong to another lane.  (With the epilogue
+        // the last blocks end with the band and the plane, as in wgrad_tile_kernel: no row past the plane meets x.)
+        const int qb = EPI ? max(min(rb * BQ, min(p.rows_per_tile, p.out_h - q0) - BQ), 0) : rb * BQ;
+        const int skip = EPI ? rb * BQ - qb : 0;
+        // (the epilogue's x image starts at the window of gy row q0 - M + E, the first one that in_grad depends on)
+        const float *base_x = lds + ((EPI ? qb + M - E : qb) * 2) * p.sx.pitch + kSlack + 4 * cb;
+        const float *base_g = lds + p.g_base + qb * p.sg.pitch + kSlack + 2 * cb;
 
         if constexpr (PF) {
             // (every lane read its gy windows of the previous tile before that tile's second barrier)
@@ -324,14 +326,10 @@ __global__ __launch_bounds__(kThreads) void bwd_s2_kernel(const BwdS2Plan p)
             for (int bq = 0; bq < BQ; ++bq) {
                 const int ty = wr - 2 * bq;
                 if (ty < 0 || ty >= K) continue;
-                // (with the epilogue a tile hangs over the plane by other rows than the plain kernel's: those past it meet no x)
-                if (EPI && !(has_item && 2 * cb < p.out_w && bq >= skip && q0 + qb + bq < p.out_h)) continue;
 #pragma unroll
-                for (int o = 0; o < 2; ++o) {
-                    if (EPI && o > 0 && 2 * cb + o >= p.out_w) continue;
+                for (int tx = 0; tx < K; ++tx)
 #pragma unroll
-                    for (int tx = 0; tx < K; ++tx) wacc[ty * K + tx] = fmaf(g[bq][o], win[2 * o + tx], wacc[ty * K + tx]);
-                }
+                    for (int o = 0; o < 2; ++o) wacc[ty * K + tx] = fmaf(g[bq][o], win[2 * o + tx], wacc[ty * K + tx]);
             }
             pin_registers(wacc);
         }

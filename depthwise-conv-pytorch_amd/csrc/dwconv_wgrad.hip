@@ -67,7 +67,7 @@ constexpr int kFusedEpilogueLds = 48 * 1024;  // both images of a tile with the 
 // EPI (with GX): gy is the gradient of act(conv * scale + shift).  The x image reaches K/2 rows further up and down, so that
 // the convolution of every row of the gy image can be recomputed from it; each lane does so for the BH x 4 block at its place
 // in the gy image and replaces gy there by the gradient of the convolution.  A tile is then units * BH - 2 (K/2) rows, and the
-// last lane of a column takes the last BH of them, of which it owns those no other lane has.  Bound by HBM and, with half
+// last lanes of a column take the last BH of them, of which they own those no other lane has.  Bound by HBM and, with half
 // again the multiply-adds of the plain kernel, by its instructions; 2 |x| + |y| elements are moved where the separate calls move 3 |x| + 5 |y|.
 // ANY_WIDTH: the instance for rows that are not whole, aligned groups of four elements (a mode 3 among st.vec_in,
 // vec_gy, vec_gx); the other instance carries none of it.
@@ -107,10 +107,6 @@ __global__ __launch_bounds__(kThreads) void wgrad_tile_kernel(const WgradPlan p)
     const int cb = rem - rb * p.ncb;
     const int ox = 4 * cb;
     constexpr int HALO = EPI ? K / 2 : 0;
-    const int row0 = EPI ? min(rb * BH, p.rows_per_tile - BH) : rb * BH;  // first row of this lane's block in the tile ...
-    const int skip = EPI ? rb * BH - row0 : 0;                            // ... whose first rows belong to another lane
-    const float *base = lds + pl * p.st.plane_pitch + (row0 * S + HALO) * p.st.pitch + kSlack + 4 * cb * S;
-    const float *base_g = EPI ? lds + p.g_base + pl * p.sg.plane_pitch + row0 * p.sg.pitch + kSlack + 4 * cb : base + p.g_base;
     static_assert(!EPI || GX, "the epilogue's instances make all gradients");
     EpilogueSums sums;
     float e_scale = 1.f, e_shift = 0.f;
@@ -126,6 +122,13 @@ __global__ __launch_bounds__(kThreads) void wgrad_tile_kernel(const WgradPlan p)
         const int n = tile / p.row_tiles, rt = tile - n * p.row_tiles;
         const long plane0 = static_cast<long>(n) * p.channel + c0;
         const int oy0 = rt * p.rows_per_tile;
+        // The first row of this lane's block in the tile, and how many of its first rows belong to another lane.  With the epilogue
+        // the last blocks move up until they end with the band and the plane: a row past the plane would be zero where it meets x,
+        // and zero times an infinite x is NaN in a tap that the plane's rows leave finite.  (Left: bands of fewer than BH rows.)
+        const int row0 = EPI ? max(min(rb * BH, min(p.rows_per_tile, p.out_h - oy0) - BH), 0) : rb * BH;
+        const int skip = EPI ? rb * BH - row0 : 0;
+        const float *base = lds + pl * p.st.plane_pitch + (row0 * S + HALO) * p.st.pitch + kSlack + 4 * cb * S;
+        const float *base_g = EPI ? lds + p.g_base + pl * p.sg.plane_pitch + row0 * p.sg.pitch + kSlack + 4 * cb : base + p.g_base;
 
         // this lane's block of gy (zero where it hangs over the edge of the plane); issued before the
         // x band is staged so that both sets of loads are in flight together
@@ -311,15 +314,11 @@ __global__ __launch_bounds__(kThreads) void wgrad_tile_kernel(const WgradPlan p)
             for (int b = 0; b < BH; ++b) {
                 const int ty = wr - b * S;
                 if (ty < 0 || ty >= K) continue;
-                // (with the epilogue the tiles hang over the plane where the plain kernels' do not: their rows and columns past it
-                // meet no x, so that one that is not finite stays out of the taps it has no part in)
-                if (EPI && !(has_item && b >= skip && oy0 + row0 + b < p.out_h)) continue;
 #pragma unroll
-                for (int o = 0; o < 4; ++o) {
-                    if (EPI && ANY_WIDTH && o > 0 && ox + o >= p.out_w) continue;
+                for (int tx = 0; tx < K; ++tx)
 #pragma unroll
-                    for (int tx = 0; tx < K; ++tx) acc[ty * K + tx] = fmaf(g[b][o], win[o * S + tx], acc[ty * K + tx]);
-                }
+                    for (int o = 0; o < 4; ++o)
+                        acc[ty * K + tx] = fmaf(g[b][o], win[o * S + tx], acc[ty * K + tx]);
             }
             pin_registers(acc);
         }
