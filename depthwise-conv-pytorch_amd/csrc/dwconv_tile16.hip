@@ -1,5 +1,5 @@
-// LDS-tiled forward / stride-1 grad-input kernel for 16-bit tensors (fp16, bf16) whose rows are whole groups of
-// eight elements.
+// LDS-tiled forward / stride-1 grad-input kernel for 16-bit tensors (fp16, bf16): rows that are whole groups of eight
+// elements, and an instance (ANY) for rows of any other width that start on any element.
 //
 // The tiled kernels of dwconv_tile.hip widen every element to fp32 on its way into LDS.  With 16-bit tensors they
 // are bound by the vector unit, not by memory: the same instructions move half the bytes.  This kernel keeps the
@@ -46,7 +46,15 @@ struct Tile16Plan {
 // PW1: parity of the left padding (the first element of a lane's window is the high half of a dword when odd).
 // EPI: the epilogue of the fused forward entry points is compiled in (its temporaries cost 12 registers, a wavefront
 // of occupancy, also when it is switched off at run time).
-template <typename IO, int K, int S, int PW1, bool FLIP, int BH, bool EPI>
+// ANY: rows of any width at any element alignment, on either side.  The fp32-image kernel, which such rows took before, loads
+// four elements at a time (three dwords each where rows start on odd elements), widens them on their way into LDS and takes a
+// multiply-add per tap: at 150x150 C=96 3x3 stride 2 the bytes take 56 us and it took 119.  Here a load brings eight elements
+// (four dwords, or five), nothing is widened, and the results, whose rows start anywhere too, leave through LDS as one run of
+// 16-byte pieces (lds_put_run16, store_run16).  bf16, batch 64, us before / now: 150x150 3x3 C=32 53.4 / 45.8, stride 2 C=96
+// 119 / 90; 75x75 C=144 3x3 71.6 / 51.3, 5x5 stride 2 58.8 / 44.3; 38x38 C=240 3x3 stride 2 26.5 / 20.9; 107x107 C=32 3x3
+// 33.9 / 27.7, stride 2 C=96 77.9 / 55.6.  What is left is the LDS traffic of the results (five writes a row where an aligned
+// one is a single write) and the lines at the ends of a band that two workgroups fetch.
+template <typename IO, int K, int S, int PW1, bool FLIP, int BH, bool EPI, bool ANY>
 __global__ __launch_bounds__(kThreads) void fir_down16_kernel(const Tile16Plan p)
 {
     extern __shared__ float4 lds_raw[];
@@ -77,7 +85,7 @@ __global__ __launch_bounds__(kThreads) void fir_down16_kernel(const Tile16Plan p
         lds32[p.tap_base + i] = j < KP ? (tap(2 * j) | (tap(2 * j + 1) << 16)) : (tap(K - 1) << 16);
     }
 
-    stage_image16(p.im, static_cast<const IO *>(p.in) + plane0 * p.im.in_plane, lds32, p.dump, nplanes, iy0);
+    stage_image16<IO, 4, ANY>(p.im, static_cast<const IO *>(p.in) + plane0 * p.im.in_plane, lds32, p.dump, nplanes, iy0);
     __syncthreads();
 
     const int n_items = nplanes * p.items_per_plane;
@@ -160,7 +168,7 @@ __global__ __launch_bounds__(kThreads) void fir_down16_kernel(const Tile16Plan p
         }
     };
 
-    if (p.lout) {
+    if (ANY || p.lout) {
         // One item per lane (the planner guarantees it).  The packed sums go back into LDS in the layout the band has
         // in memory, over the image, and leave as one linear stream per plane: 16 bytes per lane, 1 KiB of
         // consecutive bytes per wavefront and store.  Lane-owned blocks write a row segment at a time; where a row is
@@ -188,6 +196,21 @@ __global__ __launch_bounds__(kThreads) void fir_down16_kernel(const Tile16Plan p
             for (int b = 0; b < BH; ++b) pack_row(acc[b], packed[b]);
         }
         __syncthreads();  // every window has been read: the image can be overwritten
+        if constexpr (ANY) {
+            // (a tile of several planes holds whole ones: its results are one run too)
+            IO *to = static_cast<IO *>(p.out) + plane0 * p.out_plane + static_cast<long>(oy0) * p.out_w;
+            const int head = run_head(to);
+            uint16_t *image = reinterpret_cast<uint16_t *>(lds_raw);
+            if (has_item) {
+#pragma unroll
+                for (int b = 0; b < BH; ++b)
+                    if (rb * BH + b < rows_here)
+                        lds_put_run16(image, head + __mul24(pl, p.out_plane) + __mul24(rb * BH + b, p.out_w) + cb * OWI, p.out_w - cb * OWI, packed[b]);
+            }
+            __syncthreads();
+            store_run16(to, image, head, (nplanes - 1) * p.out_plane + run);
+            return;
+        }
         if (has_item) {
 #pragma unroll
             for (int b = 0; b < BH; ++b) {
@@ -217,7 +240,7 @@ __global__ __launch_bounds__(kThreads) void fir_down16_kernel(const Tile16Plan p
         return;
     }
 
-    for (int item = threadIdx.x; item < n_items; item += blockDim.x) {
+    if constexpr (!ANY) for (int item = threadIdx.x; item < n_items; item += blockDim.x) {
         const int pl = fast_div(item, p.ipp_magic);
         const int rem = item - __mul24(pl, p.items_per_plane);
         const int rb = fast_div(rem, p.ncb_magic);
@@ -245,7 +268,7 @@ __global__ __launch_bounds__(kThreads) void fir_down16_kernel(const Tile16Plan p
     }
 }
 
-template <typename IO, int K, int S, int PW1, bool FLIP, int BH>
+template <typename IO, int K, int S, int PW1, bool FLIP, int BH, bool ANY>
 int launch_down16(Tile16Plan &p, hipStream_t stream)
 {
     constexpr int OWI = S == 1 ? 8 : 4;
@@ -253,11 +276,12 @@ int launch_down16(Tile16Plan &p, hipStream_t stream)
     constexpr int TPP = K * (KP + 1);
     const int threads = kThreads;
     const int target_items = env_int("DWCONV_TILE16_ITEMS", threads);
-    const int budget = env_int("DWCONV_TILE16_LDS", S == 2 ? 32 * 1024 : 24 * 1024);
+    // (ANY, stride 2: 150x150 C=96 3x3 98 us with 32 KiB, 91 with 40, 88 with 48, but 75x75 C=144 5x5 46, 46 and 54)
+    const int budget = env_int("DWCONV_TILE16_LDS", S == 2 ? (ANY ? 40 : 32) * 1024 : 24 * 1024);
 
-    p.ncb = p.out_w / OWI;
-    // elements of a row the windows touch: up to input column (out_w - 1) * S - pad_w + K - 1, and its pair partner
-    const int last_col = (p.out_w - 1) * S - p.pad_w + K;
+    p.ncb = ceil_div(p.out_w, OWI);
+    // elements of a row the windows touch: up to input column (ncb * OWI - 1) * S - pad_w + K - 1, and its pair partner
+    const int last_col = (p.ncb * OWI - 1) * S - p.pad_w + K;
     layout_image16(p.im, last_col);
     auto rows_for = [](int units) { return (units * BH - 1) * S + K; };
     auto bytes = [&](int units, int planes) {
@@ -297,24 +321,32 @@ int launch_down16(Tile16Plan &p, hipStream_t stream)
     p.n_tiles = static_cast<int>(tiles);
     p.lout = env_int("DWCONV_T16_LOUT", 1) && planes_per_tile * p.items_per_plane <= threads &&
              (p.rows_per_tile * p.out_w) % 8 == 0 && p.out_plane % 8 == 0;
-    const size_t lds = static_cast<size_t>(p.tap_base) * 4 + static_cast<size_t>(planes_per_tile) * TPP * 4;
+    size_t lds = static_cast<size_t>(p.tap_base) * 4 + static_cast<size_t>(planes_per_tile) * TPP * 4;
+    if (ANY) {
+        if (planes_per_tile * p.items_per_plane > threads) return -1;
+        // the run of results takes the place of the image (and of the taps): seven elements in front, whole 16-byte pieces
+        const size_t run = (static_cast<size_t>(planes_per_tile - 1) * p.out_plane + static_cast<size_t>(p.rows_per_tile) * p.out_w + 7 + 8) * 2;
+        lds = std::max(lds, run);
+        if (planes_per_tile > 1 && p.row_tiles != 1) return -1;
+    }
 
     if (!FLIP && p.epi.enabled())
-        hipLaunchKernelGGL((fir_down16_kernel<IO, K, S, PW1, FLIP, BH, !FLIP>), dim3(p.n_tiles), dim3(threads), lds, stream, p);
+        hipLaunchKernelGGL((fir_down16_kernel<IO, K, S, PW1, FLIP, BH, !FLIP, ANY>), dim3(p.n_tiles), dim3(threads), lds, stream, p);
     else
-        hipLaunchKernelGGL((fir_down16_kernel<IO, K, S, PW1, FLIP, BH, false>), dim3(p.n_tiles), dim3(threads), lds, stream, p);
+        hipLaunchKernelGGL((fir_down16_kernel<IO, K, S, PW1, FLIP, BH, false, ANY>), dim3(p.n_tiles), dim3(threads), lds, stream, p);
     note_variant("tile_down16_dot2<k%d,s%d,%s,bh%d> P%d rows%d%s", K, S, FLIP ? "rot" : "fwd", BH, p.planes_per_tile, p.rows_per_tile,
-                 p.lout ? " ldsout" : "");
+                 ANY ? " runout anywidth" : p.lout ? " ldsout" : "");
     return check_launch("fir_down16_kernel");
 }
 
 template <typename IO, int K, int S, bool FLIP>
-int launch_down16_parity(Tile16Plan &p, hipStream_t stream)
+int launch_down16_parity(Tile16Plan &p, bool any, hipStream_t stream)
 {
     const int forced = env_int("DWCONV_TILE_BH", 0);
     const bool seven = forced ? forced == 7 : (p.out_h % 7 == 0 || p.out_h > 64) && p.out_h % 4 != 0;
     constexpr int PW1 = (K / 2) & 1;  // the left padding is K / 2
-    return seven ? launch_down16<IO, K, S, PW1, FLIP, 7>(p, stream) : launch_down16<IO, K, S, PW1, FLIP, 4>(p, stream);
+    if (any) return launch_down16<IO, K, S, PW1, FLIP, 4, true>(p, stream);
+    return seven ? launch_down16<IO, K, S, PW1, FLIP, 7, false>(p, stream) : launch_down16<IO, K, S, PW1, FLIP, 4, false>(p, stream);
 }
 
 }  // namespace
@@ -331,13 +363,27 @@ int try_launch_fir_tiled16(const IO *in, const IO *taps, IO *out, const Geometry
     if (S == 2 && !g.forward) return -1;
     // (the window's place within its LDS slots is a compile-time constant: left padding K/2 only)
     if (g.pad_h0 < 0 || g.pad_h0 > 7 || g.pad_w0 != K / 2) return -1;
-    if (g.in_w % 8 != 0 || g.out_w % (S == 1 ? 8 : 4) != 0 || g.in_h < 1) return -1;
+    if (g.in_h < 1 || g.out_w < 1) return -1;
+    // whole groups of eight that start on 16-byte boundaries, or rows of any width at any element alignment
+    const bool any = g.in_w % 8 != 0 || g.out_w % (S == 1 ? 8 : 4) != 0 || reinterpret_cast<uintptr_t>(in) % 16 != 0 ||
+                     reinterpret_cast<uintptr_t>(out) % 16 != 0;
     // Input rows of at least 48 elements at stride 2 and 72 at stride 1: measured against the fp32-image and stacked
     // kernels on 48 ... 88 wide maps (batch 64, C = 144, bf16 and fp16), stride 2 is 3-29 % faster here at every
     // width, stride 1 6-19 % from 72 on (88 x 88 5x5: equal) and mixed below (56 x 56 3x3 and 7x7: 8-12 % slower;
     // narrower planes have too few 8-wide blocks to occupy the lanes).
-    if (g.in_w < env_int("DWCONV_T16_MIN_W", S == 2 ? 48 : 72)) return -1;
-    if (reinterpret_cast<uintptr_t>(in) % 16 != 0 || reinterpret_cast<uintptr_t>(out) % 16 != 0) return -1;
+    // Rows of any width, measured against the fp32-image kernel on 26 widths from 33 to 257 (batch 16, bf16 and fp16): stride 2
+    // is 2-38 % faster here at every width.  At stride 1 rows of an odd width are 2-25 % faster with 3x3 and 5x5 filters from 65
+    // columns on (below, 33 to 57: between 20 % faster and 8 % slower), even ones that are no multiple of four 5-13 % from 128 on
+    // (below: 7 % faster to 16 % slower, as the lanes fill), and multiples of four, which that kernel loads aligned, are up to
+    // 25 % slower (92: 14.2 us there, 18.0 here).  With 7x7 filters every width from 56 on that is no multiple of four is 6-37 %
+    // faster.
+    if (any) {
+        const bool odd = (g.in_w & 1) != 0, four = g.in_w % 4 == 0;
+        const int least = S == 2 ? 33 : four ? 1 << 30 : K == 7 ? 56 : odd ? 65 : 128;
+        if (g.in_w < env_int("DWCONV_T16_ANY_MIN_W", least)) return -1;
+    } else if (g.in_w < env_int("DWCONV_T16_MIN_W", S == 2 ? 48 : 72)) {
+        return -1;
+    }
     if (static_cast<long>(g.in_h) * g.in_w >= (1l << 30) || static_cast<long>(g.out_h) * g.out_w >= (1l << 30)) return -1;
 
     Tile16Plan p{};
@@ -357,13 +403,13 @@ int try_launch_fir_tiled16(const IO *in, const IO *taps, IO *out, const Geometry
     p.pad_w = g.pad_w0;
     const bool rot = !g.forward;
     if (S == 1) {
-        if (K == 3) return rot ? launch_down16_parity<IO, 3, 1, true>(p, stream) : launch_down16_parity<IO, 3, 1, false>(p, stream);
-        if (K == 5) return rot ? launch_down16_parity<IO, 5, 1, true>(p, stream) : launch_down16_parity<IO, 5, 1, false>(p, stream);
-        return rot ? launch_down16_parity<IO, 7, 1, true>(p, stream) : launch_down16_parity<IO, 7, 1, false>(p, stream);
+        if (K == 3) return rot ? launch_down16_parity<IO, 3, 1, true>(p, any, stream) : launch_down16_parity<IO, 3, 1, false>(p, any, stream);
+        if (K == 5) return rot ? launch_down16_parity<IO, 5, 1, true>(p, any, stream) : launch_down16_parity<IO, 5, 1, false>(p, any, stream);
+        return rot ? launch_down16_parity<IO, 7, 1, true>(p, any, stream) : launch_down16_parity<IO, 7, 1, false>(p, any, stream);
     }
-    if (K == 3) return launch_down16_parity<IO, 3, 2, false>(p, stream);
-    if (K == 5) return launch_down16_parity<IO, 5, 2, false>(p, stream);
-    return launch_down16_parity<IO, 7, 2, false>(p, stream);
+    if (K == 3) return launch_down16_parity<IO, 3, 2, false>(p, any, stream);
+    if (K == 5) return launch_down16_parity<IO, 5, 2, false>(p, any, stream);
+    return launch_down16_parity<IO, 7, 2, false>(p, any, stream);
 }
 
 template int try_launch_fir_tiled16<half_t>(const half_t *, const half_t *, half_t *, const Geometry &, hipStream_t);

@@ -15,7 +15,7 @@ constexpr int kPadL = 8;  // element j of an image row holds input column j - kP
 // four) the same reads use half the banks twice over: the counters showed the LDS busy 60 % of the time, two thirds
 // of it in bank conflicts.
 struct Image16 {
-    int in_h, in_w, in_plane;   // in_w is a multiple of eight
+    int in_h, in_w, in_plane;   // in_w is a multiple of eight, unless the rows are staged with ANY
     int lds_rows;
     unsigned lds_rows_magic;
     int spr;
@@ -66,17 +66,51 @@ __device__ __forceinline__ float dot2(uint32_t a, uint32_t b, float c)
 // slot of every row is written, with zeros (loads beyond the view) outside the plane.  `image` is the first dword,
 // `dump` the index of a spare slot.  A lane keeps its column and walks down the rows: per slot two additions, a range check and a
 // select.  kBatch loads are in flight per lane.
-template <typename IO, int kBatch = 4>
+// ANY: rows of any width that start on any element.  A slot's load starts on a 32-bit boundary: 128 bits at a multiple of 4
+// where every row does; where some start 2 bytes past one, a fifth dword and four funnel shifts when the slot enters LDS.
+// What a row's last slot read of the next row is masked there too (the masks belong to the lane's column).
+template <typename IO, int kBatch = 4, bool ANY = false>
 __device__ __forceinline__ void stage_image16(const Image16 &im, const IO *src, uint32_t *image, int dump, int nplanes, int iy0)
 {
-    const __amdgpu_buffer_rsrc_t view = buffer_view(src, static_cast<long>(nplanes) * im.in_plane * sizeof(IO));
+    const bool split = ANY && mixed_row_starts(src, im.in_w);
+    AnyWidthView wide{};
+    if constexpr (ANY) wide = any_width_view(src, static_cast<long>(nplanes) * im.in_plane * sizeof(IO));
+    else wide.view = buffer_view(src, static_cast<long>(nplanes) * im.in_plane * sizeof(IO));
+    struct Slot {
+        u32x4 v;
+        unsigned more, shift;  // split rows: the dword behind v, and how far the slot starts inside its first dword
+    };
+    auto load = [&](unsigned off) {
+        Slot s;
+        if (ANY && split) {
+            const unsigned at = off < kOob ? off + wide.bias : kOob;
+            s.v = __builtin_amdgcn_raw_buffer_load_b128(wide.view, at & ~3u, 0, 0);
+            s.more = __builtin_amdgcn_raw_buffer_load_b32(wide.view, (at & ~3u) + 16u, 0, 0);
+            s.shift = (at & 2u) << 3;
+        } else {
+            s.v = __builtin_amdgcn_raw_buffer_load_b128(wide.view, off, 0, 0);
+            s.more = s.shift = 0u;
+        }
+        return s;
+    };
     const int nthreads = blockDim.x;
     const int rpp_raw = fast_div(nthreads, im.spr_magic);
     const int rpp = max(rpp_raw, 1);                     // rows per pass of the workgroup
     const int col_step = rpp_raw ? im.spr : nthreads;    // one trip unless a row has more slots than lanes
     const int rl = fast_div(threadIdx.x, im.spr_magic);
     const int spitch = im.pitch >> 3;                    // in slots
-    auto put = [&](int slot, const u32x4 &v) {
+    u32x4 keep = {~0u, ~0u, ~0u, ~0u};  // ANY: the elements of the lane's column that belong to its rows
+    auto put = [&](int slot, const Slot &s) {
+        u32x4 v = s.v;
+        if constexpr (ANY) {
+            if (split) {
+                v.x = __builtin_amdgcn_alignbit(s.v.y, s.v.x, s.shift);
+                v.y = __builtin_amdgcn_alignbit(s.v.z, s.v.y, s.shift);
+                v.z = __builtin_amdgcn_alignbit(s.v.w, s.v.z, s.shift);
+                v.w = __builtin_amdgcn_alignbit(s.more, s.v.w, s.shift);
+            }
+            v &= keep;
+        }
         uint32_t *d = image + slot * 5;
         d[0] = v.x;
         d[1] = v.y;
@@ -87,6 +121,11 @@ __device__ __forceinline__ void stage_image16(const Image16 &im, const IO *src, 
     for (int sc = threadIdx.x - __mul24(rl, im.spr); sc < im.spr; sc += col_step) {
         const int ix = 8 * sc - kPadL;
         const bool col_ok = static_cast<unsigned>(ix) < static_cast<unsigned>(im.in_w);
+        if constexpr (ANY) {
+            const int n = im.in_w - ix;  // elements of the row from this column on
+#pragma unroll
+            for (int d = 0; d < 4; ++d) keep[d] = n > 2 * d + 1 ? ~0u : (n > 2 * d ? 0xffffu : 0u);
+        }
         if (nplanes == 1) {
             const int lo = max(iy0, 0);
             const unsigned span = static_cast<unsigned>(max(min(im.in_h, iy0 + im.lds_rows) - lo, 0));
@@ -100,11 +139,11 @@ __device__ __forceinline__ void stage_image16(const Image16 &im, const IO *src, 
             // the spare slot.  A store under a per-lane condition would drag its load into the conditional block,
             // behind the other loads' wait.
             for (; rb + rpp * kBatch <= im.lds_rows; rb += rpp * kBatch) {
-                u32x4 v[kBatch];
+                Slot v[kBatch];
 #pragma unroll
                 for (int u = 0; u < kBatch; ++u) {
                     const bool ok = col_ok && static_cast<unsigned>(iy + u * rpp - lo) < span;
-                    v[u] = __builtin_amdgcn_raw_buffer_load_b128(view, ok ? off + u * off_step : kOob, 0, 0);
+                    v[u] = load(ok ? off + u * off_step : kOob);
                 }
 #pragma unroll
                 for (int u = 0; u < kBatch; ++u) put(dst + u * dst_step, v[u]);
@@ -113,11 +152,11 @@ __device__ __forceinline__ void stage_image16(const Image16 &im, const IO *src, 
                 dst += dst_step * kBatch;
             }
             if (rb < im.lds_rows) {
-                u32x4 v[kBatch];
+                Slot v[kBatch];
 #pragma unroll
                 for (int u = 0; u < kBatch; ++u) {
                     const bool ok = col_ok && static_cast<unsigned>(iy + u * rpp - lo) < span;
-                    v[u] = __builtin_amdgcn_raw_buffer_load_b128(view, ok ? off + u * off_step : kOob, 0, 0);
+                    v[u] = load(ok ? off + u * off_step : kOob);
                 }
 #pragma unroll
                 for (int u = 0; u < kBatch; ++u) put(rb + rl + u * rpp < im.lds_rows ? dst + u * dst_step : dump, v[u]);
@@ -126,7 +165,7 @@ __device__ __forceinline__ void stage_image16(const Image16 &im, const IO *src, 
             const int total_rows = nplanes * im.lds_rows;
             const int pslots = im.lds_rows * spitch;
             for (int ra = rl; ra < total_rows; ra += rpp * kBatch) {
-                u32x4 v[kBatch];
+                Slot v[kBatch];
                 int dst[kBatch];
 #pragma unroll
                 for (int u = 0; u < kBatch; ++u) {
@@ -137,12 +176,50 @@ __device__ __forceinline__ void stage_image16(const Image16 &im, const IO *src, 
                     const int iy = iy0 + r;
                     const bool ok = live && col_ok && static_cast<unsigned>(iy) < static_cast<unsigned>(im.in_h);
                     const unsigned off = (__mul24(pl, im.in_plane) + __mul24(iy, im.in_w) + ix) * 2u;
-                    v[u] = __builtin_amdgcn_raw_buffer_load_b128(view, ok ? off : kOob, 0, 0);
+                    v[u] = load(ok ? off : kOob);
                     dst[u] = live ? __mul24(pl, pslots) + __mul24(r, spitch) + sc : dump;
                 }
 #pragma unroll
                 for (int u = 0; u < kBatch; ++u) put(dst[u], v[u]);
             }
+        }
+    }
+}
+
+// `n` packed results (n <= 2 NP) into a run of consecutive 16-bit elements in LDS, from element `at` on, which need not be
+// even.  A whole group goes as NP - 1 dwords on 32-bit boundaries and the two elements that are left: the first two where the
+// group starts on such a boundary, the first and the last where it does not.
+template <int NP>
+__device__ __forceinline__ void lds_put_run16(uint16_t *run, int at, int n, const uint32_t (&v)[NP])
+{
+    uint16_t *d = run + at;
+    if (n >= 2 * NP) {
+        const bool odd = (at & 1) != 0;
+        uint32_t *mid = reinterpret_cast<uint32_t *>(d + (odd ? 1 : 2));
+#pragma unroll
+        for (int i = 0; i + 1 < NP; ++i) mid[i] = odd ? __builtin_amdgcn_alignbit(v[i + 1], v[i], 16) : v[i + 1];
+        d[0] = static_cast<uint16_t>(v[0]);
+        d[odd ? 2 * NP - 1 : 1] = static_cast<uint16_t>((odd ? v[NP - 1] : v[0]) >> 16);
+    } else {
+#pragma unroll
+        for (int e = 0; e < 2 * NP - 1; ++e)
+            if (e < n) d[e] = static_cast<uint16_t>(v[e / 2] >> (16 * (e & 1)));
+    }
+}
+// A run of 16-bit results that starts on any element: lds[head .. head + n) leaves for to[0 .. n), `head` being the elements
+// between the 16-byte boundary before `to` and `to` (run_head).  Whole 16-byte pieces leave as such, the two ends element by
+// element.  The workgroup calls it together, after a barrier behind the writes into LDS.
+template <typename IO>
+__device__ __forceinline__ void store_run16(IO *to, const uint16_t *lds, int head, int n)
+{
+    uint16_t *const base = reinterpret_cast<uint16_t *>(to) - head;
+    const int end = head + n;
+    const __amdgpu_buffer_rsrc_t view = buffer_view(base, static_cast<long>(end) * 2);
+    for (int c = threadIdx.x * 8; c < end; c += blockDim.x * 8) {
+        if (c >= head && c + 8 <= end) {
+            __builtin_amdgcn_raw_buffer_store_b128(*reinterpret_cast<const u32x4 *>(lds + c), view, c * 2u, 0, kStoreStreaming);
+        } else {
+            for (int e = max(c, head); e < min(c + 8, end); ++e) base[e] = lds[e];
         }
     }
 }
