@@ -13,7 +13,7 @@
 //     adds the chunks in a fixed order: bit-identical from run to run, no atomics.
 // Geometries outside the fast kernels (C not a multiple of 4, filters other than 3/5/7, fp64) take the
 // one-lane-per-element kernels at the end of the file.
-#include "dwconv_tile_common.hpp"
+#include "dwconv_tile16_common.hpp"
 
 #include <algorithm>
 #include <type_traits>
@@ -155,6 +155,114 @@ __device__ __forceinline__ void nhwc_taps(const float *wl, float (&w)[CV])
     }
 }
 
+// ---- 16-bit elements: two products per instruction ------------------------------------------------------------
+// Two taps (grad-weight: two pixels) at a time: a two-element dot product (v_dot2, at the rate of a multiply-add; both products
+// exact, one fp32 sum, subnormals kept) of two pixels of one channel and two taps.  A pixel holds its channels side by side, so a
+// pair of pixels of one channel is one byte permutation of the two dwords, taken from a row as loaded: it stands where the
+// widening stood.  A tap without a partner (the filters are odd) stays a multiply-add of the widened element: a partner with a
+// zero tap would turn an infinity next to the window into NaN.
+template <typename IO>
+constexpr bool kPairs = sizeof(IO) == 2;
+
+// pair[CV * j + q]: channel q of pixels j (low half) and j + D.
+template <int D, typename IO, int COLS, int CV>
+__device__ __forceinline__ void nhwc_pair_row(const RawPixel<IO, CV> (&raw)[COLS], uint32_t (&pair)[COLS * CV])
+{
+    if constexpr (kPairs<IO>) {
+#pragma unroll
+        for (int j = 0; j + D < COLS; ++j)
+#pragma unroll
+            for (int q = 0; q < CV; ++q)
+                pair[CV * j + q] = __builtin_amdgcn_perm(raw[j + D].w[q / 2], raw[j].w[q / 2], q & 1 ? 0x07060302u : 0x05040100u);
+    }
+}
+
+// The taps of a filter row as K / 2 pairs (2 j with 2 j + 1) and a single one (fp32 bits): [ty][PER_ROW][channel] dwords in LDS.
+template <int K>
+struct TapPairs {
+    static constexpr int N = K / 2, PER_ROW = N + 1, TOTAL = K * PER_ROW;
+};
+template <typename IO, int K, bool FLIP>
+__device__ __forceinline__ void nhwc_stage_tap_pairs(const IO *__restrict__ taps, uint32_t *lds, int c0, int nch)
+{
+    using P = TapPairs<K>;
+    constexpr int kTapBatch = 4;  // (two loads each: see nhwc_stage_taps)
+    const uint16_t *src = reinterpret_cast<const uint16_t *>(taps) + static_cast<long>(c0) * (K * K);
+    const int total = nch * P::TOTAL;
+    for (int i0 = threadIdx.x; i0 < total; i0 += kTapBatch * kNhwcThreads) {
+        uint16_t first[kTapBatch], second[kTapBatch];
+#pragma unroll
+        for (int k = 0; k < kTapBatch; ++k) {
+            const int i = min(i0 + k * kNhwcThreads, total - 1), cl = i / P::TOTAL, e = i - cl * P::TOTAL;
+            const int ty = e / P::PER_ROW, j = e - ty * P::PER_ROW;
+            const int a = 2 * j, b = min(a + 1, K - 1);
+            const int row = cl * (K * K) + (FLIP ? K - 1 - ty : ty) * K;
+            first[k] = src[row + (FLIP ? K - 1 - a : a)];
+            second[k] = src[row + (FLIP ? K - 1 - b : b)];
+        }
+#pragma unroll
+        for (int k = 0; k < kTapBatch; ++k) {
+            const int i = i0 + k * kNhwcThreads, cl = i / P::TOTAL, e = i - cl * P::TOTAL;
+            const uint32_t pair = first[k] | (static_cast<uint32_t>(second[k]) << 16);
+            const uint32_t single = __float_as_uint(Io<IO>::in(__builtin_bit_cast(IO, first[k])));
+            if (i < total) lds[e * nch + cl] = e % P::PER_ROW == P::N ? single : pair;
+        }
+    }
+}
+// The taps of filter row ty for a lane's channels (`wl`: the table at its first channel).
+template <int K, int CV>
+__device__ __forceinline__ void nhwc_tap_row(const uint32_t *wl, int ty, int nch, uint32_t (&w)[TapPairs<K>::PER_ROW][CV])
+{
+#pragma unroll
+    for (int j = 0; j < TapPairs<K>::PER_ROW; ++j) {
+        const uint32_t *at = wl + (ty * TapPairs<K>::PER_ROW + j) * nch;
+        if constexpr (CV == 2) {
+            const uint2 t = *reinterpret_cast<const uint2 *>(at);
+            w[j][0] = t.x, w[j][1] = t.y;
+        } else {
+#pragma unroll
+            for (int q = 0; q < CV; ++q) w[j][q] = at[q];
+        }
+    }
+}
+// The same from a filter row of the [tap][channel] table in fp32 (nhwc_stage_taps), which is quicker to fill.  The taps are 16-bit values, so packing them is exact.
+template <typename IO, int K, int CV>
+__device__ __forceinline__ void nhwc_pack_tap_row(const float *wl, int nch, uint32_t (&w)[TapPairs<K>::PER_ROW][CV])
+{
+    static_assert(CV == 2, "two channels per lane");
+#pragma unroll
+    for (int j = 0; j < K / 2; ++j) {
+        float a[CV], b[CV];
+        nhwc_taps<CV>(wl + 2 * j * nch, a);
+        nhwc_taps<CV>(wl + (2 * j + 1) * nch, b);
+#pragma unroll
+        for (int q = 0; q < CV; ++q) {
+            if constexpr (std::is_same<IO, bf16_t>::value) w[j][q] = bf16_pack2(a[q], b[q]);
+            else w[j][q] = f16_pack2(a[q], b[q]);
+        }
+    }
+    float last[CV];
+    nhwc_taps<CV>(wl + (K - 1) * nch, last);
+#pragma unroll
+    for (int q = 0; q < CV; ++q) w[K / 2][q] = __float_as_uint(last[q]);
+}
+// One filter row into TW sums: sum[o] += pixels o * S ... o * S + K - 1 of the window row times the taps.
+template <typename IO, int K, int S, int TW, int CV, int COLS>
+__device__ __forceinline__ void nhwc_pairs_row(const uint32_t (&pair)[COLS * CV], const float (&cur)[COLS * CV],
+                                               const uint32_t (&w)[TapPairs<K>::PER_ROW][CV], float (&sum)[TW * CV])
+{
+#pragma unroll
+    for (int j = 0; j < K / 2; ++j)
+#pragma unroll
+        for (int o = 0; o < TW; ++o)
+#pragma unroll
+            for (int q = 0; q < CV; ++q) sum[CV * o + q] = dot2<IO>(pair[CV * (o * S + 2 * j) + q], w[j][q], sum[CV * o + q]);
+#pragma unroll
+    for (int o = 0; o < TW; ++o)
+#pragma unroll
+        for (int q = 0; q < CV; ++q)
+            sum[CV * o + q] = fmaf(cur[CV * (o * S + K - 1) + q], __uint_as_float(w[K / 2][q]), sum[CV * o + q]);
+}
 // CV results of a pixel at byte offset `off` of the view (dropped when that is at or beyond kOob).
 template <typename IO, int CV>
 __device__ __forceinline__ void store_pixel(__amdgpu_buffer_rsrc_t view, unsigned off, const float *v)
@@ -212,7 +320,14 @@ __global__ __launch_bounds__(kNhwcThreads) void nhwc_down_kernel(const NhwcPlan 
     const int pg = wg / p.cgroups;
     const int c0 = (wg - pg * p.cgroups) * p.lanes_c * CV;
     const int nch = min(p.lanes_c * CV, C - c0);
-    nhwc_stage_taps<IO, KK, FLIP>(static_cast<const IO *>(p.taps), lds, c0, nch);
+    // 16 bits: two taps at a time in the tall blocks of 5x5 filters and with 7x7 ones (us, multiply-adds / pairs: bf16 batch 64, 7x7 56x56 C=96
+    // 42.7 / 37.7, 7x7 C=768 12.2 / 11.0; batch 128, 5x5 28x28 C=240 29.0 / 27.9; fp16 batch 32, 5x5 13x13 C=672 10.3 / 8.9);
+    // 4 x 4 blocks lose with them (bf16 batch 64, 5x5 16x16 C=672 14.1 / 15.4), 3x3 filters wait for memory either way.  Up to 5x5 the taps of two channels stay in
+    // registers.
+    constexpr bool PAIRS = kPairs<IO> && (K == 7 || (K == 5 && BH == 7));
+    constexpr bool TAP_REGS = sizeof(IO) == 2 && K <= 5;
+    if constexpr (PAIRS && !TAP_REGS) nhwc_stage_tap_pairs<IO, K, FLIP>(static_cast<const IO *>(p.taps), reinterpret_cast<uint32_t *>(lds), c0, nch);
+    else nhwc_stage_taps<IO, KK, FLIP>(static_cast<const IO *>(p.taps), lds, c0, nch);
     __syncthreads();
 
     const int pb_local = fast_div(threadIdx.x, p.lanes_c_magic);
@@ -245,10 +360,12 @@ __global__ __launch_bounds__(kNhwcThreads) void nhwc_down_kernel(const NhwcPlan 
     // Rows are loaded AHEAD rows before their use (a ring of row buffers, as loaded) and the sums pinned after every
     // row: otherwise the compiler hoists the loads of the whole window to the top and keeps all of it widened.
     constexpr int RING = AHEAD + 1;
-    // (16 bits, up to 5x5: the taps of two channels stay in registers)
-    constexpr bool TAP_REGS = sizeof(IO) == 2 && KK * CV <= 50;
-    float taps[TAP_REGS ? KK : 1][CV];
-    if constexpr (TAP_REGS) {
+    uint32_t tap_pairs[PAIRS && TAP_REGS ? K : 1][TapPairs<K>::PER_ROW][CV];
+    float taps[TAP_REGS && !PAIRS ? KK : 1][CV];
+    if constexpr (PAIRS && TAP_REGS) {
+#pragma unroll
+        for (int ty = 0; ty < K; ++ty) nhwc_pack_tap_row<IO, K, CV>(wl + ty * K * nch, nch, tap_pairs[ty]);
+    } else if constexpr (TAP_REGS) {
 #pragma unroll
         for (int t = 0; t < KK; ++t) nhwc_taps<CV>(wl + t * nch, taps[t]);
     }
@@ -263,10 +380,17 @@ __global__ __launch_bounds__(kNhwcThreads) void nhwc_down_kernel(const NhwcPlan 
         issue_loads<IO>();
         float cur[COLS * CV];
         nhwc_widen_row<IO, COLS, CV>(raw[r % RING], cur);
+        uint32_t pair[COLS * CV];
+        nhwc_pair_row<1, IO, COLS, CV>(raw[r % RING], pair);
 #pragma unroll
         for (int b = 0; b < BH; ++b) {
             const int ty = r - b * S;
             if (ty < 0 || ty >= K) continue;
+            if constexpr (PAIRS) {
+                if constexpr (!TAP_REGS) nhwc_tap_row<K, CV>(reinterpret_cast<const uint32_t *>(wl), ty, nch, tap_pairs[0]);
+                nhwc_pairs_row<IO, K, S, TW, CV, COLS>(pair, cur, tap_pairs[TAP_REGS ? ty : 0], acc[b]);
+                continue;
+            }
 #pragma unroll
             for (int tx = 0; tx < K; ++tx) {
                 float w[CV];
@@ -529,8 +653,9 @@ __global__ __launch_bounds__(kNhwcThreads) void nhwc_wgrad_kernel(const NhwcPlan
 // as soon as its last window row has passed) and its centre pixels are kept for the K rows of x they meet in the
 // grad-weight sums.  The loop is unrolled, so only the rows in use are live.  out_grad is read once instead of
 // twice and the separate grad-input kernel goes away.  The end of the kernel is that of nhwc_wgrad_kernel.
-template <typename IO, int K, int CV, int BH, int TW>
-__global__ __launch_bounds__(kNhwcThreads) void nhwc_bwd_fused_kernel(const NhwcPlan p)
+// AHEAD: window rows in flight; WAVES: wavefronts per SIMD asked for.
+template <typename IO, int K, int CV, int BH, int TW, int AHEAD, int WAVES>
+__global__ __launch_bounds__(kNhwcThreads, WAVES) void nhwc_bwd_fused_kernel(const NhwcPlan p)
 {
     extern __shared__ float4 lds_raw[];
     float *lds = reinterpret_cast<float *>(lds_raw);
@@ -547,7 +672,8 @@ __global__ __launch_bounds__(kNhwcThreads) void nhwc_bwd_fused_kernel(const Nhwc
     const bool lane_ok = pb_local < p.blocks_per_wg && CV * lane_c < nch;
     const int c = c0 + (lane_ok ? CV * lane_c : 0);
     const int per_image = p.blocks_x * p.blocks_y;
-    nhwc_stage_taps<IO, KK, true>(static_cast<const IO *>(p.taps), lds, c0, nch);
+    if constexpr (kPairs<IO>) nhwc_stage_tap_pairs<IO, K, true>(static_cast<const IO *>(p.taps), reinterpret_cast<uint32_t *>(lds), c0, nch);
+    else nhwc_stage_taps<IO, KK, true>(static_cast<const IO *>(p.taps), lds, c0, nch);
     __syncthreads();
     const float *wl = lds + (lane_ok ? CV * lane_c : 0);
 
@@ -581,11 +707,12 @@ __global__ __launch_bounds__(kNhwcThreads) void nhwc_bwd_fused_kernel(const Nhwc
 
         float gxs[BH][TW * CV];  // in_grad sums
         float gb[BH][TW * CV];   // centre pixels of the out_grad rows (the block itself)
+        uint32_t gbpair[BH][TW * CV];  // (16 bits: the even ones' pairs)
 #pragma unroll
         for (int b = 0; b < BH; ++b)
 #pragma unroll
             for (int o = 0; o < TW * CV; ++o) gxs[b][o] = 0.f;
-        constexpr int AHEAD = 1, RING = AHEAD + 1;
+        constexpr int RING = AHEAD + 1;
         RawPixel<IO, CV> xr[RING][COLS], gr[RING][COLS];
 #pragma unroll
         for (int t = 0; t < AHEAD; ++t) {
@@ -602,11 +729,19 @@ __global__ __launch_bounds__(kNhwcThreads) void nhwc_bwd_fused_kernel(const Nhwc
             if (t < ROWS) {
                 float gcur[COLS * CV];
                 nhwc_widen_row<IO, COLS, CV>(gr[t % RING], gcur);
+                uint32_t gpair[COLS * CV];
+                nhwc_pair_row<1, IO, COLS, CV>(gr[t % RING], gpair);
                 // in_grad row b meets this row in rotated tap row u = t - b
 #pragma unroll
                 for (int u = 0; u < K; ++u) {
                     const int b = t - u;
                     if (b < 0 || b >= BH) continue;
+                    if constexpr (kPairs<IO>) {
+                        uint32_t w[TapPairs<K>::PER_ROW][CV];
+                        nhwc_tap_row<K, CV>(reinterpret_cast<const uint32_t *>(wl), u, nch, w);
+                        nhwc_pairs_row<IO, K, 1, TW, CV, COLS>(gpair, gcur, w, gxs[b]);
+                        continue;
+                    }
 #pragma unroll
                     for (int v = 0; v < K; ++v) {
                         float w[CV];
@@ -620,7 +755,10 @@ __global__ __launch_bounds__(kNhwcThreads) void nhwc_bwd_fused_kernel(const Nhwc
                 }
                 if (t - P >= 0 && t - P < BH) {
 #pragma unroll
-                    for (int o = 0; o < TW * CV; ++o) gb[t - P][o] = gcur[CV * P + o];
+                    for (int o = 0; o < TW * CV; ++o) {
+                        gb[t - P][o] = gcur[CV * P + o];
+                        if constexpr (kPairs<IO>) gbpair[t - P][o] = o / CV + 1 < TW ? gpair[CV * P + o] : 0u;
+                    }
                 }
                 if (t - (K - 1) >= 0 && t - (K - 1) < BH) {
                     const int b = t - (K - 1);
@@ -634,11 +772,24 @@ __global__ __launch_bounds__(kNhwcThreads) void nhwc_bwd_fused_kernel(const Nhwc
             if (r >= 0 && r < ROWS) {
                 float xcur[COLS * CV];
                 nhwc_widen_row<IO, COLS, CV>(xr[r % RING], xcur);
+                uint32_t xpair[COLS * CV];
+                nhwc_pair_row<1, IO, COLS, CV>(xr[r % RING], xpair);
                 // window row r of x meets out_grad row b in tap row ty = r - b
 #pragma unroll
                 for (int ty = 0; ty < K; ++ty) {
                     const int b = r - ty;
                     if (b < 0 || b >= BH) continue;
+                    if constexpr (kPairs<IO>) {
+                        static_assert(TW % 2 == 0, "pixels of out_grad go in pairs");
+#pragma unroll
+                        for (int tx = 0; tx < K; ++tx)
+#pragma unroll
+                            for (int o = 0; o < TW; o += 2)
+#pragma unroll
+                                for (int q = 0; q < CV; ++q)
+                                    acc[ty * K + tx][q] = dot2<IO>(gbpair[b][CV * o + q], xpair[CV * (o + tx) + q], acc[ty * K + tx][q]);
+                        continue;
+                    }
 #pragma unroll
                     for (int tx = 0; tx < K; ++tx)
 #pragma unroll
@@ -1249,9 +1400,10 @@ long nhwc_wgrad_fast(int mode, const IO *x, const IO *gy, IO *gw, void *ws, size
     return -1;
 }
 
-// Fused backward of K x K stride-1 layers with pad K/2: CV channels per lane, BH x TW results per lane.
+// Fused backward of K x K stride-1 layers with pad K/2: CV channels per lane, BH x TW results per lane; AHEAD and WAVES: see the
+// kernel.
 // mode 0: workspace bytes; mode 1: launch.  -1 when the kernel does not cover g.
-template <typename IO, int K, int CV = 2, int BH = 7, int TW = 4>
+template <typename IO, int K, int CV = 2, int BH = 7, int TW = 4, int AHEAD = 1, int WAVES = 1>
 long nhwc_bwd_fused_case(int mode, const IO *x, const IO *gy, const IO *taps, IO *gx, IO *gw, void *ws, size_t ws_bytes,
                          const NhwcGeometry &g, hipStream_t stream)
 {
@@ -1266,7 +1418,8 @@ long nhwc_bwd_fused_case(int mode, const IO *x, const IO *gy, const IO *taps, IO
     // 49.0, 28x28 C=240 91.9 -> 90.1); the 3x3 kernels wait for memory and lose 3-20 % with more than two.
     // The two-channel 3x3 instance (168 registers, three workgroups per unit; what 16-bit tensors run) takes 768 as well:
     // bf16 7x7 C=1152 23.7 -> 18.6 us, 56x56 C=144 94.2 -> 90.6, 112x112 C=32 72.6 -> 70.3, 14x14 C=480 30.0 -> 31.4.
-    long groups = env_int("DWCONV_NHWC_WGRAD_WGS", K == 5 || CV == 2 ? 768 : 512) / cgroups;
+    // The 7x7 instance (246 registers) holds two per unit: 512.
+    long groups = env_int("DWCONV_NHWC_WGRAD_WGS", K == 5 || (K == 3 && CV == 2) ? 768 : 512) / cgroups;
     groups = std::max(1l, std::min(groups, wg_iters));
     p.groups = static_cast<int>(groups);
     p.xcd_chunks = env_int("DWCONV_NHWC_XCD_CHUNKS", 0);
@@ -1286,7 +1439,7 @@ long nhwc_bwd_fused_case(int mode, const IO *x, const IO *gy, const IO *taps, IO
     p.pad_h = g.pad_h;
     p.pad_w = g.pad_w;
     const size_t shmem = static_cast<size_t>(p.lanes_c) * CV * 4 * std::max(K * K, p.blocks_per_wg * K);
-    hipLaunchKernelGGL((nhwc_bwd_fused_kernel<IO, K, CV, BH, TW>), dim3(p.groups * cgroups), dim3(kNhwcThreads), shmem, stream, p);
+    hipLaunchKernelGGL((nhwc_bwd_fused_kernel<IO, K, CV, BH, TW, AHEAD, WAVES>), dim3(p.groups * cgroups), dim3(kNhwcThreads), shmem, stream, p);
     int rc = check_launch("nhwc_bwd_fused_kernel");
     if (rc != DWCONV_OK) return rc;
     note_variant("nhwc_bwd%s<k%d,s1,cv%d,%dx%d> lanes_c%d chunks%d", sizeof(IO) == 2 ? "16" : "", K, CV, BH, TW, p.lanes_c, p.groups);
@@ -1353,12 +1506,12 @@ bool nhwc_fused_s2_ok(const NhwcGeometry &g)
            g.in_w % 2 == 0 && g.out_h == g.in_h / 2 && g.out_w == g.in_w / 2;
 }
 
-bool nhwc_fused_ok(const NhwcGeometry &g)
+bool nhwc_fused_ok(const NhwcGeometry &g, bool half)
 {
     if (!env_int("DWCONV_NHWC_FUSED_BWD", 1) || !nhwc_fast_ok(g)) return false;
     const int K = g.kernel_h;
-    return (K == 3 || K == 5) && g.stride_h == 1 && g.pad_h == K / 2 && g.pad_w == K / 2 && g.out_h == g.in_h &&
-           g.out_w == g.in_w;
+    return (K == 3 || K == 5 || (half && K == 7)) && g.stride_h == 1 && g.pad_h == K / 2 && g.pad_w == K / 2 &&
+           g.out_h == g.in_h && g.out_w == g.in_w;
 }
 
 template <typename IO>
@@ -1382,7 +1535,16 @@ long nhwc_bwd_fused(int mode, const IO *x, const IO *gy, const IO *taps, IO *gx,
         }
         return -1;
     }
-    if (!nhwc_fused_ok(g)) return -1;
+    if (!nhwc_fused_ok(g, sizeof(IO) == 2)) return -1;
+    if (g.kernel_h == 7) {
+        // 16 bits, 7x7: 49 sums for each of two channels and 4 x 4 blocks in 246 registers.  bf16, batch 64, us with the two separate
+        // kernels (both on pairs too) / here: 56x56 C=96 101 / 94.5, 28x28 C=192 55 / 51, 14x14 C=384 39.3 / 39.3, 7x7 C=768 33 / 28;
+        // blocks of 7 x 2: 107, 58, 38, 28; 4 x 2: 115, 64, 44, 36; 2 x 4: 110, 59, 42, 35.  Batch 1: 28.7 / 23.3, 22.3 / 18.8, 19.9 / 18.1,
+        // 20.2 / 18.7 (37632 elements).  Calls of less than 2^15 elements, one or two workgroups, stay on the separate kernels.
+        if constexpr (sizeof(IO) == 2) if (static_cast<long>(g.batch) * g.in_h * g.in_w * g.channel >= 1l << 15)
+            return nhwc_bwd_fused_case<IO, 7, 2, 4, 4, 1, 2>(mode, x, gy, taps, gx, gw, ws, ws_bytes, g, stream);
+        return -1;
+    }
     if (g.kernel_h == 5) {
         // 25 sums per channel.  fp32: with two channels per lane the kernel needs 228 registers (7 x 2 blocks) to 262 (4 x 4)
         // and loses to the two separate kernels; with ONE channel per lane (dword accesses, 32 lanes per
@@ -1390,9 +1552,11 @@ long nhwc_bwd_fused(int mode, const IO *x, const IO *gy, const IO *taps, IO *gx,
         // layer of the stack (28x28 C=240: 112 -> 91 us, 14x14 C=672: 75 -> 68, C=480: 59 -> 50, 7x7 C=1152: 42 -> 39).
         // 16 bits: two channels (rows travel raw, in half the registers) and 7 x 2 blocks; bf16 28x28 C=240 75 us with the
         // separate kernels, 64 with 7 x 2 or 7 x 4 blocks; 14x14 C=480 45 / 37 / 38, C=672 58 / 47 / 51; 7x7 C=1152 31 / 29 / 34.
+        // On pairs it needs 170 registers, two wavefronts per SIMD; with two rows in flight and three asked for 161: multiply-adds /
+        // pairs / pairs with three wavefronts 70.7 / 75.0 / 66.9, 40.3 / 43.8 / 36.2, 49.5 / 54.4 / 46.7, 31.4 / 31.1 / 28.4.
         if (env_int("DWCONV_NHWC_FUSED5", 1)) {
             if constexpr (sizeof(IO) == 4) return nhwc_bwd_fused_case<IO, 5, 1, 7, 4>(mode, x, gy, taps, gx, gw, ws, ws_bytes, g, stream);
-            else return nhwc_bwd_fused_case<IO, 5, 2, 7, 2>(mode, x, gy, taps, gx, gw, ws, ws_bytes, g, stream);
+            else return nhwc_bwd_fused_case<IO, 5, 2, 7, 2, 2, 3>(mode, x, gy, taps, gx, gw, ws, ws_bytes, g, stream);
         }
         return -1;
     }

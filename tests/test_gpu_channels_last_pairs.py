@@ -1,0 +1,56 @@
+"""16-bit channels-last kernels that take two taps or two pixels at a time: the 5x5 and 7x7 sweeps for both gradients and the
+tall forward blocks, where a block, a channel group or a pair ends, and with infinities beside the windows."""
+import pytest
+import torch
+
+import oracle
+from shapes import make_inputs, shape_id
+
+pytestmark = pytest.mark.gpu
+
+# 7x7: from 2^15 elements on; blocks of 4 x 4 (backward), 7 x 4 or 4 x 4 (forward).  5x5: blocks of 7 x 2 and 7 x 4
+CASES = [((2, 96, 13, 15, 7, 1, 3), "nhwc_bwd16<k7"), ((1, 768, 7, 7, 7, 1, 3), "nhwc_bwd16<k7"), ((3, 36, 28, 12, 7, 1, 3), "nhwc_bwd16<k7"),
+         ((5, 132, 9, 6, 7, 1, 3), "nhwc_bwd16<k7"), ((1, 8, 64, 65, 7, 1, 3), "nhwc_bwd16<k7"), ((40, 840, 1, 1, 7, 1, 3), "nhwc_bwd16<k7"),
+         ((2, 64, 16, 15, 7, 1, 3), "nhwc_down16<k7"), ((2, 68, 14, 13, 5, 1, 2), "nhwc_bwd16<k5"), ((9, 32, 7, 8, 5, 1, 2), "nhwc_bwd16<k5"),
+         ((1, 100, 21, 3, 5, 1, 2), "nhwc_bwd16<k5"), ((1, 12, 35, 1, 5, 1, 2), "nhwc_bwd16<k5")]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("case", CASES, ids=lambda c: shape_id(c[0]))
+def test_both_directions(gpu, case, dtype):
+    """|error| <= u |ref| + 1e-5 of the largest result: one rounding to the element type and fp32 sums."""
+    from torch_dwconv import _C, depthwise_conv2d
+
+    shape, backward = case
+    n, c, h, w, k, s, p = shape
+    x, wt, gy = (t.to(dtype) for t in make_inputs(shape, seed=41))
+    xg, gyg = (t.to(gpu).contiguous(memory_format=torch.channels_last) for t in (x, gy))
+    y = depthwise_conv2d(xg, wt.to(gpu), stride=s, padding=p)
+    gx, gw = _C.dwconv2d_backward_nhwc(xg, gyg, wt.to(gpu), s, s, p, p)
+    assert _C.last_variant().startswith(backward), _C.last_variant()
+    u = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    for got, ref in zip((y, gx, gw), oracle.torch_reference(x, wt, gy, s, p)):
+        assert got.shape == ref.shape
+        err = (got.cpu().double() - ref).abs()
+        assert bool((err <= u * ref.abs() + 1e-5 * ref.abs().max()).all()), float(err.max())
+    gx2, gw2 = _C.dwconv2d_backward_nhwc(xg, gyg, wt.to(gpu), s, s, p, p)
+    assert torch.equal(gx, gx2) and torch.equal(gw, gw2)
+
+
+@pytest.mark.parametrize("k", [5, 7])
+def test_infinite_elements_reach_their_windows_only(gpu, k):
+    from torch_dwconv import _C, depthwise_conv2d
+
+    n, c, h, w, p = 2, 64, 28, 28, k // 2
+    x, wt, gy = (t.to(torch.bfloat16) for t in make_inputs((n, c, h, w, k, 1, p), seed=42))
+    wt = wt.abs() + 0.25  # (an infinite element gives an infinite result under every tap)
+    gy2 = gy.clone()
+    x[0, 3, 9, 11] = x[1, 0, 0, 0] = gy2[1, 5, 14, 13] = gy2[0, 63, 27, 27] = float("inf")
+    xg, gyg = (t.to(gpu).contiguous(memory_format=torch.channels_last) for t in (x, gy2))
+    y = depthwise_conv2d(xg, wt.to(gpu), stride=1, padding=p).cpu()
+    gx, _ = _C.dwconv2d_backward_nhwc(xg, gyg, wt.to(gpu), 1, 1, p, p)
+    ref = torch.nn.functional.conv2d(x.double(), wt.double(), padding=p, groups=c)
+    gx_ref = torch.nn.grad.conv2d_input(x.shape, wt.double(), gy2.double(), padding=p, groups=c)
+    for got, want in ((y, ref), (gx.cpu(), gx_ref)):
+        assert not bool(got.isnan().any())
+        assert torch.equal(got.isinf(), want.isinf())
