@@ -17,7 +17,7 @@
 // Width instances (exact or ragged) as in dwconv_small_fir.hpp: W is the width of x, or its capacity class.
 #pragma once
 
-#include "dwconv_small_common.hpp"
+#include "dwconv_small16.hpp"
 
 namespace dwconv {
 
@@ -76,6 +76,17 @@ __device__ __forceinline__ void run_commit(const IO *__restrict__ g, float *lds,
     // (a run with padded rows is whole groups of four)
     const int tail = n4 * 4 + threadIdx.x;
     if (GPR == 0 && tail < n) lds[tail] = Io<IO>::in(g[tail]);
+}
+
+// (16-bit images)
+template <typename IO, int RR>
+__device__ __forceinline__ void run_commit16(const IO *__restrict__ g, uint16_t *lds, int n, const uint2 (&v)[RR])
+{
+    const int n4 = n >> 2;
+#pragma unroll
+    for (int u = 0; u < RR; ++u) reinterpret_cast<uint2 *>(lds)[min(static_cast<int>(threadIdx.x) + u * kWave, n4 - 1)] = v[u];
+    const int tail = n4 * 4 + threadIdx.x;
+    if (tail < n) lds[tail] = reinterpret_cast<const uint16_t *>(g)[tail];
 }
 
 // PF: the runs of the next image are fetched into registers while the current image is processed
@@ -398,6 +409,93 @@ __global__ __launch_bounds__(kWave, EPI ? 2 : 1) void small_bwd_kernel(const Sma
     }
 }
 
+// Both gradients of a stride-1 layer of 16-bit elements, with 16-bit images (dwconv_small16.hpp).  The steps of small_bwd_kernel.
+template <typename IO, int W, bool RAG, int K, int BH>
+__global__ __launch_bounds__(kWave) void small_bwd16_kernel(const SmallBwdPlan p)
+{
+    extern __shared__ float4 lds_raw[];
+    uint16_t *lds = reinterpret_cast<uint16_t *>(lds_raw);
+    constexpr int KK = K * K, P = K / 2, ND = row_dwords(W), RR = run_regs(W);
+    const int w = RAG ? p.in_w : W;
+    const int group = blockIdx.x / p.chunks;
+    const int chunk = blockIdx.x - group * p.chunks;
+    const int c0 = group * p.planes_per_run;
+    const int nplanes = min(p.planes_per_run, p.channel - c0);
+    const int n0 = chunk * p.images_per_chunk;
+    const int n1 = min(p.batch, n0 + p.images_per_chunk);
+    const int plane = p.in_h * w, nx = nplanes * plane;
+    uint16_t *lds_x = lds, *lds_g = lds + p.g_off;
+    clear_zero_row16<W>(lds, p.zero_off);
+
+    const int pl_raw = fast_div(threadIdx.x, p.lpp_magic);
+    const int rb = threadIdx.x - pl_raw * p.lanes_per_plane;
+    const bool active = pl_raw < nplanes;
+    const int pl = active ? pl_raw : 0;
+    const int oy0 = rb * BH;
+
+    float wacc[KK];
+#pragma unroll
+    for (int t = 0; t < KK; ++t) wacc[t] = 0.f;
+    Taps16<IO, K> taps;
+    taps.template load<true>(p.taps, c0 + pl, p.channel);
+
+    const IO *const x = static_cast<const IO *>(p.x);
+    const IO *const gy = static_cast<const IO *>(p.gy);
+    uint2 rx[RR], rg[RR];
+    auto fetch = [&](int n) {
+        const long e0 = (static_cast<long>(n) * p.channel + c0) * plane;
+        const int h = static_cast<int>(e0 & 3);
+        run_fetch<IO, RR>(x + (e0 - h), nx + h, rx);
+        run_fetch<IO, RR>(gy + (e0 - h), nx + h, rg);
+    };
+    fetch(n0);
+    for (int n = n0; n < n1; ++n) {
+        const long e0 = (static_cast<long>(n) * p.channel + c0) * plane;
+        const int head = static_cast<int>(e0 & 3);
+        if (n != n0) __syncthreads();  // the previous image is done with the LDS runs
+        run_commit16<IO, RR>(x + (e0 - head), lds_x, nx + head, rx);
+        run_commit16<IO, RR>(gy + (e0 - head), lds_g, nx + head, rg);
+        __syncthreads();
+        if (n + 1 < n1) fetch(n + 1);
+
+        const int at0 = head + pl * plane;  // the lane's plane in either run
+        auto row_at = [&](int base, int iy) { return static_cast<unsigned>(iy) < static_cast<unsigned>(p.in_h) ? base + at0 + iy * w : p.zero_off; };
+        uint32_t g[BH][ND];
+#pragma unroll
+        for (int b = 0; b < BH; ++b)
+            lds_load_row16<W, RAG>(lds, active ? row_at(p.g_off, oy0 + b) : p.zero_off, g[b], w);
+        grad_weight16<IO, W, K, BH>(g, [&](int wr, uint32_t(&d)[ND]) { lds_load_row16<W, RAG>(lds, row_at(0, oy0 - P + wr), d, w); }, wacc);
+
+        float xacc[BH][W];
+#pragma unroll
+        for (int b = 0; b < BH; ++b)
+#pragma unroll
+            for (int o = 0; o < W; ++o) xacc[b][o] = 0.f;
+        convolve16<IO, W, K, 1, BH, W>(taps, [&](int wr, uint32_t(&d)[ND]) { lds_load_row16<W, RAG>(lds, row_at(p.g_off, oy0 - P + wr), d, w); }, xacc);
+        __syncthreads();  // every lane is done with the x run: overwrite it with the gx run
+        if (active) {
+#pragma unroll
+            for (int b = 0; b < BH; ++b)
+                if (oy0 + b < p.in_h) lds_store_row16<IO, W, RAG>(lds_x, at0 + (oy0 + b) * w, xacc[b], w);
+        }
+        __syncthreads();
+        lds_to_run16(static_cast<IO *>(p.gx) + (e0 - head), lds_x, nx + head, head);
+    }
+
+    __syncthreads();  // the runs are dead; reuse the LDS to bring the lanes of each channel together
+    float *red = reinterpret_cast<float *>(lds_raw);
+#pragma unroll
+    for (int t = 0; t < KK; ++t) red[t * kSmallRedPitch + threadIdx.x] = wacc[t];
+    __syncthreads();
+    for (int e = threadIdx.x; e < nplanes * KK; e += kWave) {
+        const int q = e / KK, t = e - q * KK;
+        const float *col = red + t * kSmallRedPitch + q * p.lanes_per_plane;
+        float s = 0;
+        for (int i = 0; i < p.lanes_per_plane; ++i) s += col[i];
+        p.partial[(static_cast<long>(c0 + q) * p.chunks + chunk) * KK + t] = s;
+    }
+}
+
 template <int W, bool RAG, int K, int S, int BH, bool PAD>
 bool plan_small_bwd(SmallBwdPlan &p, const WgradGeometry &g)
 {
@@ -476,9 +574,25 @@ long small_bwd_case(int mode, const SmallBwdArgs &a, const WgradGeometry &g, hip
                      PAD ? ",pad" : "", p.planes_per_run, p.chunks);
         return launch_fused_final(p.partial, static_cast<IO *>(a.gw), a.param_grad, g.channel, K * K, p.chunks, stream);
     } else {
-        if (mode == 2)
-            hipLaunchKernelGGL((small_bwd_kernel<IO, W, RAG, K, S, BH, true, PAD, D>), dim3(groups * p.chunks), dim3(kWave), shmem, stream, p);
-        else
+        if constexpr (sizeof(IO) == 2 && D == 1 && S == 1) {
+            if (mode == 2 && small16_backward<K>(g.in_w)) {
+                const int run = p.planes_per_run * g.in_h * g.in_w + 3;
+                p.g_off = round_up(run, 8);
+                p.zero_off = round_up(p.g_off + run + (RAG ? W + 2 : 2), 8);
+                const size_t runs16 = static_cast<size_t>(p.zero_off + zero_row_elems16(W)) * 2;
+                hipLaunchKernelGGL((small_bwd16_kernel<IO, W, RAG, K, BH>), dim3(groups * p.chunks), dim3(kWave), std::max(runs16, red), stream, p);
+                const int rc = check_launch("small_bwd16_kernel");
+                if (rc != DWCONV_OK) return rc;
+                note_variant("small_bwd16<%s%d,k%d,s1,bh%d,dot2> P%d chunks%d", RAG ? "r" : "w", W, K, BH, p.planes_per_run, p.chunks);
+                return launch_wgrad_final(p.partial, static_cast<IO *>(a.gw), g.channel, K * K, p.chunks, stream);
+            }
+        }
+        // (no ragged width is one of those that stay)
+        constexpr bool kNever = sizeof(IO) == 2 && D == 1 && S == 1 && (RAG || small16_backward<K>(W));
+        if (mode == 2) {
+            if constexpr (kNever) return -1;
+            else hipLaunchKernelGGL((small_bwd_kernel<IO, W, RAG, K, S, BH, true, PAD, D>), dim3(groups * p.chunks), dim3(kWave), shmem, stream, p);
+        } else
             hipLaunchKernelGGL((small_bwd_kernel<IO, W, RAG, K, S, BH, false, PAD, D>), dim3(groups * p.chunks), dim3(kWave), shmem, stream, p);
         const int rc = check_launch("small_bwd_kernel");
         if (rc != DWCONV_OK) return rc;

@@ -26,6 +26,23 @@ inline bool small_width_is_exact(int w)
         return false;
     }
 }
+// Which 16-bit calls at dilation 1 get 16-bit LDS images (dwconv_small16.hpp) by their width, measured against the fp32 images on
+// every width from 4 to 32, C * W * W = 480 * 196, batch 64.  Forward (and grad-input of stride 1): 1 to 46 % faster, but for
+// bfloat16 (whose widening is a shift) at odd widths below 17, where rows start on any element (3 to 13 % slower with 3x3, up to 6 %
+// with larger filters), and 3x3 at 10 and 12 (4 and 8 % slower); float16 3x3 at odd widths below 10 (up to 5 % slower).  Both
+// gradients at stride 1: 1 to 47 % faster, but for 3x3 at 7 and 7x7 at 15 (4 and 10 % slower).
+template <typename IO, int K, int S>
+constexpr bool small16_forward(int w)
+{
+    if (S == 2) return true;
+    if (std::is_same<IO, bf16_t>::value) return (w % 2 == 0 || w >= 17) && !(K == 3 && (w == 10 || w == 12));
+    return !(K == 3 && w % 2 != 0 && w < 10);
+}
+template <int K>
+constexpr bool small16_backward(int w)
+{
+    return !(K == 3 && w == 7) && !(K == 7 && w == 15);
+}
 // capacity class of a width that has no exact instance; 0 when it is too wide for this family
 inline int small_ragged_class(int w) { return w < 1 || w > 32 ? 0 : (w + 7) / 8 * 8; }
 

@@ -26,7 +26,7 @@
 // (grad-weight and the fused backward of these maps: dwconv_small_bwd.hpp)
 #pragma once
 
-#include "dwconv_small_common.hpp"
+#include "dwconv_small16.hpp"
 
 namespace dwconv {
 
@@ -124,6 +124,54 @@ __global__ __launch_bounds__(kWave) void small_down_kernel(const SmallPlan p)
         lds_to_run_rows(static_cast<IO *>(p.out) + (out0 - hout), lds, nplanes * out_plane + hout, hout, p.magic_out);
     else
         lds_to_run(static_cast<IO *>(p.out) + (out0 - hout), lds, nplanes * out_plane + hout, hout);
+}
+
+// The same for 16-bit elements, with 16-bit images (dwconv_small16.hpp).  Rows lie at their own width, whatever it is.
+template <typename IO, int W, bool RAG, int K, int S, bool FLIP, int BH>
+__global__ __launch_bounds__(kWave) void small_down16_kernel(const SmallPlan p)
+{
+    extern __shared__ float4 lds_raw[];
+    uint16_t *lds = reinterpret_cast<uint16_t *>(lds_raw);
+    constexpr int OW = (W - 1) / S + 1;
+    const int w_in = RAG ? p.in_w : W, w_out = RAG ? p.out_w : OW;
+    const long plane0 = static_cast<long>(blockIdx.x) * p.planes_per_run;
+    const int nplanes = static_cast<int>(min(static_cast<long>(p.planes_per_run), p.planes - plane0));
+    const int in_plane = p.in_h * w_in, out_plane = p.out_h * w_out;
+    const int pl_raw = fast_div(threadIdx.x, p.lpp_magic);
+    const int rb = threadIdx.x - pl_raw * p.lanes_per_plane;
+    const bool active = pl_raw < nplanes;
+    const int pl = active ? pl_raw : 0;
+    const long in0 = plane0 * in_plane, out0 = plane0 * out_plane;
+    const int hin = static_cast<int>(in0 & 3), hout = static_cast<int>(out0 & 3);
+
+    const int c = plane_channel(plane0, pl, p.planes, p.channel);
+    Taps16<IO, K> taps;
+    taps.template load<FLIP>(p.taps, c, p.channel);
+    run_to_lds16(static_cast<const IO *>(p.in) + (in0 - hin), lds, nplanes * in_plane + hin);
+    clear_zero_row16<W>(lds, p.zero_off);
+    __syncthreads();
+
+    float acc[BH][OW];
+#pragma unroll
+    for (int b = 0; b < BH; ++b)
+#pragma unroll
+        for (int o = 0; o < OW; ++o) acc[b][o] = 0.f;
+    const int oy0 = rb * BH, at0 = hin + pl * in_plane;
+    convolve16<IO, W, K, S, BH, OW>(taps, [&](int wr, uint32_t(&d)[row_dwords(W)]) {
+        const int iy = oy0 * S - p.pad_h + wr;
+        lds_load_row16<W, RAG>(lds, static_cast<unsigned>(iy) < static_cast<unsigned>(p.in_h) ? at0 + iy * w_in : p.zero_off, d, w_in);
+    }, acc);
+    if constexpr (!FLIP) {
+        if (p.epi.enabled()) epilogue_apply_block<1>(acc, p.epi, c);
+    }
+    __syncthreads();  // every lane has read its input rows: the run can be overwritten in place
+    if (active) {
+#pragma unroll
+        for (int b = 0; b < BH; ++b)
+            if (oy0 + b < p.out_h) lds_store_row16<IO, OW, RAG>(lds, hout + pl * out_plane + (oy0 + b) * w_out, acc[b], w_out);
+    }
+    __syncthreads();
+    lds_to_run16(static_cast<IO *>(p.out) + (out0 - hout), lds, nplanes * out_plane + hout, hout);
 }
 
 // up = 2, taps rotated, "same" padding of the forward conv (leading pad of the transposed problem = K/2):
@@ -270,11 +318,26 @@ int launch_small_down(SmallPlan &p, hipStream_t stream)
     size_t shmem;
     long runs;
     if (!finish_plan(p, shmem, runs, RAG ? W : 0, zero_row_floats(W), RAG)) return -1;
-    hipLaunchKernelGGL((small_down_kernel<IO, W, RAG, K, S, FLIP, BH, D>), dim3(static_cast<unsigned>(runs)), dim3(kWave),
-                       shmem, stream, p);
-    note_variant("small_down%s<%s%d,k%d,s%d,%s,bh%d%s> P%d", sizeof(IO) == 2 ? "16" : "", RAG ? "r" : "w", W, K, S,
-                 FLIP ? "rot" : "fwd", BH, D == 2 ? ",d2" : "", p.planes_per_run);
-    return check_launch("small_down_kernel");
+    if constexpr (sizeof(IO) == 2 && D == 1) {
+        if (small16_forward<IO, K, S>(p.in_w)) {
+            // (elements: the run, up to three in front of it, and what a ragged row's read takes past its end)
+            p.zero_off = round_up(p.planes_per_run * std::max(p.in_h * p.in_w, p.out_h * p.out_w) + 4 + (RAG ? W + 2 : 2), 8);
+            shmem = static_cast<size_t>(p.zero_off + zero_row_elems16(W)) * 2;
+            hipLaunchKernelGGL((small_down16_kernel<IO, W, RAG, K, S, FLIP, BH>), dim3(static_cast<unsigned>(runs)), dim3(kWave), shmem, stream, p);
+            note_variant("small_down16<%s%d,k%d,s%d,%s,bh%d,dot2> P%d", RAG ? "r" : "w", W, K, S, FLIP ? "rot" : "fwd", BH, p.planes_per_run);
+            return check_launch("small_down16_kernel");
+        }
+    }
+    // (the classes from 24 on hold no width below 17)
+    constexpr bool kNever = sizeof(IO) == 2 && D == 1 && (RAG ? S == 2 || W >= 24 : small16_forward<IO, K, S>(W));
+    if constexpr (kNever) return -1;
+    else {
+        hipLaunchKernelGGL((small_down_kernel<IO, W, RAG, K, S, FLIP, BH, D>), dim3(static_cast<unsigned>(runs)), dim3(kWave),
+                           shmem, stream, p);
+        note_variant("small_down%s<%s%d,k%d,s%d,%s,bh%d%s> P%d", sizeof(IO) == 2 ? "16" : "", RAG ? "r" : "w", W, K, S,
+                     FLIP ? "rot" : "fwd", BH, D == 2 ? ",d2" : "", p.planes_per_run);
+        return check_launch("small_down_kernel");
+    }
 }
 
 template <typename IO, int W, bool RAG, int K>
