@@ -177,12 +177,17 @@ __device__ __forceinline__ void nhwc_pair_row(const RawPixel<IO, CV> (&raw)[COLS
     }
 }
 
-// The taps of a filter row as K / 2 pairs (2 j with 2 j + 1) and a single one (fp32 bits): [ty][PER_ROW][channel] dwords in LDS.
+// The taps of a filter row as K / 2 pairs and a single one (fp32 bits): [ty][PER_ROW][channel] dwords in LDS.  In the order that
+// a stride-1 correlation meets them (tap 2 j with 2 j + 1), or, for the transposed stride-2 one (UP2), that consecutive pixels of
+// out_grad do: the EVEN pairs of even taps K - 1, K - 3, ..., then those of odd taps K - 2, K - 4, ..., each class falling; the
+// class with an odd number of taps leaves the single one (its last).
 template <int K>
 struct TapPairs {
     static constexpr int N = K / 2, PER_ROW = N + 1, TOTAL = K * PER_ROW;
+    static constexpr int EVEN = (K + 1) / 4, ODD = K / 2 / 2;
+    static constexpr int SINGLE = (K + 1) / 2 % 2 ? 0 : 1;  // UP2: the tap without a partner, and its class
 };
-template <typename IO, int K, bool FLIP>
+template <typename IO, int K, bool FLIP, bool UP2 = false>
 __device__ __forceinline__ void nhwc_stage_tap_pairs(const IO *__restrict__ taps, uint32_t *lds, int c0, int nch)
 {
     using P = TapPairs<K>;
@@ -195,7 +200,15 @@ __device__ __forceinline__ void nhwc_stage_tap_pairs(const IO *__restrict__ taps
         for (int k = 0; k < kTapBatch; ++k) {
             const int i = min(i0 + k * kNhwcThreads, total - 1), cl = i / P::TOTAL, e = i - cl * P::TOTAL;
             const int ty = e / P::PER_ROW, j = e - ty * P::PER_ROW;
-            const int a = 2 * j, b = min(a + 1, K - 1);
+            int a, b;
+            if constexpr (UP2) {
+                a = j < P::EVEN ? K - 1 - 4 * j : K - 2 - 4 * (j - P::EVEN);
+                a = j < P::N ? a : P::SINGLE;
+                b = j < P::N ? a - 2 : a;
+            } else {
+                a = 2 * j;
+                b = min(a + 1, K - 1);
+            }
             const int row = cl * (K * K) + (FLIP ? K - 1 - ty : ty) * K;
             first[k] = src[row + (FLIP ? K - 1 - a : a)];
             second[k] = src[row + (FLIP ? K - 1 - b : b)];
@@ -263,6 +276,32 @@ __device__ __forceinline__ void nhwc_pairs_row(const uint32_t (&pair)[COLS * CV]
         for (int q = 0; q < CV; ++q)
             sum[CV * o + q] = fmaf(cur[CV * (o * S + K - 1) + q], __uint_as_float(w[K / 2][q]), sum[CV * o + q]);
 }
+// The same for a row of the transposed stride-2 kernels: sum[o] += out_grad pixels j of the window times taps
+// tx = o + PE - 2 (DMIN + j).
+template <typename IO, int K, int PE, int DMIN, int TW, int CV, int GCOLS>
+__device__ __forceinline__ void nhwc_pairs_up2_row(const uint32_t (&pair)[GCOLS * CV], const float (&cur)[GCOLS * CV],
+                                                   const uint32_t (&w)[TapPairs<K>::PER_ROW][CV], float (&sum)[TW * CV])
+{
+    using P = TapPairs<K>;
+#pragma unroll
+    for (int o = 0; o < TW; ++o) {
+        const int odd = (o + PE) & 1, n = odd ? P::ODD : P::EVEN;
+        const int j0 = (o + PE - (K - 1 - odd)) / 2 - DMIN;  // the window pixel under the class's first tap (exact division)
+#pragma unroll
+        for (int m = 0; m < (P::EVEN > P::ODD ? P::EVEN : P::ODD); ++m) {
+            if (m >= n) continue;
+#pragma unroll
+            for (int q = 0; q < CV; ++q)
+                sum[CV * o + q] = dot2<IO>(pair[CV * (j0 + 2 * m) + q], w[odd ? P::EVEN + m : m][q], sum[CV * o + q]);
+        }
+        if (odd == P::SINGLE) {
+#pragma unroll
+            for (int q = 0; q < CV; ++q)
+                sum[CV * o + q] = fmaf(cur[CV * (j0 + 2 * n) + q], __uint_as_float(w[P::N][q]), sum[CV * o + q]);
+        }
+    }
+}
+
 // CV results of a pixel at byte offset `off` of the view (dropped when that is at or beyond kOob).
 template <typename IO, int CV>
 __device__ __forceinline__ void store_pixel(__amdgpu_buffer_rsrc_t view, unsigned off, const float *v)
@@ -836,8 +875,9 @@ __global__ __launch_bounds__(kNhwcThreads, WAVES) void nhwc_bwd_fused_kernel(con
 // the lane's own block, is kept for the x rows it meets; two x rows are consumed per out_grad row, right behind it.
 // The loop is unrolled, so only the rows in use are live.  out_grad is read once instead of twice and the separate
 // grad-input kernel (nhwc_up2_kernel) goes away.  The end of the kernel is that of nhwc_wgrad_kernel.
-template <typename IO, int K, int CV, int BQH, int BQW>
-__global__ __launch_bounds__(kNhwcThreads) void nhwc_bwd_s2_fused_kernel(const NhwcPlan p)
+// WAVES: wavefronts per SIMD asked for.
+template <typename IO, int K, int CV, int BQH, int BQW, int WAVES>
+__global__ __launch_bounds__(kNhwcThreads, WAVES) void nhwc_bwd_s2_fused_kernel(const NhwcPlan p)
 {
     extern __shared__ float4 lds_raw[];
     float *lds = reinterpret_cast<float *>(lds_raw);
@@ -859,7 +899,8 @@ __global__ __launch_bounds__(kNhwcThreads) void nhwc_bwd_s2_fused_kernel(const N
     const bool lane_ok = pb_local < p.blocks_per_wg && CV * lane_c < nch;
     const int c = c0 + (lane_ok ? CV * lane_c : 0);
     const int per_image = p.blocks_x * p.blocks_y;
-    nhwc_stage_taps<IO, KK, false>(static_cast<const IO *>(p.taps), lds, c0, nch);
+    if constexpr (kPairs<IO>) nhwc_stage_tap_pairs<IO, K, false, true>(static_cast<const IO *>(p.taps), reinterpret_cast<uint32_t *>(lds), c0, nch);
+    else nhwc_stage_taps<IO, KK, false>(static_cast<const IO *>(p.taps), lds, c0, nch);
     __syncthreads();
     const float *wl = lds + (lane_ok ? CV * lane_c : 0);
 
@@ -895,6 +936,7 @@ __global__ __launch_bounds__(kNhwcThreads) void nhwc_bwd_s2_fused_kernel(const N
 
         float gxs[GXH][GXW * CV];   // in_grad sums
         float gb[BQH][BQW * CV];    // the lane's own rows of out_grad
+        uint32_t gbpair[BQH][BQW * CV];  // (16 bits: the even pixels' pairs)
 #pragma unroll
         for (int b = 0; b < GXH; ++b)
 #pragma unroll
@@ -908,6 +950,8 @@ __global__ __launch_bounds__(kNhwcThreads) void nhwc_bwd_s2_fused_kernel(const N
             if (t < GROWS) {
                 float gcur[GCOLS * CV];
                 nhwc_widen_row<IO, GCOLS, CV>(gr[t & 1], gcur);
+                uint32_t gpair[GCOLS * CV];
+                nhwc_pair_row<1, IO, GCOLS, CV>(gr[t & 1], gpair);
                 const int d = DMIN + t;
                 // in_grad row b meets this row in tap row ty = b + P - 2 d, in_grad column o meets window column j
                 // in tap column tx = o + P - 2 (DMIN + j)
@@ -915,6 +959,12 @@ __global__ __launch_bounds__(kNhwcThreads) void nhwc_bwd_s2_fused_kernel(const N
                 for (int b = 0; b < GXH; ++b) {
                     const int ty = b + P - 2 * d;
                     if (ty < 0 || ty >= K) continue;
+                    if constexpr (kPairs<IO>) {
+                        uint32_t w[TapPairs<K>::PER_ROW][CV];
+                        nhwc_tap_row<K, CV>(reinterpret_cast<const uint32_t *>(wl), ty, nch, w);
+                        nhwc_pairs_up2_row<IO, K, P, DMIN, GXW, CV, GCOLS>(gpair, gcur, w, gxs[b]);
+                        continue;
+                    }
 #pragma unroll
                     for (int o = 0; o < GXW; ++o)
 #pragma unroll
@@ -928,7 +978,10 @@ __global__ __launch_bounds__(kNhwcThreads) void nhwc_bwd_s2_fused_kernel(const N
                 }
                 if (d >= 0 && d < BQH) {
 #pragma unroll
-                    for (int o = 0; o < BQW * CV; ++o) gb[d >= 0 && d < BQH ? d : 0][o] = gcur[CV * (-DMIN) + o];
+                    for (int o = 0; o < BQW * CV; ++o) {
+                        gb[d >= 0 && d < BQH ? d : 0][o] = gcur[CV * (-DMIN) + o];
+                        if constexpr (kPairs<IO>) gbpair[d >= 0 && d < BQH ? d : 0][o] = o / CV + 1 < BQW ? gpair[CV * (-DMIN) + o] : 0u;
+                    }
                 }
                 // rows no later out_grad row reaches: b < 2 (d + 1) - P; those finished before this step were stored then
 #pragma unroll
@@ -951,11 +1004,24 @@ __global__ __launch_bounds__(kNhwcThreads) void nhwc_bwd_s2_fused_kernel(const N
                 if (r + 1 < XROWS) nhwc_load_row<IO, XCOLS, CV>(xview, xr0 + r + 1, p.in_h, xrow_bytes, xcols, xr[(r + 1) & 1]);
                 float xcur[XCOLS * CV];
                 nhwc_widen_row<IO, XCOLS, CV>(xr[r & 1], xcur);
+                uint32_t xpair[XCOLS * CV];  // what pixels i and i + 1 of out_grad meet in one tap
+                nhwc_pair_row<2, IO, XCOLS, CV>(xr[r & 1], xpair);
 #pragma unroll
                 for (int ty = 0; ty < K; ++ty) {
                     if ((r - ty) % 2 != 0) continue;
                     const int j = (r - ty) / 2;
                     if (r - ty < 0 || j >= BQH) continue;
+                    if constexpr (kPairs<IO>) {
+                        static_assert(BQW % 2 == 0, "pixels of out_grad go in pairs");
+#pragma unroll
+                        for (int tx = 0; tx < K; ++tx)
+#pragma unroll
+                            for (int i = 0; i < BQW; i += 2)
+#pragma unroll
+                                for (int q = 0; q < CV; ++q)
+                                    acc[ty * K + tx][q] = dot2<IO>(gbpair[j][CV * i + q], xpair[CV * (2 * i + tx) + q], acc[ty * K + tx][q]);
+                        continue;
+                    }
 #pragma unroll
                     for (int tx = 0; tx < K; ++tx)
 #pragma unroll
@@ -1450,7 +1516,7 @@ long nhwc_bwd_fused_case(int mode, const IO *x, const IO *gy, const IO *taps, IO
 
 // Fused backward of K x K stride-2 layers with pad K/2 and even input extents.  mode 0: workspace bytes; mode 1:
 // launch.  -1 when the kernel does not cover g.
-template <typename IO, int K, int CV, int BQH, int BQW>
+template <typename IO, int K, int CV, int BQH, int BQW, int WAVES = 1>
 long nhwc_bwd_s2_fused_case(int mode, const IO *x, const IO *gy, const IO *taps, IO *gx, IO *gw, void *ws, size_t ws_bytes,
                             const NhwcGeometry &g, hipStream_t stream)
 {
@@ -1489,7 +1555,7 @@ long nhwc_bwd_s2_fused_case(int mode, const IO *x, const IO *gy, const IO *taps,
     p.pad_h = g.pad_h;
     p.pad_w = g.pad_w;
     const size_t shmem = static_cast<size_t>(p.lanes_c) * CV * 4 * std::max(K * K, p.blocks_per_wg * K);
-    hipLaunchKernelGGL((nhwc_bwd_s2_fused_kernel<IO, K, CV, BQH, BQW>), dim3(p.groups * cgroups), dim3(kNhwcThreads), shmem, stream, p);
+    hipLaunchKernelGGL((nhwc_bwd_s2_fused_kernel<IO, K, CV, BQH, BQW, WAVES>), dim3(p.groups * cgroups), dim3(kNhwcThreads), shmem, stream, p);
     int rc = check_launch("nhwc_bwd_s2_fused_kernel");
     if (rc != DWCONV_OK) return rc;
     note_variant("nhwc_bwd%s<k%d,s2,cv%d,%dx%d> lanes_c%d chunks%d", sizeof(IO) == 2 ? "16" : "", K, CV, BQH, BQW, p.lanes_c, p.groups);
@@ -1526,12 +1592,17 @@ long nhwc_bwd_fused(int mode, const IO *x, const IO *gy, const IO *taps, IO *gx,
         // with 2 x 2 blocks (186 registers, 260 and 64 us), 7 x 4 blocks for 5x5 (256 registers: twice the time).
         // 16-bit elements, 3x3: two channels per lane (one 4-byte access) and blocks of 2 x 4 out_grad pixels; bf16 112x112
         // C=96 155.7 us with the two separate kernels, 144.7 with 4 x 2 blocks, 139.4 with 4 x 4, 141.0 with 2 x 4; 28x28 C=240
-        // 46.0, 39.9, 44.4, 39.0.  5x5 stays on the separate kernels (56x56 C=144 85 us against 92-102 with 2 x 2 to 4 x 2 blocks).
+        // 46.0, 39.9, 44.4, 39.0.  5x5 on pairs: 4 x 2 blocks in 158 registers, three wavefronts asked for (without: 153, and 4-8 %
+        // slower).  bf16, us with the two separate kernels / here: batch 128 56x56 C=144 87.4 / 82.3, 14x14 C=672 38.7 / 34.3, batch 64
+        // 64x64 C=144 68.0 / 60.8, 16x16 C=672 28.1 / 23.7; 2 x 2, 2 x 4 and 4 x 4 blocks: 98, 87 and 92 us on the first.  Calls of less
+        // than 2^15 elements, one or two workgroups, stay on the separate kernels.
         if constexpr (sizeof(IO) == 4) {
             if (g.kernel_h == 3) return nhwc_bwd_s2_fused_case<IO, 3, 1, 7, 4>(mode, x, gy, taps, gx, gw, ws, ws_bytes, g, stream);
             return nhwc_bwd_s2_fused_case<IO, 5, 1, 4, 2>(mode, x, gy, taps, gx, gw, ws, ws_bytes, g, stream);
         } else {
             if (g.kernel_h == 3) return nhwc_bwd_s2_fused_case<IO, 3, 2, 2, 4>(mode, x, gy, taps, gx, gw, ws, ws_bytes, g, stream);
+            if (static_cast<long>(g.batch) * g.in_h * g.in_w * g.channel >= 1l << 15)
+                return nhwc_bwd_s2_fused_case<IO, 5, 2, 4, 2, 3>(mode, x, gy, taps, gx, gw, ws, ws_bytes, g, stream);
         }
         return -1;
     }

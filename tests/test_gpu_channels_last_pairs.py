@@ -8,10 +8,13 @@ from shapes import make_inputs, shape_id
 
 pytestmark = pytest.mark.gpu
 
-# 7x7: from 2^15 elements on; blocks of 4 x 4 (backward), 7 x 4 or 4 x 4 (forward).  5x5: blocks of 7 x 2 and 7 x 4
+# 7x7: from 2^15 elements on; blocks of 4 x 4 (backward), 7 x 4 or 4 x 4 (forward).  5x5: blocks of 7 x 2 and 7 x 4; stride 2, from
+# 2^15 elements on and on even extents: 4 x 2 pixels of out_grad
 CASES = [((2, 96, 13, 15, 7, 1, 3), "nhwc_bwd16<k7"), ((1, 768, 7, 7, 7, 1, 3), "nhwc_bwd16<k7"), ((3, 36, 28, 12, 7, 1, 3), "nhwc_bwd16<k7"),
          ((5, 132, 9, 6, 7, 1, 3), "nhwc_bwd16<k7"), ((1, 8, 64, 65, 7, 1, 3), "nhwc_bwd16<k7"), ((40, 840, 1, 1, 7, 1, 3), "nhwc_bwd16<k7"),
          ((2, 64, 16, 15, 7, 1, 3), "nhwc_down16<k7"), ((2, 68, 14, 13, 5, 1, 2), "nhwc_bwd16<k5"), ((9, 32, 7, 8, 5, 1, 2), "nhwc_bwd16<k5"),
+         ((2, 64, 18, 18, 5, 2, 2), "nhwc_bwd16<k5,s2"), ((1, 36, 34, 30, 5, 2, 2), "nhwc_bwd16<k5,s2"), ((3, 132, 2, 46, 5, 2, 2), "nhwc_bwd16<k5,s2"),
+         ((5, 100, 36, 2, 5, 2, 2), "nhwc_bwd16<k5,s2"), ((2, 64, 17, 18, 5, 2, 2), "nhwc_up216<k5"), ((2, 68, 14, 26, 3, 2, 1), "nhwc_bwd16<k3,s2"),
          ((1, 100, 21, 3, 5, 1, 2), "nhwc_bwd16<k5"), ((1, 12, 35, 1, 5, 1, 2), "nhwc_bwd16<k5")]
 
 
@@ -54,3 +57,20 @@ def test_infinite_elements_reach_their_windows_only(gpu, k):
     for got, want in ((y, ref), (gx.cpu(), gx_ref)):
         assert not bool(got.isnan().any())
         assert torch.equal(got.isinf(), want.isinf())
+
+
+@pytest.mark.parametrize("k", [3, 5])
+def test_infinite_gradients_of_stride_2_layers(gpu, k):
+    """The transposed taps go in pairs of their own classes: no result takes a pixel of out_grad under a tap it does not have."""
+    from torch_dwconv import _C
+
+    n, c, h, w, p = 2, 64, 28, 28, k // 2
+    x, wt, gy = (t.to(torch.bfloat16) for t in make_inputs((n, c, h, w, k, 2, p), seed=43))
+    wt = wt.abs() + 0.25
+    gy[1, 5, 7, 6] = gy[0, 63, 13, 13] = gy[0, 0, 0, 0] = gy[1, 8, 4, 13] = float("inf")
+    xg, gyg = (t.to(gpu).contiguous(memory_format=torch.channels_last) for t in (x, gy))
+    gx, _ = _C.dwconv2d_backward_nhwc(xg, gyg, wt.to(gpu), 2, 2, p, p)
+    assert _C.last_variant().startswith(f"nhwc_bwd16<k{k},s2"), _C.last_variant()
+    want = torch.nn.grad.conv2d_input(x.shape, wt.double(), gy.double(), stride=2, padding=p, groups=c)
+    gx = gx.cpu()
+    assert not bool(gx.isnan().any()) and torch.equal(gx.isinf(), want.isinf())
