@@ -1,5 +1,5 @@
 // Whole-plane kernels for small feature maps (up to 32 elements wide, "same" column padding); element type fp32,
-// fp16 or bf16, LDS and arithmetic fp32.
+// fp16 or bf16, LDS and arithmetic fp32 (16-bit tensors: 16-bit images where small16_forward says so, small_down16_kernel).
 //
 // Planes of a small map are tiny (196 B to 4 KiB) and sit back to back in memory,
 // so the only way to move them at HBM speed is to treat a run of P planes as one
