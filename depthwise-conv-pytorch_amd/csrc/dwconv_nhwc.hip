@@ -693,7 +693,12 @@ __global__ __launch_bounds__(kNhwcThreads) void nhwc_wgrad_kernel(const NhwcPlan
 // grad-weight sums.  The loop is unrolled, so only the rows in use are live.  out_grad is read once instead of
 // twice and the separate grad-input kernel goes away.  The end of the kernel is that of nhwc_wgrad_kernel.
 // AHEAD: window rows in flight; WAVES: wavefronts per SIMD asked for.
-template <typename IO, int K, int CV, int BH, int TW, int AHEAD, int WAVES>
+// EDGE: the map's height is not whole blocks, and the sums of the rows of out_grad past it are dropped.  Those rows are zeros, but
+// they meet rows of x that are not (the last P, in the tap rows above the centre), and zero times an infinite x is NaN in taps
+// that it has no part in.  A select after each such tap row, not a branch around it: with branches the 7x7 instance spills 263
+// registers.  bf16, batch 64, us without / with: 14x14 C=384 7x7 38.1 / 39.5, 7x7 C=768 27.8 / 28.4.  (Blocks of the other
+// filters hang over the map as those of nhwc_wgrad_kernel do, and every block does over the last column: their zeros meet x.)
+template <typename IO, int K, int CV, int BH, int TW, int AHEAD, int WAVES, bool EDGE>
 __global__ __launch_bounds__(kNhwcThreads, WAVES) void nhwc_bwd_fused_kernel(const NhwcPlan p)
 {
     extern __shared__ float4 lds_raw[];
@@ -820,13 +825,16 @@ __global__ __launch_bounds__(kNhwcThreads, WAVES) void nhwc_bwd_fused_kernel(con
                     if (b < 0 || b >= BH) continue;
                     if constexpr (kPairs<IO>) {
                         static_assert(TW % 2 == 0, "pixels of out_grad go in pairs");
+                        const bool past = EDGE && b > 0 && ty < P && oy0 + b >= p.in_h;
 #pragma unroll
                         for (int tx = 0; tx < K; ++tx)
 #pragma unroll
-                            for (int o = 0; o < TW; o += 2)
+                            for (int q = 0; q < CV; ++q) {
+                                float sum = acc[ty * K + tx][q];
 #pragma unroll
-                                for (int q = 0; q < CV; ++q)
-                                    acc[ty * K + tx][q] = dot2<IO>(gbpair[b][CV * o + q], xpair[CV * (o + tx) + q], acc[ty * K + tx][q]);
+                                for (int o = 0; o < TW; o += 2) sum = dot2<IO>(gbpair[b][CV * o + q], xpair[CV * (o + tx) + q], sum);
+                                acc[ty * K + tx][q] = past ? acc[ty * K + tx][q] : sum;
+                            }
                         continue;
                     }
 #pragma unroll
@@ -875,8 +883,8 @@ __global__ __launch_bounds__(kNhwcThreads, WAVES) void nhwc_bwd_fused_kernel(con
 // the lane's own block, is kept for the x rows it meets; two x rows are consumed per out_grad row, right behind it.
 // The loop is unrolled, so only the rows in use are live.  out_grad is read once instead of twice and the separate
 // grad-input kernel (nhwc_up2_kernel) goes away.  The end of the kernel is that of nhwc_wgrad_kernel.
-// WAVES: wavefronts per SIMD asked for.
-template <typename IO, int K, int CV, int BQH, int BQW, int WAVES>
+// WAVES: wavefronts per SIMD asked for.  EDGE: as in nhwc_bwd_fused_kernel (bf16, batch 128, 14x14 C=672 5x5, us without / with: 34.2 / 34.5).
+template <typename IO, int K, int CV, int BQH, int BQW, int WAVES, bool EDGE>
 __global__ __launch_bounds__(kNhwcThreads, WAVES) void nhwc_bwd_s2_fused_kernel(const NhwcPlan p)
 {
     extern __shared__ float4 lds_raw[];
@@ -1013,13 +1021,16 @@ __global__ __launch_bounds__(kNhwcThreads, WAVES) void nhwc_bwd_s2_fused_kernel(
                     if (r - ty < 0 || j >= BQH) continue;
                     if constexpr (kPairs<IO>) {
                         static_assert(BQW % 2 == 0, "pixels of out_grad go in pairs");
+                        const bool past = EDGE && j > 0 && ty < P && q0 + j >= p.out_h;
 #pragma unroll
                         for (int tx = 0; tx < K; ++tx)
 #pragma unroll
-                            for (int i = 0; i < BQW; i += 2)
+                            for (int q = 0; q < CV; ++q) {
+                                float sum = acc[ty * K + tx][q];
 #pragma unroll
-                                for (int q = 0; q < CV; ++q)
-                                    acc[ty * K + tx][q] = dot2<IO>(gbpair[j][CV * i + q], xpair[CV * (2 * i + tx) + q], acc[ty * K + tx][q]);
+                                for (int i = 0; i < BQW; i += 2) sum = dot2<IO>(gbpair[j][CV * i + q], xpair[CV * (2 * i + tx) + q], sum);
+                                acc[ty * K + tx][q] = past ? acc[ty * K + tx][q] : sum;
+                            }
                         continue;
                     }
 #pragma unroll
@@ -1505,7 +1516,12 @@ long nhwc_bwd_fused_case(int mode, const IO *x, const IO *gy, const IO *taps, IO
     p.pad_h = g.pad_h;
     p.pad_w = g.pad_w;
     const size_t shmem = static_cast<size_t>(p.lanes_c) * CV * 4 * std::max(K * K, p.blocks_per_wg * K);
-    hipLaunchKernelGGL((nhwc_bwd_fused_kernel<IO, K, CV, BH, TW, AHEAD, WAVES>), dim3(p.groups * cgroups), dim3(kNhwcThreads), shmem, stream, p);
+    auto launch = [&](auto edge) {
+        hipLaunchKernelGGL((nhwc_bwd_fused_kernel<IO, K, CV, BH, TW, AHEAD, WAVES, decltype(edge)::value>), dim3(p.groups * cgroups),
+                           dim3(kNhwcThreads), shmem, stream, p);
+    };
+    if (kPairs<IO> && K == 7 && g.in_h % BH != 0) launch(std::bool_constant<kPairs<IO> && K == 7>{});
+    else launch(std::false_type{});
     int rc = check_launch("nhwc_bwd_fused_kernel");
     if (rc != DWCONV_OK) return rc;
     note_variant("nhwc_bwd%s<k%d,s1,cv%d,%dx%d> lanes_c%d chunks%d", sizeof(IO) == 2 ? "16" : "", K, CV, BH, TW, p.lanes_c, p.groups);
@@ -1555,7 +1571,12 @@ long nhwc_bwd_s2_fused_case(int mode, const IO *x, const IO *gy, const IO *taps,
     p.pad_h = g.pad_h;
     p.pad_w = g.pad_w;
     const size_t shmem = static_cast<size_t>(p.lanes_c) * CV * 4 * std::max(K * K, p.blocks_per_wg * K);
-    hipLaunchKernelGGL((nhwc_bwd_s2_fused_kernel<IO, K, CV, BQH, BQW, WAVES>), dim3(p.groups * cgroups), dim3(kNhwcThreads), shmem, stream, p);
+    auto launch = [&](auto edge) {
+        hipLaunchKernelGGL((nhwc_bwd_s2_fused_kernel<IO, K, CV, BQH, BQW, WAVES, decltype(edge)::value>), dim3(p.groups * cgroups),
+                           dim3(kNhwcThreads), shmem, stream, p);
+    };
+    if (kPairs<IO> && K == 5 && g.out_h % BQH != 0) launch(std::bool_constant<kPairs<IO> && K == 5>{});
+    else launch(std::false_type{});
     int rc = check_launch("nhwc_bwd_s2_fused_kernel");
     if (rc != DWCONV_OK) return rc;
     note_variant("nhwc_bwd%s<k%d,s2,cv%d,%dx%d> lanes_c%d chunks%d", sizeof(IO) == 2 ? "16" : "", K, CV, BQH, BQW, p.lanes_c, p.groups);

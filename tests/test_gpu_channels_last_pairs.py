@@ -74,3 +74,30 @@ def test_infinite_gradients_of_stride_2_layers(gpu, k):
     want = torch.nn.grad.conv2d_input(x.shape, wt.double(), gy.double(), stride=2, padding=p, groups=c)
     gx = gx.cpu()
     assert not bool(gx.isnan().any()) and torch.equal(gx.isinf(), want.isinf())
+
+
+# heights that are not whole blocks of four rows, and two that are: the block that hangs over the map has zeros for out_grad there
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("shape", [(3, 64, 14, 16, 7, 1, 3), (3, 64, 13, 16, 7, 1, 3), (3, 36, 23, 20, 7, 1, 3), (40, 64, 2, 8, 7, 1, 3), (80, 64, 1, 8, 7, 1, 3),
+                                   (3, 64, 16, 16, 7, 1, 3), (3, 64, 14, 16, 5, 2, 2), (3, 36, 26, 20, 5, 2, 2), (40, 64, 2, 8, 5, 2, 2), (3, 64, 16, 16, 5, 2, 2)],
+                         ids=shape_id)
+def test_infinite_input_reaches_its_own_taps_only(gpu, shape, dtype):
+    """One infinite element of x a channel, in every row of the map's lower end and some others: the taps of the filter's gradient
+    whose sums hold it are not finite, all others are.  (The widths are whole blocks.)"""
+    from torch_dwconv import _C
+
+    n, c, h, w, k, s, p = shape
+    x, wt, gy = (t.to(dtype) for t in make_inputs(shape, seed=44))
+    oh, ow = gy.shape[2:]
+    own = torch.zeros(c, 1, k, k, dtype=torch.bool)
+    for i in range(c):
+        iy, ix = max(0, h - 1 - i % 8), (5 * i) % w
+        x[i % n, i, iy, ix] = float("inf")
+        for t in range(k):
+            for u in range(k):
+                oy, ox = iy + p - t, ix + p - u
+                own[i, 0, t, u] = oy % s == 0 and ox % s == 0 and 0 <= oy // s < oh and 0 <= ox // s < ow
+    xg, gyg = (t.to(gpu).contiguous(memory_format=torch.channels_last) for t in (x, gy))
+    gw = _C.dwconv2d_backward_nhwc(xg, gyg, wt.to(gpu), s, s, p, p)[1].cpu()
+    assert _C.last_variant().startswith(f"nhwc_bwd16<k{k},s{s}"), _C.last_variant()
+    assert torch.equal(~gw.isfinite(), own)
