@@ -101,3 +101,30 @@ def test_infinite_input_reaches_its_own_taps_only(gpu, shape, dtype):
     gw = _C.dwconv2d_backward_nhwc(xg, gyg, wt.to(gpu), s, s, p, p)[1].cpu()
     assert _C.last_variant().startswith(f"nhwc_bwd16<k{k},s{s}"), _C.last_variant()
     assert torch.equal(~gw.isfinite(), own)
+
+
+# channel counts off the lane groups, maps off the blocks, images that end between two trips
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("shape", [(5, 40, 23, 17, 7, 1, 3), (5, 64, 28, 28, 7, 1, 3), (5, 40, 23, 17, 5, 1, 2), (40, 132, 7, 7, 5, 1, 2),
+                                   (5, 36, 34, 30, 5, 2, 2), (5, 40, 28, 28, 3, 2, 1), (7, 36, 32, 20, 3, 1, 1)], ids=shape_id)
+def test_several_trips_a_workgroup(gpu, monkeypatch, shape, dtype):
+    """One workgroup a channel group: it carries its sums through every block of every image, and its views to later images."""
+    from torch_dwconv import _C
+
+    n, c, h, w, k, s, p = shape
+    monkeypatch.setenv("DWCONV_TUNING", "1")
+    monkeypatch.setenv("DWCONV_NHWC_WGRAD_WGS", "1")
+    x, wt, gy = (t.to(dtype) for t in make_inputs(shape, seed=45))
+    xg, gyg = (t.to(gpu).contiguous(memory_format=torch.channels_last) for t in (x, gy))
+    gx, gw = _C.dwconv2d_backward_nhwc(xg, gyg, wt.to(gpu), s, s, p, p)
+    variant = _C.last_variant()
+    assert variant.startswith(f"nhwc_bwd16<k{k},s{s}") and variant.endswith(" chunks1"), variant
+    rows, columns = (int(v) for v in variant.split(">")[0].split(",")[-1].split("x"))  # a block of out_grad
+    lanes_c = int(variant.split(" lanes_c")[1].split(" ")[0])
+    oh, ow = gy.shape[2:]
+    blocks = n * -(-oh // rows) * -(-ow // columns)
+    assert blocks >= 3 * (256 // lanes_c), variant
+    u = 2.0 ** -8 if dtype == torch.bfloat16 else 2.0 ** -11
+    for got, ref in zip((gx, gw), oracle.torch_reference(x, wt, gy, s, p)[1:]):
+        err = (got.cpu().double() - ref).abs()
+        assert bool((err <= u * ref.abs() + 1e-5 * ref.abs().max()).all()), float(err.max())

@@ -91,3 +91,22 @@ def test_fused_epilogue(gpu, shape):
     conv = torch.nn.functional.conv2d(x.double(), wt.double(), stride=s, padding=p, groups=c)
     z = conv * scale.double().view(1, -1, 1, 1) + bias.double().view(1, -1, 1, 1)
     check(y, z * torch.sigmoid(z), UNIT[torch.float16])
+
+
+# odd planes and odd channel counts: the runs of consecutive images start on different elements of a group of four
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("shape", [(6, 3, 19, 19, 5, 1, 2), (5, 5, 13, 13, 3, 1, 1), (7, 7, 9, 9, 7, 1, 3), (5, 9, 11, 17, 5, 1, 2), (5, 3, 15, 15, 5, 1, 2),
+                                   (6, 5, 28, 28, 3, 1, 1), (5, 3, 31, 31, 7, 1, 3), (9, 40, 7, 7, 5, 1, 2)], ids=shape_id)
+def test_several_images_a_wavefront(gpu, monkeypatch, shape, dtype):
+    """One wavefront a channel group: the next image is fetched while one is worked on, sums go on from image to image."""
+    from torch_dwconv import _C
+
+    n, c, h, w, k, s, p = shape
+    monkeypatch.setenv("DWCONV_TUNING", "1")
+    monkeypatch.setenv("DWCONV_SMALL_WGRAD_WAVES", "1")
+    x, wt, gy = (t.to(dtype) for t in make_inputs(shape, seed=54))
+    gx, gw = _C.dwconv2d_backward(x.to(gpu), gy.to(gpu), wt.to(gpu), s, s, p, p)
+    assert ",dot2>" in _C.last_variant() and _C.last_variant().endswith(" chunks1"), _C.last_variant()
+    _, gx_ref, gw_ref = oracle.torch_reference(x, wt, gy, s, p)
+    check(gx, gx_ref, UNIT[dtype])
+    check(gw, gw_ref, UNIT[dtype])

@@ -22,10 +22,15 @@ def test_backward(gpu, shape, dtype, by):
     n, c, h, w, k, s, p = shape
     x, wt, gy = (t.to(dtype) for t in make_inputs(shape, seed=61))
     gx, gw = _C.dwconv2d_backward(shifted(x, gpu, by), shifted(gy, gpu, by), wt.to(gpu), s, s, p, p)
-    assert _C.last_variant().startswith("bwd_stack16<"), _C.last_variant()
+    variant = _C.last_variant()
+    assert variant.startswith("bwd_stack16<") and " dot2" in variant, variant
+    # rows that start on any element: grad-input leaves through LDS as one run an image
+    assert (" anystart" in variant) == bool(w % 2 or by), variant
     _, gx_ref, gw_ref = oracle.torch_reference(x, wt, gy, s, p)
     check(gx, gx_ref, UNIT[dtype])
     check(gw, gw_ref, UNIT[dtype])
+    gx2, gw2 = _C.dwconv2d_backward(shifted(x, gpu, by), shifted(gy, gpu, by), wt.to(gpu), s, s, p, p)
+    assert torch.equal(gx, gx2) and torch.equal(gw, gw2)
 
 
 @pytest.mark.parametrize("shape", [(2, 2, 48, 48, 3, 1, 1), (2, 2, 40, 51, 5, 1, 2), (2, 2, 40, 54, 7, 1, 3)], ids=shape_id)
