@@ -156,8 +156,8 @@ __device__ __forceinline__ void nhwc_taps(const float *wl, float (&w)[CV])
 }
 
 // ---- 16-bit elements: two products per instruction ------------------------------------------------------------
-// Two taps (grad-weight: two pixels) at a time: a two-element dot product (v_dot2, at the rate of a multiply-add; both products
-// exact, one fp32 sum, subnormals kept) of two pixels of one channel and two taps.  A pixel holds its channels side by side, so a
+// Two taps (grad-weight: two pixels) at a time: a two-element dot product (v_dot2, at the rate of a multiply-add; it rounds like two
+// multiply-adds of widened elements, subnormals kept) of two pixels of one channel and two taps.  A pixel holds its channels side by side, so a
 // pair of pixels of one channel is one byte permutation of the two dwords, taken from a row as loaded: it stands where the
 // widening stood.  A tap without a partner (the filters are odd) stays a multiply-add of the widened element: a partner with a
 // zero tap would turn an infinity next to the window into NaN.

@@ -1,6 +1,6 @@
 // 16-bit LDS images for the whole-plane kernels (dwconv_small_fir.hpp, dwconv_small_bwd.hpp): runs of planes travel into LDS and
 // back as they are in memory, a lane's rows are dwords of two elements, and sums take two products at a time (two-element dot
-// products: both products exact, one fp32 sum).
+// products: each rounds like two multiply-adds of widened elements, subnormals kept; a product beyond fp32's range is an infinity).
 //
 // With fp32 images these kernels were bound by the instructions they issue: every element widened on its way in, K * K
 // multiply-adds a result.  Pairs cost next to nothing here, because a lane holds whole rows:
@@ -12,8 +12,10 @@
 // C=480 3x3 23.7 / 21.8; batch 64 19x19 C=672 5x5 64.6 / 57.4, 16x16 C=672 5x5 38.4 / 24.8; forward, 14x14 C=672 5x5 stride 2
 // 13.5 / 10.9, fp16 28x28 C=240 5x5 31.2 / 23.7, bf16 batch 64 32x32 C=240 5x5 30.1 / 15.5 (its fp32 rows meet on the same banks).  Of
 // the 29 us of 14x14 C=480 5x5 both gradients 13 are launches, first loads and the sums' way out, 13 the products, 4 memory.
-// A product never takes part in a sum that it does not belong to (no zero taps, no zero elements for the sake of a pair): an
-// infinity reaches the results of its windows only.
+// No product is made for the sake of a pair (no zero taps, no zero elements), so in the forward pass and in grad-input an infinity
+// reaches the results of its windows only.  Grad-weight multiplies the padding's zeros, as with fp32 images: those of the rows above
+// and below a plane and of a lane's rows past it, and in the ragged instances those of the columns past a row.  An infinity
+// that they meet makes NaN of taps it has no part in.
 #pragma once
 
 #include "dwconv_small_common.hpp"

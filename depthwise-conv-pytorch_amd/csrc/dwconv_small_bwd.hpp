@@ -41,8 +41,8 @@ struct SmallBwdPlan {
     int in_w, out_w;     // real widths (the kernels of an exact instance use their template constant)
     int pad_h;
     int planes_per_run;  // channels per wavefront
-    int g_off;           // float offset of the gy run's span in LDS (a multiple of four)
-    int zero_off;        // float offset of the row of zeros in LDS (a multiple of four)
+    int g_off;           // where the gy run's span starts in LDS, in the images' elements (a multiple of four; 16 bits: of eight)
+    int zero_off;        // ... and the row of zeros
     int lds_x_floats, lds_g_floats;  // LDS images of the two runs (host side only)
     int lds_x_off;       // float offset of the x run's span (0)
     int lp_in, lp_out;   // ragged instances: LDS row pitch of the x / gy rows (width | 1)

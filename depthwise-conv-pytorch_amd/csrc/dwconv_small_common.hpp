@@ -58,7 +58,7 @@ struct SmallPlan {
     int planes_per_run;    // P
     int lanes_per_plane;   // LPP
     unsigned lpp_magic;
-    int zero_off;          // float offset of the row of zeros in LDS (a multiple of four)
+    int zero_off;          // where the row of zeros starts in LDS, in the image's elements (a multiple of four; 16 bits: of eight)
     int lp_in, lp_out;     // ragged instances: LDS row pitch of the input / output rows (width | 1)
     unsigned magic_in, magic_out;  // ... and the reciprocals for padded_index (0: pitch == width, flat copies)
     Epilogue epi;          // forward kernels: applied to every sum before it is stored

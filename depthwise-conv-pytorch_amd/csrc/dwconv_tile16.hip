@@ -9,7 +9,7 @@
 //   taps  = packed in pairs (t[2j], t[2j+1]) as the tensor's own 16-bit values.
 //   item  = BH x 8 outputs (stride 1) or BH x 4 outputs (stride 2) per lane.  A window row is read as dwords; the
 //           pairs that start at an odd element are formed with one v_alignbit each, and every output takes
-//           ceil(K/2) two-element dot products (v_dot2c_f32_f16 / v_dot2c_f32_bf16: exact products, fp32 sum) per
+//           ceil(K/2) two-element dot products (v_dot2c_f32_f16 / v_dot2c_f32_bf16, each as exact as two multiply-adds in fp32) per
 //           filter row instead of K multiply-adds.  The last tap of a row has no partner: its element is isolated
 //           with a mask (a garbage partner times a zero tap would turn an Inf next to the window into a NaN).
 // Same results as the fp32-image kernel up to the order of the fp32 additions.
@@ -180,7 +180,7 @@ __global__ __launch_bounds__(kThreads) void fir_down16_kernel(const Tile16Plan p
         const int rb = fast_div(rem, p.ncb_magic);
         const int cb = rem - __mul24(rb, p.ncb);
         const int rows_here = min(p.rows_per_tile, p.out_h - oy0);
-        const int run = rows_here * p.out_w;  // elements per plane, a multiple of eight
+        const int run = rows_here * p.out_w;  // elements per plane (a multiple of eight unless ANY)
         // Wavefronts with no item at all skip the arithmetic; lanes without one in the others compute item 0 again.
         // The sums never leave the arm that makes them (merged with the arm that has none, every sum would be zeroed
         // first); what leaves it are the packed rows, and every wavefront meets the one barrier after the branch.
