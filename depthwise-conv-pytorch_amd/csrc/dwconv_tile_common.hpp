@@ -834,7 +834,8 @@ __device__ __forceinline__ void commit_rows_any(const StageLayout &s, const RowL
 // A block of four 16-bit results of a row of any width (`rem` = width % 4, uniform) at byte offset `off` of a view that starts on
 // a 32-bit boundary; `n` results are left of the row from here on.  `odd`: the block starts 2 bytes past such a
 // boundary, and leaves as 16 + 32 + 16 bits; else as 64, or at the end of the row 32 and / or 16 bits.  A branch on `odd` (uniform in the
-// stride-2 kernel, its caller), none on the rest, as in view_store_first.  Dropped when `off` is at or beyond kOob.
+// stride-2 kernel; in the stacked one it follows the lane's image, where an image has an odd number of elements), none on the rest, as in
+// view_store_first.  Dropped when `off` is at or beyond kOob.
 template <typename IO>
 __device__ __forceinline__ void view_store_any(__amdgpu_buffer_rsrc_t view, unsigned off, int n, int rem, bool odd, float a, float b,
                                                float c, float d)

@@ -24,13 +24,65 @@ def test_backward(gpu, shape, dtype, by):
     gx, gw = _C.dwconv2d_backward(shifted(x, gpu, by), shifted(gy, gpu, by), wt.to(gpu), s, s, p, p)
     variant = _C.last_variant()
     assert variant.startswith("bwd_stack16<") and " dot2" in variant, variant
-    # rows that start on any element: grad-input leaves through LDS as one run an image
     assert (" anystart" in variant) == bool(w % 2 or by), variant
     _, gx_ref, gw_ref = oracle.torch_reference(x, wt, gy, s, p)
     check(gx, gx_ref, UNIT[dtype])
     check(gw, gw_ref, UNIT[dtype])
     gx2, gw2 = _C.dwconv2d_backward(shifted(x, gpu, by), shifted(gy, gpu, by), wt.to(gpu), s, s, p, p)
     assert torch.equal(gx, gx2) and torch.equal(gw, gw2)
+
+
+# the last and first sizes of the rule that sends grad-input of rows on any element through LDS as one run an image
+@pytest.mark.parametrize("shape,run", [((71, 42, 75, 75, 3, 1, 1), False), ((19, 157, 75, 75, 3, 1, 1), True), ((19, 100, 95, 95, 3, 1, 1), True),
+                                       ((19, 100, 97, 97, 3, 1, 1), False), ((64, 173, 39, 39, 5, 1, 2), True), ((64, 173, 41, 41, 5, 1, 2), False),
+                                       ((64, 242, 33, 33, 7, 1, 3), False), ((64, 161, 40, 41, 3, 1, 1), True), ((64, 75, 59, 60, 3, 1, 1), False)],
+                         ids=lambda v: shape_id(v) if isinstance(v, tuple) else str(v))
+def test_results_as_one_run_where_it_is_faster(gpu, monkeypatch, shape, run):
+    """Both ways leave the same bits (those of a few planes are checked against 64 bits)."""
+    from torch_dwconv import _C
+
+    n, c, h, w, k, s, p = shape
+    g = torch.Generator(gpu).manual_seed(63)
+    x, gy = (torch.randn(n, c, h, w, device=gpu, generator=g).to(torch.bfloat16) for _ in range(2))
+    wt = (torch.randn(c, 1, k, k, device=gpu, generator=g) / k).to(torch.bfloat16)
+    gx, gw = _C.dwconv2d_backward(x, gy, wt, s, s, p, p)
+    variant = _C.last_variant()
+    assert variant.startswith("bwd_stack16<") and (" runout" in variant) == run, variant
+    monkeypatch.setenv("DWCONV_TUNING", "1")
+    monkeypatch.setenv("DWCONV_STACK_RUN", "0" if run else "1")
+    gx2, gw2 = _C.dwconv2d_backward(x, gy, wt, s, s, p, p)
+    assert (" runout" in _C.last_variant()) == (not run and k <= 5 and w % 2 != 0), _C.last_variant()
+    assert torch.equal(gx, gx2) and torch.equal(gw, gw2)
+    last = slice(c - 2, c)
+    want = torch.nn.grad.conv2d_input((n, 2, h, w), wt[last].double().cpu(), gy[:, last].double().cpu(), padding=p, groups=2)
+    check(gx[:, last], want, UNIT[torch.bfloat16])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16], ids=["bf16", "f16"])
+@pytest.mark.parametrize("shape,by", [((5, 2, 34, 49, 3, 1, 1), 0), ((5, 2, 34, 50, 3, 1, 1), 1), ((2, 3, 9, 133, 3, 1, 1), 0), ((7, 1, 33, 33, 5, 1, 2), 0),
+                                      ((33, 2, 36, 38, 5, 1, 2), 1), ((33, 3, 35, 51, 5, 1, 2), 0), ((3, 2, 130, 66, 3, 1, 1), 1)],
+                         ids=lambda v: shape_id(v) if isinstance(v, tuple) else str(v))
+def test_results_as_one_run(gpu, monkeypatch, shape, by, dtype):
+    """Small tensors through the switch: remainders, shifted tensors, tiles that span images, one and many tiles a workgroup."""
+    from torch_dwconv import _C
+
+    n, c, h, w, k, s, p = shape
+    x, wt, gy = (t.to(dtype) for t in make_inputs(shape, seed=64))
+    args = (shifted(x, gpu, by), shifted(gy, gpu, by), wt.to(gpu), s, s, p, p)
+    gx, gw = _C.dwconv2d_backward(*args)
+    assert " runout" not in _C.last_variant(), _C.last_variant()
+    monkeypatch.setenv("DWCONV_TUNING", "1")
+    monkeypatch.setenv("DWCONV_STACK_RUN", "1")
+    gx2, gw2 = _C.dwconv2d_backward(*args)
+    assert " runout" in _C.last_variant(), _C.last_variant()
+    assert torch.equal(gx, gx2) and torch.equal(gw, gw2)
+    monkeypatch.setenv("DWCONV_STACK_WGS", "1")
+    gx3, gw3 = _C.dwconv2d_backward(*args)
+    assert " chunks1 " in _C.last_variant(), _C.last_variant()
+    _, gx_ref, gw_ref = oracle.torch_reference(x, wt, gy, s, p)
+    check(gx3, gx_ref, UNIT[dtype])
+    check(gw3, gw_ref, UNIT[dtype])
+    assert torch.equal(gx, gx3)
 
 
 @pytest.mark.parametrize("shape", [(2, 2, 48, 48, 3, 1, 1), (2, 2, 40, 51, 5, 1, 2), (2, 2, 40, 54, 7, 1, 3)], ids=shape_id)
