@@ -85,6 +85,23 @@ def test_results_as_one_run(gpu, monkeypatch, shape, by, dtype):
     assert torch.equal(gx, gx3)
 
 
+@pytest.mark.parametrize("shape,chunks", [((16, 64, 91, 91, 3, 1, 1), 24), ((8, 32, 193, 193, 3, 1, 1), 48), ((20, 64, 80, 80, 3, 1, 1), 24),
+                                          ((64, 96, 33, 33, 3, 1, 1), 21), ((16, 64, 83, 83, 3, 1, 1), 28), ((64, 96, 45, 45, 3, 1, 1), 22)],
+                         ids=lambda v: shape_id(v) if isinstance(v, tuple) else str(v))
+def test_workgroups_that_share_the_tiles(gpu, shape, chunks):
+    """3x3: up to 2048 workgroups where one of them then has fewer tiles than with 1536, and no more than those where it has not."""
+    from torch_dwconv import _C
+
+    n, c, h, w, k, s, p = shape
+    x, wt, gy = (t.to(torch.bfloat16) for t in make_inputs(shape, seed=65))
+    gx, gw = _C.dwconv2d_backward(x.to(gpu), gy.to(gpu), wt.to(gpu), s, s, p, p)
+    assert f" chunks{chunks} " in _C.last_variant(), _C.last_variant()
+    few = slice(0, 3)
+    _, gx_ref, gw_ref = oracle.torch_reference(x[:, few], wt[few], gy[:, few], s, p)
+    check(gx[:, few], gx_ref, UNIT[torch.bfloat16])
+    check(gw[few], gw_ref, UNIT[torch.bfloat16])
+
+
 @pytest.mark.parametrize("shape", [(2, 2, 48, 48, 3, 1, 1), (2, 2, 40, 51, 5, 1, 2), (2, 2, 40, 54, 7, 1, 3)], ids=shape_id)
 def test_infinite_gradients_reach_their_windows_only(gpu, shape):
     from torch_dwconv import _C
