@@ -349,6 +349,31 @@ int launch_down16_parity(Tile16Plan &p, bool any, hipStream_t stream)
     return seven ? launch_down16<IO, K, S, PW1, FLIP, 7, false>(p, stream) : launch_down16<IO, K, S, PW1, FLIP, 4, false>(p, stream);
 }
 
+// From how many elements of input on calls on rows of any width come here.  A call of a few workgroups a compute unit lasts about as
+// long as one of them, and one lasts longer here: more planes, loads to shift, the results through LDS.  Time here over that of the
+// kernels before (fp32 images; stacked for 5x5 and 7x7 on even rows), geometric means over 1659 layers of 33 to 257 columns, by millions
+// of elements (single layers lie up to 0.15 to either side):
+//                                          -0.6  -0.85   -1.2   -1.7   -2.4   -3.3   -4.7   -6.5   more
+//   stride 1, 3x3, odd rows                  1.08   1.05   1.01   1.00   0.98   1.00   0.94   0.89   0.78
+//             3x3, even                      1.32   1.28   1.19   1.24   1.23   1.15   1.19   1.04   0.90
+//             5x5, odd                       1.06   1.06   0.98   1.03   0.99   1.02   0.97   0.92   0.86
+//             5x5, even                      1.37   1.32   1.23   1.20   1.24   1.12   1.14   0.99   0.88
+//             7x7, odd                       1.05   1.03   0.96   1.00   1.00   0.92   0.86   0.82   0.77
+//             7x7, even                      1.20   1.18   1.07   1.00   1.03   1.02   0.92   0.89   0.85
+//   stride 2, 3x3, odd, and even below 128   1.11   1.10   1.07   1.01   1.02   1.01   0.98   0.92   0.85
+//             3x3, even from 128 on          1.02   1.03   1.01   0.97   0.93   0.96   0.97   0.94   0.78
+//             5x5, below 128                 1.06   1.06   1.02   0.97   1.00   0.98   0.94   0.90   0.83
+//             5x5, from 128 on               0.92   0.93   0.90   0.89   0.86   0.94   0.91   0.82   0.68
+//             7x7, even below 128            1.05   1.03   0.99   0.95   0.98   0.95   0.85   0.80   0.74
+//             7x7, the others                0.92   0.91   0.90   0.90   0.92   0.88   0.82   0.72   0.63
+int any_width_least_elements(int K, int S, int w)
+{
+    const bool even = w % 2 == 0, wide = w >= 128;
+    if (S == 1) return even ? (K == 7 ? 1 << 21 : 5 << 20) : (K == 7 ? 1 << 20 : 3 << 19);
+    if (K == 3) return even && wide ? 0 : 3 << 19;
+    return wide || (K == 7 && !even) ? 0 : 1 << 20;
+}
+
 }  // namespace
 
 // -1 when the kernel does not cover g (the caller goes on to the fp32-image kernel).
@@ -376,11 +401,13 @@ int try_launch_fir_tiled16(const IO *in, const IO *taps, IO *out, const Geometry
     // columns on (below, 33 to 57: between 20 % faster and 8 % slower), even ones that are no multiple of four 5-13 % from 128 on
     // (below: 7 % faster to 16 % slower, as the lanes fill), and multiples of four, which that kernel loads aligned, are up to
     // 25 % slower (92: 14.2 us there, 18.0 here).  With 7x7 filters every width from 56 on that is no multiple of four is 6-37 %
-    // faster.
+    // faster.  Small calls stay with the kernels of before: any_width_least_elements.
     if (any) {
         const bool odd = (g.in_w & 1) != 0, four = g.in_w % 4 == 0;
         const int least = S == 2 ? 33 : four ? 1 << 30 : K == 7 ? 56 : odd ? 65 : 128;
         if (g.in_w < env_int("DWCONV_T16_ANY_MIN_W", least)) return -1;
+        const long elements = static_cast<long>(g.planes()) * g.in_h * g.in_w;
+        if (elements < env_int("DWCONV_T16_ANY_MIN", any_width_least_elements(K, S, g.in_w))) return -1;
     } else if (g.in_w < env_int("DWCONV_T16_MIN_W", S == 2 ? 48 : 72)) {
         return -1;
     }

@@ -9,6 +9,15 @@ from test_gpu_any_width_staging import UNIT, check, shifted
 
 pytestmark = pytest.mark.gpu
 
+
+@pytest.fixture(autouse=True)
+def also_small_calls(request, monkeypatch):
+    """These layers are smaller than those that come to this kernel by themselves (see test_which_calls)."""
+    if "own_rule" not in request.keywords:
+        monkeypatch.setenv("DWCONV_TUNING", "1")
+        monkeypatch.setenv("DWCONV_T16_ANY_MIN", "0")
+
+
 # stride 2: blocks of four results; stride 1: blocks of eight
 SHAPES = [(2, 3, 9, 30 + w, 3, 2, 1) for w in range(3, 10)] + [(1, 3, 6, 64 + w, 3, 1, 1) for w in (1, 3, 5, 7)] + [
     (1, 2, 5, 128 + w, 5, 1, 2) for w in (1, 2, 6)] + [(2, 2, 10, 56 + w, 7, 1, 3) for w in (1, 2, 3, 5, 6, 7)] + [
@@ -61,3 +70,23 @@ def test_fused_epilogue_and_grad_input(gpu, shape):
         gx = _C.dwconv2d(gy.to(gpu), wt.to(gpu), 1, 1, 1, 1, p, p, p, p, False)
         assert _C.last_variant().endswith(" runout anywidth"), _C.last_variant()
         check(gx, oracle.torch_reference(x, wt, gy, s, p)[1], UNIT[torch.bfloat16])
+
+
+# the last and first sizes of the rule that keeps small calls on the kernels of before
+@pytest.mark.own_rule
+@pytest.mark.parametrize("shape,here", [((9, 31, 75, 75, 3, 1, 1), False), ((7, 40, 75, 75, 3, 1, 1), True), ((1, 233, 150, 150, 5, 1, 2), False),
+                                        ((3, 78, 150, 150, 5, 1, 2), True), ((13, 37, 66, 66, 7, 1, 3), False), ((2, 241, 66, 66, 7, 1, 3), True),
+                                        ((8, 31, 65, 65, 7, 1, 3), False), ((3, 83, 65, 65, 7, 1, 3), True), ((9, 31, 75, 75, 3, 2, 1), False),
+                                        ((7, 40, 75, 75, 3, 2, 1), True), ((1, 3, 150, 150, 3, 2, 1), True), ((6, 31, 75, 75, 5, 2, 2), False),
+                                        ((11, 17, 75, 75, 5, 2, 2), True), ((1, 2, 9, 131, 5, 2, 2), True), ((1, 359, 54, 54, 7, 2, 3), False),
+                                        ((1, 360, 54, 54, 7, 2, 3), True), ((1, 2, 9, 37, 7, 2, 3), True)],
+                         ids=lambda v: shape_id(v) if isinstance(v, tuple) else str(v))
+def test_which_calls(gpu, shape, here):
+    from torch_dwconv import depthwise_conv2d, _C
+
+    n, c, h, w, k, s, p = shape
+    x, wt, gy = (t.to(torch.bfloat16) for t in make_inputs(shape, seed=34))
+    y = depthwise_conv2d(x.to(gpu), wt.to(gpu), stride=s, padding=p)
+    variant = _C.last_variant()
+    assert (variant.startswith("tile_down16_dot2") and variant.endswith(" runout anywidth")) == here, variant
+    check(y, torch.nn.functional.conv2d(x.double(), wt.double(), stride=s, padding=p, groups=c), UNIT[torch.bfloat16])

@@ -15,6 +15,13 @@ CASES = [((2, 5, 14, 14, 5, 1, 2), False, ",dot2>", ",dot2>"), ((2, 3, 19, 19, 3
          ((2, 64, 28, 28, 5, 2, 2), True, "nhwc_down16<k5", "nhwc_bwd16<k5,s2")]
 
 
+@pytest.fixture(autouse=True)
+def also_small_calls(monkeypatch):
+    """(rows of any width: larger layers come to the 16-bit forward kernel by themselves)"""
+    monkeypatch.setenv("DWCONV_TUNING", "1")
+    monkeypatch.setenv("DWCONV_T16_ANY_MIN", "0")
+
+
 def both_ways(gpu, x, wt, gy, shape, nhwc, variants):
     from torch_dwconv import _C, depthwise_conv2d
 
