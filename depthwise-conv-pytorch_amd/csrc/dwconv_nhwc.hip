@@ -359,9 +359,12 @@ __global__ __launch_bounds__(kNhwcThreads) void nhwc_down_kernel(const NhwcPlan 
     const int pg = wg / p.cgroups;
     const int c0 = (wg - pg * p.cgroups) * p.lanes_c * CV;
     const int nch = min(p.lanes_c * CV, C - c0);
-    // 16 bits: two taps at a time in the tall blocks of 5x5 filters and with 7x7 ones (us, multiply-adds / pairs: bf16 batch 64, 7x7 56x56 C=96
-    // 42.7 / 37.7, 7x7 C=768 12.2 / 11.0; batch 128, 5x5 28x28 C=240 29.0 / 27.9; fp16 batch 32, 5x5 13x13 C=672 10.3 / 8.9);
-    // 4 x 4 blocks lose with them (bf16 batch 64, 5x5 16x16 C=672 14.1 / 15.4), 3x3 filters wait for memory either way.  Up to 5x5 the taps of two channels stay in
+    // 16 bits: two taps at a time with 7x7 filters (us, multiply-adds / pairs, bf16 batch 64: 56x56 C=96 38.9 / 32.8, 14x14 C=384 14.7 / 12.6,
+    // 7x7 C=768 11.4 / 10.2) and in the tall blocks of 5x5 ones.  There float16, which widens at more cost, gains 3 to 15 % on all of 17
+    // layers (batch 128 28x28 C=240 34.1 / 33.0, 14x14 C=480 16.0 / 14.1); bfloat16 gains where few workgroups wait for their taps, fewer
+    // loads in pairs (batch 8 14x14 C=480 7.2 / 6.1, batch 64 7x7 C=672 7.8 / 6.5), and is even elsewhere (28x28 C=240 33.6 / 32.5, 14x14
+    // C=480 15.1 / 14.7, C=672 19.4 / 19.8, 7x7 C=1152 11.3 / 11.5; batch 32 112x112 C=64 24.2 / 25.0).  4 x 4 blocks lose with them
+    // (bf16 batch 64, 5x5 16x16 C=672 14.1 / 15.4), 3x3 filters wait for memory either way.  Up to 5x5 the taps of two channels stay in
     // registers.
     constexpr bool PAIRS = kPairs<IO> && (K == 7 || (K == 5 && BH == 7));
     constexpr bool TAP_REGS = sizeof(IO) == 2 && K <= 5;
@@ -1616,7 +1619,8 @@ long nhwc_bwd_fused(int mode, const IO *x, const IO *gy, const IO *taps, IO *gx,
         // 46.0, 39.9, 44.4, 39.0.  5x5 on pairs: 4 x 2 blocks in 158 registers, three wavefronts asked for (without: 153, and 4-8 %
         // slower).  bf16, us with the two separate kernels / here: batch 128 56x56 C=144 87.4 / 82.3, 14x14 C=672 38.7 / 34.3, batch 64
         // 64x64 C=144 68.0 / 60.8, 16x16 C=672 28.1 / 23.7; 2 x 2, 2 x 4 and 4 x 4 blocks: 98, 87 and 92 us on the first.  Calls of less
-        // than 2^15 elements, one or two workgroups, stay on the separate kernels.
+        // than 2^15 elements stay on the separate kernels, at a cost: the sweep would take 0.63 to 0.70 of their time (12 layers; 1x8x32x32
+        // 17.8 / 12.4, 1x768x6x6 17.9 / 11.6).
         if constexpr (sizeof(IO) == 4) {
             if (g.kernel_h == 3) return nhwc_bwd_s2_fused_case<IO, 3, 1, 7, 4>(mode, x, gy, taps, gx, gw, ws, ws_bytes, g, stream);
             return nhwc_bwd_s2_fused_case<IO, 5, 1, 4, 2>(mode, x, gy, taps, gx, gw, ws, ws_bytes, g, stream);
@@ -1632,7 +1636,8 @@ long nhwc_bwd_fused(int mode, const IO *x, const IO *gy, const IO *taps, IO *gx,
         // 16 bits, 7x7: 49 sums for each of two channels and 4 x 4 blocks in 246 registers.  bf16, batch 64, us with the two separate
         // kernels (both on pairs too) / here: 56x56 C=96 101 / 94.5, 28x28 C=192 55 / 51, 14x14 C=384 39.3 / 39.3, 7x7 C=768 33 / 28;
         // blocks of 7 x 2: 107, 58, 38, 28; 4 x 2: 115, 64, 44, 36; 2 x 4: 110, 59, 42, 35.  Batch 1: 28.7 / 23.3, 22.3 / 18.8, 19.9 / 18.1,
-        // 20.2 / 18.7 (37632 elements).  Calls of less than 2^15 elements, one or two workgroups, stay on the separate kernels.
+        // 20.2 / 18.7 (37632 elements).  Calls of less than 2^15 elements stay on the separate kernels, at a cost: below it the sweep would
+        // take 0.93 to 0.98 of their time (16 layers; 1x8x32x32 20.0 / 18.6, 1x96x18x18 17.5 / 16.6, 40x768x1x1 20.8 / 20.4).
         if constexpr (sizeof(IO) == 2) if (static_cast<long>(g.batch) * g.in_h * g.in_w * g.channel >= 1l << 15)
             return nhwc_bwd_fused_case<IO, 7, 2, 4, 4, 1, 2>(mode, x, gy, taps, gx, gw, ws, ws_bytes, g, stream);
         return -1;
@@ -1644,8 +1649,9 @@ long nhwc_bwd_fused(int mode, const IO *x, const IO *gy, const IO *taps, IO *gx,
         // layer of the stack (28x28 C=240: 112 -> 91 us, 14x14 C=672: 75 -> 68, C=480: 59 -> 50, 7x7 C=1152: 42 -> 39).
         // 16 bits: two channels (rows travel raw, in half the registers) and 7 x 2 blocks; bf16 28x28 C=240 75 us with the
         // separate kernels, 64 with 7 x 2 or 7 x 4 blocks; 14x14 C=480 45 / 37 / 38, C=672 58 / 47 / 51; 7x7 C=1152 31 / 29 / 34.
-        // On pairs it needs 170 registers, two wavefronts per SIMD; with two rows in flight and three asked for 161: multiply-adds /
-        // pairs / pairs with three wavefronts 70.7 / 75.0 / 66.9, 40.3 / 43.8 / 36.2, 49.5 / 54.4 / 46.7, 31.4 / 31.1 / 28.4.
+        // On pairs it needs 170 registers, two wavefronts per SIMD; with two rows in flight and three asked for 161.  Multiply-adds / pairs
+        // with three wavefronts, in turn on one card: 64.7 / 62.4, 37.7 / 34.9, 45.7 / 44.6, 28.8 / 25.5 (with two wavefronts they lost to
+        // multiply-adds on the first three).
         if (env_int("DWCONV_NHWC_FUSED5", 1)) {
             if constexpr (sizeof(IO) == 4) return nhwc_bwd_fused_case<IO, 5, 1, 7, 4>(mode, x, gy, taps, gx, gw, ws, ws_bytes, g, stream);
             else return nhwc_bwd_fused_case<IO, 5, 2, 7, 2, 2, 3>(mode, x, gy, taps, gx, gw, ws, ws_bytes, g, stream);

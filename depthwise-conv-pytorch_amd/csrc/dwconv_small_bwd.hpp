@@ -533,7 +533,8 @@ bool plan_small_bwd(SmallBwdPlan &p, const WgradGeometry &g)
     p.g_off = round_up(p.lds_x_floats + head, 4);
     p.lpp_magic = magic_u16(p.lanes_per_plane);
     const int groups = ceil_div(g.channel, P);
-    // At these register counts two wavefronts fit a SIMD, 2048 the device: the grid stays within that one resident
+    // At these register counts two wavefronts fit a SIMD, 2048 the device (but for exact widths of 24 columns and more with 7x7
+    // filters and 16-bit images: 258 to 281 registers, one): the grid stays within that one resident
     // round (rounded down: 2112 wavefronts instead of 1536 cost the 28x28 7x7 backward 58 us instead of 47, the 64
     // stragglers run their whole chunk alone).
     int chunks = env_int("DWCONV_SMALL_WGRAD_WAVES", 2048) / groups;
